@@ -32,6 +32,7 @@
  */
 #include "tdv_internal.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cfloat>
 #include <vector>
@@ -192,9 +193,12 @@ __global__ void k_kick_bins(int nact, const int *__restrict__ active,
 		const double *__restrict__ ax, const double *__restrict__ ay,
 		const double *__restrict__ az, double *__restrict__ vx,
 		double *__restrict__ vy, double *__restrict__ vz,
-		double *__restrict__ kick_dt, TimelineDev t)
+		double *__restrict__ kick_dt, TimelineDev t,
+		unsigned *__restrict__ list_count)
 {
 	const int g = blockIdx.x * blockDim.x + threadIdx.x;
+	if (g < 2)
+		list_count[g] = 0;               /* the tree kicks' list, its queue */
 	if (g >= nact)
 		return;
 	const int i = active[g];
@@ -227,13 +231,31 @@ __device__ __forceinline__ int active_lower(const int *__restrict__ a, int n,
  * particle: each tree node on the particle's path below its subtree root
  * (the nodes whose particle range holds it) takes Dp += m dt a / M, marked
  * UPDATED; the node's particles in particle order, so the sums are the
- * reference's one-thread sums. */
+ * reference's one-thread sums.
+ *
+ * One lane per node finds the node's run [lo, hi) of the sorted active list
+ * and sums runs of up to KICK_LANE_RUN particles itself.  A longer run is a
+ * chain of that many dependent additions, so what one lane can do about it
+ * is to keep everything else (loads, products, the division) out of the
+ * chain, which it cannot: such nodes go to a list, one wavefront each
+ * (k_tree_kicks_long).  Nodes of more than 64 active particles are disjoint
+ * within a level, so TDV_NT levels hold fewer than 42 / 65 n of them and the
+ * list fits n entries.  With one lane for every node and top node a kick of
+ * all particles of the clustered 2^20 box took 67 ms here and 88 ms for the
+ * top nodes; now 0.06 ms here and 5.4 ms for the list and the top nodes. */
+#define KICK_LANE_RUN 64
+
+struct KickList {                /* build scratch, n entries each */
+	int *node, *lo, *hi;
+	unsigned *count;             /* [0] listed nodes, [1] their queue */
+};
+
 __global__ void k_tree_kicks(size_t nn, int4 *__restrict__ nc,
 		const double4 *__restrict__ na, double4 *__restrict__ dpn,
 		int nact, const int *__restrict__ active,
 		const double *__restrict__ m, const double *__restrict__ dtk,
 		const double *__restrict__ ax, const double *__restrict__ ay,
-		const double *__restrict__ az)
+		const double *__restrict__ az, KickList list)
 {
 	const size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	if (j >= nn)
@@ -245,9 +267,37 @@ __global__ void k_tree_kicks(size_t nn, int4 *__restrict__ nc,
 	const int hi = active_lower(active, nact, c.w + c.y);
 	if (lo >= hi)
 		return;
+	nc[j].z = c.z | (1 << TDV_BIT_UPDATED);   /* only this node's own */
+	if (hi - lo > KICK_LANE_RUN) {
+		const unsigned slot = atomicAdd(&list.count[0], 1u);
+		list.node[slot] = (int)j;
+		list.lo[slot] = lo;
+		list.hi[slot] = hi;
+		return;
+	}
 	const double M = na[j].w;
 	double4 d = dpn[j];
-	for (int g = lo; g < hi; g++) {
+	/* four particles' loads and quotients at a time, then their additions
+	 * in order */
+	int g = lo;
+	for (; g + 4 <= hi; g += 4) {
+		double qx[4], qy[4], qz[4];
+#pragma unroll
+		for (int u = 0; u < 4; u++) {
+			const int i = active[g + u];
+			const double mdt = m[i] * dtk[i];
+			qx[u] = mdt * ax[i] / M;
+			qy[u] = mdt * ay[i] / M;
+			qz[u] = mdt * az[i] / M;
+		}
+#pragma unroll
+		for (int u = 0; u < 4; u++) {
+			d.x = d.x + qx[u];
+			d.y = d.y + qy[u];
+			d.z = d.z + qz[u];
+		}
+	}
+	for (; g < hi; g++) {
 		const int i = active[g];
 		const double mdt = m[i] * dtk[i];
 		d.x = d.x + mdt * ax[i] / M;
@@ -255,36 +305,105 @@ __global__ void k_tree_kicks(size_t nn, int4 *__restrict__ nc,
 		d.z = d.z + mdt * az[i] / M;
 	}
 	dpn[j] = d;
-	nc[j].z = c.z | (1 << TDV_BIT_UPDATED);   /* only this node's own */
 }
 
-/* the same for the top nodes (tree_update.c:43-55), in float: Dp is a
- * float in D[].TNode, and the node is marked kicked */
-__global__ void k_top_kicks(const TopNodes T, int nact,
+/* The sum of one run [lo, hi) of the active list by one wavefront: the
+ * lanes load 64 particles and form their quotients m dt a / M side by side,
+ * the next 64 particles' loads in flight meanwhile; lane c of the first
+ * three then adds component c in particle order from LDS, `step` making one
+ * addition.  What is left of the chain is one dependent addition (and, for
+ * the float top nodes, its two conversions) per particle. */
+template <typename Step>
+__device__ __forceinline__ double kick_run(int lo, int hi, double M,
 		const int *__restrict__ active, const double *__restrict__ m,
 		const double *__restrict__ dtk, const double *__restrict__ ax,
-		const double *__restrict__ ay, const double *__restrict__ az)
+		const double *__restrict__ ay, const double *__restrict__ az,
+		double start, double (*sh)[64], Step step)
 {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= *T.ntop)
-		return;
-	const int lo = active_lower(active, nact, T.first[t]);
-	const int hi = active_lower(active, nact, T.first[t] + T.npart[t]);
-	if (lo >= hi)
-		return;
-	const double M = (double)T.mass[t];
-	float dx = T.dp[3 * t], dy = T.dp[3 * t + 1], dz = T.dp[3 * t + 2];
-	for (int g = lo; g < hi; g++) {
-		const int i = active[g];
-		const double mdt = m[i] * dtk[i];
-		dx = (float)((double)dx + mdt * ax[i] / M);
-		dy = (float)((double)dy + mdt * ay[i] / M);
-		dz = (float)((double)dz + mdt * az[i] / M);
+	const int lane = threadIdx.x;
+	const double *row = sh[lane < 3 ? lane : 0];
+	double s = start, nm = 0, nx = 0, ny = 0, nz = 0;
+	if (lo + lane < hi) {
+		const int i = active[lo + lane];
+		nm = m[i] * dtk[i];
+		nx = ax[i];
+		ny = ay[i];
+		nz = az[i];
 	}
-	T.dp[3 * t] = dx;
-	T.dp[3 * t + 1] = dy;
-	T.dp[3 * t + 2] = dz;
-	T.kicked[t] = 1;
+	for (int b0 = lo; b0 < hi; b0 += 64) {
+		const double qx = nm * nx / M, qy = nm * ny / M, qz = nm * nz / M;
+		if (b0 + 64 + lane < hi) {
+			const int i = active[b0 + 64 + lane];
+			nm = m[i] * dtk[i];
+			nx = ax[i];
+			ny = ay[i];
+			nz = az[i];
+		}
+		__syncthreads();                 /* the last block's row is read */
+		sh[0][lane] = qx;
+		sh[1][lane] = qy;
+		sh[2][lane] = qz;
+		__syncthreads();
+		const int nb = hi - b0 < 64 ? hi - b0 : 64;
+		int q = 0;
+		for (; q + 16 <= nb; q += 16) {
+			double t[16];
+#pragma unroll
+			for (int u = 0; u < 16; u++)
+				t[u] = row[q + u];
+#pragma unroll
+			for (int u = 0; u < 16; u++)
+				s = step(s, t[u]);
+		}
+		for (; q < nb; q++)
+			s = step(s, row[q]);
+	}
+	return s;
+}
+
+/* The listed nodes, a wavefront each, and before them the top nodes
+ * (tree_update.c:43-55), whose runs are the longest: their Dp is a float in
+ * D[].TNode, rounded after every addition, and the node is marked kicked.
+ * Workgroup b < ntop takes top node b, then every workgroup takes listed
+ * nodes from one counter. */
+__global__ void __launch_bounds__(64) k_tree_kicks_long(const TopNodes T,
+		const double4 *__restrict__ na, double4 *__restrict__ dpn, int nact,
+		const int *__restrict__ active, const double *__restrict__ m,
+		const double *__restrict__ dtk, const double *__restrict__ ax,
+		const double *__restrict__ ay, const double *__restrict__ az,
+		KickList list)
+{
+	__shared__ double sh[3][64];
+	const int lane = threadIdx.x;
+	const int ntop = *T.ntop;
+	for (int t = blockIdx.x; t < ntop; t += gridDim.x) {
+		const int lo = active_lower(active, nact, T.first[t]);
+		const int hi = active_lower(active, nact, T.first[t] + T.npart[t]);
+		if (lo >= hi)
+			continue;
+		const double s = kick_run(lo, hi, (double)T.mass[t], active, m, dtk,
+				ax, ay, az, lane < 3 ? (double)T.dp[3 * t + lane] : 0.0, sh,
+				[](double a, double q) { return (double)(float)(a + q); });
+		if (lane < 3)
+			T.dp[3 * t + lane] = (float)s;
+		if (lane == 0)
+			T.kicked[t] = 1;
+	}
+	const int nl = (int)list.count[0];
+	for (;;) {
+		/* wave-uniform ticket, as in the walk's queue */
+		const unsigned tk = atomicAdd(&list.count[1], lane == 0 ? 1u : 0u);
+		const int item = __builtin_amdgcn_readfirstlane((int)tk);
+		if (item >= nl)
+			break;
+		const int j = list.node[item];
+		double *dp = reinterpret_cast<double *>(dpn + j);
+		const double s = kick_run(list.lo[item], list.hi[item], na[j].w,
+				active, m, dtk, ax, ay, az, lane < 3 ? dp[lane] : 0.0, sh,
+				[](double a, double q) { return a + q; });
+		if (lane < 3)
+			dp[lane] = s;
+	}
 }
 
 /* Gravity_Tree_Update_Drift (tree_update.c:64-104): the updated nodes move
@@ -536,16 +655,23 @@ int tdv_kick_halfstep(tdv_context *c, int update_tree)
 		hipLaunchKernelGGL(k_kick_bins, dim3(tdv_blocks((size_t)c->nactive,
 				256)), dim3(256), 0, c->stream, c->nactive, c->active,
 				c->time_bin, c->it_kick, c->acc[0], c->acc[1], c->acc[2],
-				c->vel[0], c->vel[1], c->vel[2], c->kick_dt, timeline_dev(c));
+				c->vel[0], c->vel[1], c->vel[2], c->kick_dt, timeline_dev(c),
+				c->long_count);
 	if (update_tree && c->nactive) {
+		const KickList list = { reinterpret_cast<int *>(c->minpack), c->cnt,
+			c->lohi, c->long_count };
 		if (c->nnodes)
 			hipLaunchKernelGGL(k_tree_kicks, dim3(tdv_blocks(c->nnodes, 256)),
 					dim3(256), 0, c->stream, c->nnodes, c->node_c, c->node_a,
 					c->node_dp, c->nactive, c->active, c->mass, c->kick_dt,
-					c->acc[0], c->acc[1], c->acc[2]);
-		hipLaunchKernelGGL(k_top_kicks, dim3(tdv_blocks((size_t)c->ntop, 64)),
-				dim3(64), 0, c->stream, c->top, c->nactive, c->active, c->mass,
-				c->kick_dt, c->acc[0], c->acc[1], c->acc[2]);
+					c->acc[0], c->acc[1], c->acc[2], list);
+		/* the top nodes first, then at most a wave per 65 active */
+		const unsigned grid = (unsigned)std::min((size_t)TDV_LONG_GRID,
+				(size_t)c->ntop + (size_t)c->nactive / (KICK_LANE_RUN + 1));
+		hipLaunchKernelGGL(k_tree_kicks_long, dim3(grid), dim3(64), 0,
+				c->stream, c->top, c->node_a, c->node_dp, c->nactive,
+				c->active, c->mass, c->kick_dt, c->acc[0], c->acc[1],
+				c->acc[2], list);
 	}
 	(void)hipEventRecord(c->ev[EV_KICK1], c->stream);
 	TDV_HIP(c, hipGetLastError());

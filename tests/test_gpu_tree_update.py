@@ -80,3 +80,29 @@ def _first_particle(tree, j):
     while tree["DNext"][k] >= 0:
         k += 1
     return -int(tree["DNext"][k]) - 1
+
+
+@pytest.mark.parametrize("n", [200, 4096 + 63, 30001])
+def test_tree_kicks_of_long_runs_match_oracle(n):
+    """Every particle active: runs of the active list below, at and far
+    beyond a wavefront, with a remainder."""
+    pos, vel, m = ics.hernquist_sphere(n, seed=5)
+    e = Engine(periodic=False, softening=0.01, alpha_rel=0.005)
+    e.set_particles(pos, m, vel=vel)
+    e.setup_domain()
+    e.domain_decomposition()
+    e.compute_acceleration(True)
+    e.make_active_list(31, time_bin=np.full(n, 9, np.int32))
+    e.set_timeline(engine.timeline(False, 0.0, 1.0))
+    st = e.get("mass", "acc", "tree_parent")
+    dt = np.full(n, 2.0 ** 8 / 2.0 ** 31)
+    tree, top = e.tree(), e.top_nodes()
+    for _ in range(2):                   # the second on top of the first
+        e.kick_halfstep(update_tree=True)
+        tree, top = U.kicks(tree, top, st["mass"], st["acc"], dt,
+                            st["tree_parent"], np.arange(n, dtype=np.int32))
+        got, gtop = e.tree(), e.top_nodes()
+        for f in ("Bitfield", "Dp", "CoM"):
+            np.testing.assert_array_equal(got[f], tree[f], err_msg=f)
+        for f in ("Level", "Dp", "CoM"):
+            np.testing.assert_array_equal(gtop[f], top[f], err_msg=f)
