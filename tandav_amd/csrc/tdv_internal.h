@@ -221,6 +221,11 @@ void tdv_graph_drop(tdv_context *c);
                                             one wavefront each */
 #define TDV_LONG_GRID 2048               /* waves of that kernel */
 #define TDV_SPLIT_AUTO_MAX 64            /* parts per group, split 0 */
+#define TDV_SMALL_RUN 16                 /* split walk: particles of a top
+                                            node without subtree per run */
+#define TDV_TURN_NODES 8                 /* split walk: parts turned by top
+                                            node below this many nodes per
+                                            part */
 #define TDV_WANT_WORDS 4                 /* a split walk's wanted-top-node
                                             mask: up to 256 top nodes */
 #define TDV_ORDER_MIN_GROUPS 2048        /* FP32 walks of this many whole

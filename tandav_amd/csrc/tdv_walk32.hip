@@ -610,11 +610,21 @@ struct EwaldLocal {
 	float Sxxx, Syyy, Szzz, Sxxy, Sxxz, Sxyy, Syyz, Sxzz, Syzz, Sxyz;
 };
 
-__device__ __forceinline__ EwaldLocal ewald_local(const float4 *__restrict__ t,
-		const EwaldNode &c, const Walk32Params &w)
+struct EwaldRec {                    /* a table node's record */
+	float4 r0, r1, r2, r3;
+};
+
+__device__ __forceinline__ EwaldRec ewald_fetch(const float4 *__restrict__ t,
+		const EwaldNode &c)
 {
 	const float4 *r = t + 4 * c.b;
-	const float4 r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3];
+	return EwaldRec{ r[0], r[1], r[2], r[3] };
+}
+
+__device__ __forceinline__ EwaldLocal ewald_eval(const EwaldRec &R,
+		const EwaldNode &c, const Walk32Params &w)
+{
+	const float4 r0 = R.r0, r1 = R.r1, r2 = R.r2, r3 = R.r3;
 	EwaldLocal e;
 	e.Sxxx = h2lo(r2.y);
 	e.Syyy = h2hi(r2.y);
@@ -647,16 +657,23 @@ __device__ __forceinline__ EwaldLocal ewald_local(const float4 *__restrict__ t,
 	return e;
 }
 
-/* Ewald_Correction (Gravity/periodic.c:35-113) of a point mass m' */
-__device__ __forceinline__ void ewald16(Acc32 &a, const float4 *__restrict__ t,
-		float m, float dx, float dy, float dz, const Walk32Params &w)
+/* Ewald_Correction (Gravity/periodic.c:35-113) of a point mass m' whose
+ * table record is at hand */
+__device__ __forceinline__ void ewald16_rec(Acc32 &a, const EwaldRec &R,
+		const EwaldNode &c, float m, const Walk32Params &w)
 {
-	const EwaldNode c = ewald_node(dx, dy, dz, w);
-	const EwaldLocal e = ewald_local(t, c, w);
+	const EwaldLocal e = ewald_eval(R, c, w);
 	a.x = fmaf(m * c.sx, e.ex, a.x);
 	a.y = fmaf(m * c.sy, e.ey, a.y);
 	a.z = fmaf(m * c.sz, e.ez, a.z);
 	a.ewald++;
+}
+
+__device__ __forceinline__ void ewald16(Acc32 &a, const float4 *__restrict__ t,
+		float m, float dx, float dy, float dz, const Walk32Params &w)
+{
+	const EwaldNode c = ewald_node(dx, dy, dz, w);
+	ewald16_rec(a, ewald_fetch(t, c), c, m, w);
 }
 
 /* The correction of a node of mass m' and traceless second moment T'
@@ -671,7 +688,7 @@ __device__ __forceinline__ void ewald16q(Acc32 &a, const float4 *__restrict__ t,
 		const Walk32Params &w)
 {
 	const EwaldNode c = ewald_node(dx, dy, dz, w);
-	const EwaldLocal e = ewald_local(t, c, w);
+	const EwaldLocal e = ewald_eval(ewald_fetch(t, c), c, w);
 	/* T' (masses G S^2, lengths S) to table units: / (S^4 Box^4), in two
 	 * steps so no constant is subnormal */
 	const float cxx = qa.x * w.inv_s2 * w.inv_s2_box4,
@@ -822,6 +839,25 @@ __device__ __forceinline__ bool top_want(const int4 tc, float ts,
 	return want || r2 < 3.f * ts * ts;
 }
 
+/* The particles [q, l), q < l, one by one, Newton and the Ewald correction
+ * of each (E(0) = 0: the self term adds 0) */
+__device__ __forceinline__ void ewald_pp(Acc32 &a, const float4 *__restrict__ tab,
+		const int4 *__restrict__ p32, int q, int l, const int4 me, int every,
+		const Walk32Params &w)
+{
+	int4 pn = p32[q];
+	for (; q < l; q++) {
+		const int4 pq = pn;
+		if (q + 1 < l)
+			pn = p32[q + 1];
+		const float dx = fdiff(pq.x, me.x), dy = fdiff(pq.y, me.y),
+				dz = fdiff(pq.z, me.z), m = __int_as_float(pq.w);
+		newton32(a, m, dx, dy, dz, w);
+		ewald16(a, tab, m, dx, dy, dz, w);
+		tick(a, every);
+	}
+}
+
 /* One wave walks `group` (64 active particles, one per lane) over part
  * `part` of `nparts`: every subtree the group walks is cut into nparts
  * contiguous node ranges and this wave takes range `part` of each, so
@@ -830,9 +866,11 @@ __device__ __forceinline__ bool top_want(const int4 tc, float ts,
  * starts at the first node >= its start that the whole walk would visit:
  * the descent below replays the whole walk's decisions on the range
  * start's ancestors (and their Ewald state) without interacting.  Part 0
- * also takes the top-node interactions.  With nparts == 1 the results go
+ * also takes the top-node interactions; the particles of top nodes without
+ * subtree are dealt out over the parts.  With nparts == 1 the results go
  * to the particles; otherwise to partial[part * nslot + slot], summed in
  * part order by k_walk32_parts_sum. */
+template <bool SPLIT>
 __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 		double4 *__restrict__ partial, int nslot, int nact,
 		const int *__restrict__ active, const int4 *__restrict__ p32,
@@ -875,8 +913,6 @@ __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 			j += (int)__builtin_ctzll(bits);
 			if (j >= ntop)
 				break;
-			if (T.npart[j] <= w.vs)      /* part 0's */
-				continue;
 		} else {
 		const int4 tc = top32[j];
 		const float tm = __int_as_float(tc.w);
@@ -899,35 +935,59 @@ __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 			tick(a, every);
 			continue;
 		}
+		}
 		if (T.npart[j] <= w.vs) {
-			if (part != 0)
-				continue;
-			const int f = T.first[j], l = f + T.npart[j];
-			for (int q = f; q < l; q++) {
-				const int4 pq = p32[q];
-				const float dx = fdiff(pq.x, me.x), dy = fdiff(pq.y, me.y),
-						dz = fdiff(pq.z, me.z);
-				const float m = __int_as_float(pq.w);
-				newton32(a, m, dx, dy, dz, w);
-				if (w.periodic)           /* E(0) = 0: the self term adds 0 */
-					ewald16(a, tab, m, dx, dy, dz, w);
-				tick(a, every);
+			/* no subtree: its particles, in the split walk in runs of
+			 * TDV_SMALL_RUN dealt out over the parts (with all of them
+			 * part 0's, the 16^3 box, whose 64 top nodes are all of this
+			 * kind, took 7.0 ms in 64 of 4096 waves; now 0.22 ms) */
+			const int f = T.first[j], e = f + T.npart[j];
+			unsigned r = (unsigned)j * (64 / TDV_SMALL_RUN);
+			for (int q = f; q < e; r++) {
+				const int l = SPLIT ? min(q + TDV_SMALL_RUN, e) : e;
+				if (!SPLIT || nparts == 1 || (int)(r % (unsigned)nparts) == part) {
+					if (w.periodic) {
+						ewald_pp(a, tab, p32, q, l, me, every, w);
+					} else {
+						for (int i = q; i < l; i++) {
+							const int4 pq = p32[i];
+							newton32(a, __int_as_float(pq.w),
+									fdiff(pq.x, me.x), fdiff(pq.y, me.y),
+									fdiff(pq.z, me.z), w);
+							tick(a, every);
+						}
+					}
+				}
+				q = l;
 			}
 			continue;
 		}
-		}
 		const int start = T.target[j];
 		int lo = start, hi = T.term[j];
-		if (nparts > 1) {
+		if (SPLIT && nparts > 1) {
+			const int len = hi - start;
+			/* Subtrees of few nodes per part give their nonempty ranges to
+			 * the same parts at every top node (9 nodes in 32 parts: nine
+			 * parts took a bundle each of all 64 top nodes, the other 23
+			 * nothing: the 32^3 box's walk 18.5 ms), so there the parts are
+			 * turned by a fraction of nparts that differs from top node to
+			 * top node, multiples of the golden ratio (4.0 ms).  From
+			 * TDV_TURN_NODES nodes per part the ranges are even anyway (the
+			 * 100^3 box, two parts: 35 ms turned or not). */
+			int vp = part;
+			if (len < TDV_TURN_NODES * nparts) {
+				vp += (int)__umulhi((unsigned)j * 2654435769u,
+						(unsigned)nparts);
+				vp -= vp >= nparts ? nparts : 0;
+			}
 			/* cut at floor(len p / nparts) in float: monotone in p, 0 at
 			 * p = 0 and below len for p < nparts, so every part computes
 			 * the same cuts and the ranges tile the subtree (a 64-bit
 			 * integer division here cost ~100 scalar instructions per cut,
 			 * twice per top node and part) */
-			const int len = hi - start;
-			lo = start + (int)((float)len * ((float)part * inv_parts));
-			if (part + 1 < nparts)
-				hi = start + (int)((float)len * ((float)(part + 1) * inv_parts));
+			lo = start + (int)((float)len * ((float)vp * inv_parts));
+			if (vp + 1 < nparts)
+				hi = start + (int)((float)len * ((float)(vp + 1) * inv_parts));
 			if (lo >= hi)
 				continue;
 		}
@@ -1076,19 +1136,7 @@ __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 						tick(a, every);
 					}
 				} else {
-					int4 pn = p32[f];
-					for (int q = f; q < l; q++) {
-						const int4 pq = pn;
-						if (q + 1 < l)
-							pn = p32[q + 1];
-						const float dx = fdiff(pq.x, me.x),
-								dy = fdiff(pq.y, me.y), dz = fdiff(pq.z, me.z);
-						const float m = __int_as_float(pq.w);
-						newton32(a, m, dx, dy, dz, w);
-						if (pending)          /* E(0) = 0 for the self term */
-							ewald16(a, tab, m, dx, dy, dz, w);
-						tick(a, every);
-					}
+					ewald_pp(a, tab, p32, f, l, me, every, w);
 				}
 				node++;
 				continue;
@@ -1171,12 +1219,13 @@ __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 		const int4 *__restrict__ top32, const float4 *__restrict__ tq32, \
 		const float4 *__restrict__ p32o, const uint32_t *__restrict__ gorder
 #define TDV_WALK32_CALL_PARTW(g, part, nparts, partial, nslot, wmask) \
-		walk32_body(g, part, nparts, partial, nslot, nact, active, p32, \
+		walk32_body<true>(g, part, nparts, partial, nslot, nact, active, p32, \
 		last_acc, T, rec, tab, w, ax, ay, az, gx, gy, gz, cost, \
 		counter, top32, tq32, p32o, wmask)
-#define TDV_WALK32_CALL_PART(g, part, nparts, partial, nslot) \
-		TDV_WALK32_CALL_PARTW(g, part, nparts, partial, nslot, nullptr)
-#define TDV_WALK32_CALL(g) TDV_WALK32_CALL_PART(g, 0, 1, nullptr, 0)
+#define TDV_WALK32_CALL(g) \
+		walk32_body<false>(g, 0, 1, nullptr, 0, nact, active, p32, \
+		last_acc, T, rec, tab, w, ax, ay, az, gx, gy, gz, cost, \
+		counter, top32, tq32, p32o, nullptr)
 /* the i-th group to walk: by descending expected cost when ordered */
 #define TDV_GROUP(i) (gorder ? (int)gorder[i] : (i))
 

@@ -297,3 +297,29 @@ def test_substep_walk_graph():
     unmoved = e.get("acc")["acc"][sub]
     assert np.abs(unmoved - got).max() > 0
     e.close()
+
+
+@pytest.mark.parametrize("n,split", [(4096, 0), (4096, 7), (4096, 256),
+                                     (1700, 5), (3000, 64), (20000, 64)])
+def test_split_walk_of_small_top_nodes_matches_whole_walk(n, split):
+    """Top nodes without subtree (their particles dealt out in runs over the
+    parts) and subtrees of few nodes per part (the parts turned): the whole
+    walk's interactions, each by one part."""
+    g = np.random.Generator(np.random.Philox(21))
+    pos, m = g.uniform(0.0, 1.0, (n, 3)), np.full(n, 1.0 / n)
+    whole = _engine(pos, m, 0, split=1, softening=1e-3)
+    parts = _engine(pos, m, 0, split=split, softening=1e-3)
+    ref = whole.get("pos", "last_acc_mag")
+    for sub in (np.arange(n), np.arange(5, n, 37)):
+        for e in (whole, parts):         # the same criterion input
+            e.set_active(sub)
+            e.update_particles(ref["pos"], acc=np.zeros((n, 3)),
+                               last_acc_mag=ref["last_acc_mag"])
+            e.tree_acceleration(False)
+        a, b = whole.get("acc", "cost"), parts.get("acc", "cost")
+        np.testing.assert_array_equal(a["cost"][sub], b["cost"][sub])
+        assert whole.interaction_counts() == parts.interaction_counts()
+        err = (np.linalg.norm(a["acc"][sub] - b["acc"][sub], axis=1)
+               / np.linalg.norm(a["acc"][sub], axis=1))
+        # FP32 rounding of partial sums, as in the test above
+        assert err.max() < 1e-4, (n, split, len(sub), err.max())
