@@ -610,21 +610,11 @@ struct EwaldLocal {
 	float Sxxx, Syyy, Szzz, Sxxy, Sxxz, Sxyy, Syyz, Sxzz, Syzz, Sxyz;
 };
 
-struct EwaldRec {                    /* a table node's record */
-	float4 r0, r1, r2, r3;
-};
-
-__device__ __forceinline__ EwaldRec ewald_fetch(const float4 *__restrict__ t,
-		const EwaldNode &c)
-{
-	const float4 *r = t + 4 * c.b;
-	return EwaldRec{ r[0], r[1], r[2], r[3] };
-}
-
-__device__ __forceinline__ EwaldLocal ewald_eval(const EwaldRec &R,
+__device__ __forceinline__ EwaldLocal ewald_local(const float4 *__restrict__ t,
 		const EwaldNode &c, const Walk32Params &w)
 {
-	const float4 r0 = R.r0, r1 = R.r1, r2 = R.r2, r3 = R.r3;
+	const float4 *r = t + 4 * c.b;
+	const float4 r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3];
 	EwaldLocal e;
 	e.Sxxx = h2lo(r2.y);
 	e.Syyy = h2hi(r2.y);
@@ -657,23 +647,16 @@ __device__ __forceinline__ EwaldLocal ewald_eval(const EwaldRec &R,
 	return e;
 }
 
-/* Ewald_Correction (Gravity/periodic.c:35-113) of a point mass m' whose
- * table record is at hand */
-__device__ __forceinline__ void ewald16_rec(Acc32 &a, const EwaldRec &R,
-		const EwaldNode &c, float m, const Walk32Params &w)
-{
-	const EwaldLocal e = ewald_eval(R, c, w);
-	a.x = fmaf(m * c.sx, e.ex, a.x);
-	a.y = fmaf(m * c.sy, e.ey, a.y);
-	a.z = fmaf(m * c.sz, e.ez, a.z);
-	a.ewald++;
-}
-
+/* Ewald_Correction (Gravity/periodic.c:35-113) of a point mass m' */
 __device__ __forceinline__ void ewald16(Acc32 &a, const float4 *__restrict__ t,
 		float m, float dx, float dy, float dz, const Walk32Params &w)
 {
 	const EwaldNode c = ewald_node(dx, dy, dz, w);
-	ewald16_rec(a, ewald_fetch(t, c), c, m, w);
+	const EwaldLocal e = ewald_local(t, c, w);
+	a.x = fmaf(m * c.sx, e.ex, a.x);
+	a.y = fmaf(m * c.sy, e.ey, a.y);
+	a.z = fmaf(m * c.sz, e.ez, a.z);
+	a.ewald++;
 }
 
 /* The correction of a node of mass m' and traceless second moment T'
@@ -688,7 +671,7 @@ __device__ __forceinline__ void ewald16q(Acc32 &a, const float4 *__restrict__ t,
 		const Walk32Params &w)
 {
 	const EwaldNode c = ewald_node(dx, dy, dz, w);
-	const EwaldLocal e = ewald_eval(ewald_fetch(t, c), c, w);
+	const EwaldLocal e = ewald_local(t, c, w);
 	/* T' (masses G S^2, lengths S) to table units: / (S^4 Box^4), in two
 	 * steps so no constant is subnormal */
 	const float cxx = qa.x * w.inv_s2 * w.inv_s2_box4,
@@ -1701,18 +1684,18 @@ int tdv_walk32(tdv_context *c, int use_bh)
 	const int nparts_h = walk32_parts(ngroups_h, split);
 	const bool parts = nparts_h > 1;
 	/* launch order of the groups: longest expected walk first, from the
-	 * Cost of the last walk, for walks of whole groups that fill the chip
-	 * a few to a few hundred times (a regular step, eager or captured as a
-	 * whole step), where the last groups to start set the end; a split
-	 * walk of few groups and a captured walk for any subset keep the list
-	 * order, and so do walks of more groups, whose neighbours in the list
-	 * then share more of their tree in the caches than the order saves
-	 * (128^3: 88 -> 59 ms, 256^3: 543 -> 524 ms, 512^3 uniform: +0.5%) */
+	 * Cost of the last walk, for walks that fill the chip a few to a few
+	 * hundred times (a regular step, eager or captured as a whole step, the
+	 * groups whole or in a few parts each), where the last groups to start
+	 * set the end; a captured walk for any subset keeps the list order, and
+	 * so do walks of fewer groups, whose many parts are short, and of more,
+	 * whose neighbours in the list then share more of their tree in the
+	 * caches than the order saves (128^3: 88 -> 59 ms, 256^3: 543 -> 524
+	 * ms, 512^3 uniform: +0.5%; in two parts each, 100^3: 36.0 -> 27.0 ms) */
 	const uint32_t *gord = nullptr;
 	const size_t ng_max = (n + 63) / 64;
 	const size_t ng_walk = c->graph_mode ? ng_max : (size_t)ngroups_h;
-	if ((c->graph_mode || (!c->capturing && !parts))
-			&& ng_walk >= TDV_ORDER_MIN_GROUPS
+	if ((c->graph_mode || !c->capturing) && ng_walk >= TDV_ORDER_MIN_GROUPS
 			&& ng_walk <= TDV_ORDER_MAX_GROUPS) {
 		const size_t ng = ng_walk;
 		hipLaunchKernelGGL(k_group_keys, dim3(tdv_blocks(ng, 4)), dim3(256),

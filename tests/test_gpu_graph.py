@@ -323,3 +323,25 @@ def test_split_walk_of_small_top_nodes_matches_whole_walk(n, split):
                / np.linalg.norm(a["acc"][sub], axis=1))
         # FP32 rounding of partial sums, as in the test above
         assert err.max() < 1e-4, (n, split, len(sub), err.max())
+
+
+@pytest.mark.parametrize("split", [0, 3])
+def test_cost_ordered_split_walk_matches_list_order(split):
+    """A split walk of 2048 groups and more starts its groups by descending
+    Cost; the captured walk of the same set, in list order, leaves the same
+    bits."""
+    n = 2048 * 64 + 17
+    g = np.random.Generator(np.random.Philox(22))
+    pos, m = g.uniform(0.0, 1.0, (n, 3)), np.full(n, 1.0 / n)
+    e = _engine(pos, m, 0, split=split, softening=1e-3)
+    ref = e.get("pos", "acc", "last_acc_mag")
+    e.compute_acceleration(False)
+    want, counts = e.get("acc", "cost"), e.interaction_counts()
+    e.update_particles(ref["pos"], acc=ref["acc"],
+                       last_acc_mag=ref["last_acc_mag"])
+    e.capture_walk()
+    e.launch_walk()
+    got = e.get("acc", "cost")
+    np.testing.assert_array_equal(got["acc"], want["acc"])
+    np.testing.assert_array_equal(got["cost"], want["cost"])
+    assert e.interaction_counts() == counts
