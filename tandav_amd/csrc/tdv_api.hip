@@ -271,6 +271,17 @@ static int alloc_top(tdv_context *c, int cap)
 	return 0;
 }
 
+/* the table with each node's three force components side by side */
+__global__ void k_ewald_rows(const double *__restrict__ t,
+		double *__restrict__ rows)
+{
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i >= TDV_NE3)
+		return;
+	for (int d = 0; d < 3; d++)
+		rows[3 * i + d] = t[(size_t)d * TDV_NE3 + i];
+}
+
 static int compute_ewald(tdv_context *c)
 {
 	double *raw = nullptr;
@@ -374,6 +385,7 @@ void tdv_destroy(tdv_context *c)
 	dfree(c->node_c);
 	dfree(c->node_up);
 	dfree(c->ewald);
+	dfree(c->ewald_rows);
 	dfree(c->tl_spline);
 	dfree(c->ewald16);
 	dfree(c->ewald_s);
@@ -1206,8 +1218,13 @@ int tdv_set_ewald_table(tdv_context *c, const double *t4)
 	}
 	if (!c->ewald)
 		TDV_TRY(dalloc(c, &c->ewald, h.size()));
+	if (!c->ewald_rows)
+		TDV_TRY(dalloc(c, &c->ewald_rows, 3 * (size_t)TDV_NE3));
 	TDV_HIP(c, hipMemcpyAsync(c->ewald, h.data(), h.size() * 8,
 			hipMemcpyHostToDevice, c->stream));
+	hipLaunchKernelGGL(k_ewald_rows, dim3(tdv_blocks(TDV_NE3, 256)),
+			dim3(256), 0, c->stream, c->ewald, c->ewald_rows);
+	TDV_HIP(c, hipGetLastError());
 	TDV_HIP(c, hipStreamSynchronize(c->stream));
 	c->ewald_host.swap(h);
 	c->have_ewald = 1;

@@ -147,23 +147,29 @@ __host__ __device__ inline void peano_key_words(double x, double y, double z,
 }
 
 /* Ewald_Correction, Gravity/periodic.c:35-113 (table already / Box^2):
- * the same code on the device (the walks, tdv_ewald_correction) and on
- * the host (tdv_ewald_correction_host) */
-__host__ __device__ inline void ewald_corr(const double *__restrict__ tab,
-		double dx, double dy, double dz, double box2ewald, double f[3])
+ * the table cell of a separation, its trilinear weights and the signs */
+struct EwaldCell {
+	int b;                           /* corner (i, j, k) */
+	double w[8];
+	double sg[3];
+};
+
+__host__ __device__ inline EwaldCell ewald_cell(double dx, double dy,
+		double dz, double box2ewald)
 {
-	double sg[3] = { -1, -1, -1 };
+	EwaldCell c;
+	c.sg[0] = c.sg[1] = c.sg[2] = -1;
 	if (dx < 0) {
 		dx = -dx;
-		sg[0] = 1;
+		c.sg[0] = 1;
 	}
 	if (dy < 0) {
 		dy = -dy;
-		sg[1] = 1;
+		c.sg[1] = 1;
 	}
 	if (dz < 0) {
 		dz = -dz;
-		sg[2] = 1;
+		c.sg[2] = 1;
 	}
 	double u = dx * box2ewald, v = dy * box2ewald, q = dz * box2ewald;
 	int i = (int)u, j = (int)v, k = (int)q;
@@ -176,19 +182,67 @@ __host__ __device__ inline void ewald_corr(const double *__restrict__ tab,
 	u -= i;
 	v -= j;
 	q -= k;
-	const double w0 = (1 - u) * (1 - v) * (1 - q), w1 = (1 - u) * (1 - v) * q,
-			w2 = (1 - u) * v * (1 - q), w3 = (1 - u) * v * q,
-			w4 = u * (1 - v) * (1 - q), w5 = u * (1 - v) * q,
-			w6 = u * v * (1 - q), w7 = u * v * q;
-	const int b = (i * TDV_NE1 + j) * TDV_NE1 + k;
+	c.w[0] = (1 - u) * (1 - v) * (1 - q);
+	c.w[1] = (1 - u) * (1 - v) * q;
+	c.w[2] = (1 - u) * v * (1 - q);
+	c.w[3] = (1 - u) * v * q;
+	c.w[4] = u * (1 - v) * (1 - q);
+	c.w[5] = u * (1 - v) * q;
+	c.w[6] = u * v * (1 - q);
+	c.w[7] = u * v * q;
+	c.b = (i * TDV_NE1 + j) * TDV_NE1 + k;
+	return c;
+}
+
+/* the lookup in the table's own layout, one component after the other (the
+ * host's, tdv_ewald_correction_host) */
+__host__ __device__ inline void ewald_corr(const double *__restrict__ tab,
+		double dx, double dy, double dz, double box2ewald, double f[3])
+{
+	const EwaldCell c = ewald_cell(dx, dy, dz, box2ewald);
+	const double *w = c.w;
 	const int di = TDV_NE1 * TDV_NE1, dj = TDV_NE1;
 #pragma unroll
 	for (int d = 0; d < 3; d++) {
-		const double *F = tab + d * TDV_NE3 + b;
-		f[d] = (w0 * F[0] + w1 * F[1] + w2 * F[dj] + w3 * F[dj + 1]
-				+ w4 * F[di] + w5 * F[di + 1] + w6 * F[di + dj]
-				+ w7 * F[di + dj + 1]) * sg[d];
+		const double *F = tab + d * TDV_NE3 + c.b;
+		f[d] = (w[0] * F[0] + w[1] * F[1] + w[2] * F[dj] + w[3] * F[dj + 1]
+				+ w[4] * F[di] + w[5] * F[di + 1] + w[6] * F[di + dj]
+				+ w[7] * F[di + dj + 1]) * c.sg[d];
 	}
+}
+
+/* The same lookup, bit for bit, in the device's layout, the three components
+ * of a node side by side: the two corners of a cell along z are 48
+ * consecutive bytes, so a lane gathers its eight corners with twelve
+ * 16-byte loads instead of 24 of 8 bytes each (a gather costs the texture
+ * addresser a cycle per lane and load, whatever its width). */
+typedef double double2_a8 __attribute__((ext_vector_type(2), aligned(8)));
+
+__device__ __forceinline__ void ewald_corr_rows(
+		const double *__restrict__ rows, double dx, double dy, double dz,
+		double box2ewald, double f[3])
+{
+	const EwaldCell c = ewald_cell(dx, dy, dz, box2ewald);
+	const double *w = c.w;
+	const int di = 3 * TDV_NE1 * TDV_NE1, dj = 3 * TDV_NE1;
+	const int at[4] = { 0, dj, di, di + dj };
+	double F[4][6];
+#pragma unroll
+	for (int r = 0; r < 4; r++) {
+		const double *R = rows + (3 * c.b + at[r]);
+#pragma unroll
+		for (int h = 0; h < 3; h++) {
+			const double2_a8 v = *reinterpret_cast<const double2_a8 *>(
+					R + 2 * h);
+			F[r][2 * h] = v.x;
+			F[r][2 * h + 1] = v.y;
+		}
+	}
+#pragma unroll
+	for (int d = 0; d < 3; d++)
+		f[d] = (w[0] * F[0][d] + w[1] * F[0][3 + d] + w[2] * F[1][d]
+				+ w[3] * F[1][3 + d] + w[4] * F[2][d] + w[5] * F[2][3 + d]
+				+ w[6] * F[3][d] + w[7] * F[3][3 + d]) * c.sg[d];
 }
 
 /* The node-size rule of create_node_from_particle (tree_build.c:546):

@@ -9,6 +9,7 @@
  * reduction.  Used to state the acceleration error of the walks.
  */
 #include "tdv_internal.h"
+#include "tdv_device.h"
 
 __device__ __forceinline__ double dwrap(double d, int periodic, double box,
 		double half)
@@ -20,44 +21,6 @@ __device__ __forceinline__ double dwrap(double d, int periodic, double box,
 	else if (d < -half)
 		d += box;
 	return d;
-}
-
-__device__ __forceinline__ void dewald(const double *__restrict__ tab,
-		double dx, double dy, double dz, double b2e, double f[3])
-{
-	double sg[3] = { -1, -1, -1 };
-	if (dx < 0) {
-		dx = -dx;
-		sg[0] = 1;
-	}
-	if (dy < 0) {
-		dy = -dy;
-		sg[1] = 1;
-	}
-	if (dz < 0) {
-		dz = -dz;
-		sg[2] = 1;
-	}
-	double u = dx * b2e, v = dy * b2e, q = dz * b2e;
-	int i = (int)u, j = (int)v, k = (int)q;
-	i = i >= TDV_NE ? TDV_NE - 1 : i;
-	j = j >= TDV_NE ? TDV_NE - 1 : j;
-	k = k >= TDV_NE ? TDV_NE - 1 : k;
-	u -= i;
-	v -= j;
-	q -= k;
-	const double w0 = (1 - u) * (1 - v) * (1 - q), w1 = (1 - u) * (1 - v) * q,
-			w2 = (1 - u) * v * (1 - q), w3 = (1 - u) * v * q,
-			w4 = u * (1 - v) * (1 - q), w5 = u * (1 - v) * q,
-			w6 = u * v * (1 - q), w7 = u * v * q;
-	const int b = (i * TDV_NE1 + j) * TDV_NE1 + k;
-	const int di = TDV_NE1 * TDV_NE1, dj = TDV_NE1;
-	for (int d = 0; d < 3; d++) {
-		const double *F = tab + d * TDV_NE3 + b;
-		f[d] = (w0 * F[0] + w1 * F[1] + w2 * F[dj] + w3 * F[dj + 1]
-				+ w4 * F[di] + w5 * F[di + 1] + w6 * F[di + dj]
-				+ w7 * F[di + dj + 1]) * sg[d];
-	}
 }
 
 __global__ void __launch_bounds__(256) k_direct(int nt,
@@ -96,7 +59,7 @@ __global__ void __launch_bounds__(256) k_direct(int nt,
 		az += fac * dz;
 		if (periodic) {
 			double f[3];
-			dewald(tab, dx, dy, dz, b2e, f);
+			ewald_corr(tab, dx, dy, dz, b2e, f);
 			ax += G * q.w * f[0];
 			ay += G * q.w * f[1];
 			az += G * q.w * f[2];

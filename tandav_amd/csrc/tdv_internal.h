@@ -136,6 +136,7 @@ struct tdv_context {
 	int top32_cap;
 
 	double *ewald;                   /* 4 * TDV_NE3, normalised */
+	double *ewald_rows;              /* 3 * TDV_NE3: Fx, Fy, Fz per node */
 	std::vector<double> ewald_host;  /* the same on the host (per-element
 	                                    Ewald_Correction) */
 	int have_ewald;

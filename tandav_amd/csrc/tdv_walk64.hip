@@ -1,6 +1,6 @@
 /*
- * FP64 tree walks, one lane per active particle, reproducing the
- * reference's per-particle decisions and summation order:
+ * FP64 tree walks, a lane or a team of lanes per active particle,
+ * reproducing the reference's per-particle decisions and summation order:
  *   k_walk64        Gravity_Tree_Acceleration (Gravity/tree_accel.c:32-394):
  *                   top-node loop, gravity_tree_walk (relative criterion +
  *                   "inside" test) or gravity_tree_walk_BH, interact()
@@ -36,11 +36,12 @@ __device__ __forceinline__ double wrap(double d, const WalkParams &w)
 }
 
 struct Acc {
-	double x, y, z, cost;
+	double x, y, z;
+	int cost;                        /* interactions */
 };
 
 /* sum of P.Cost over the launch: one atomic per wavefront */
-__device__ __forceinline__ void count_interactions(double cost,
+__device__ __forceinline__ void count_interactions(int cost,
 		unsigned long long *counter)
 {
 	unsigned long long v = (unsigned long long)cost;
@@ -50,9 +51,10 @@ __device__ __forceinline__ void count_interactions(double cost,
 		atomicAdd(counter, v);
 }
 
-/* interact (Gravity/tree_accel.c:362-394): Dehnen K1 kernel, h < 0 */
-__device__ __forceinline__ void interact(Acc &a, double m, double dx,
-		double dy, double dz, double r2, const WalkParams &w)
+/* the factor of an interaction, interact (Gravity/tree_accel.c:362-394):
+ * Dehnen K1 kernel, h < 0 */
+__device__ __forceinline__ double kernel_fac(double m, double r2,
+		const WalkParams &w)
 {
 	double fac = w.G * m;
 	if (r2 < w.eps2) {
@@ -62,32 +64,166 @@ __device__ __forceinline__ void interact(Acc &a, double m, double dx,
 		const double r_inv = 1 / sqrt(r2);
 		fac *= r_inv * r_inv * r_inv;
 	}
+	return fac;
+}
+
+__device__ __forceinline__ void interact(Acc &a, double m, double dx,
+		double dy, double dz, double r2, const WalkParams &w)
+{
+	const double fac = kernel_fac(m, r2, w);
 	a.x += fac * dx;
 	a.y += fac * dy;
 	a.z += fac * dz;
-	a.cost += 1;
+	a.cost++;
 }
 
-/* P-P with the particles [first, last) for the lanes with `on`, in the
- * reference's order; the range is the wavefront's, so the loads are
- * uniform */
+/* ---- lane teams -----------------------------------------------------------
+ *
+ * L lanes work for one particle: a bundle's particles are dealt out to them
+ * L at a time, each lane forms one particle's contribution, and the team's
+ * lanes then all add the L contributions in particle order, taken from one
+ * another by DPP, so the sums round exactly as one lane's would.  A walk is
+ * one long chain of interactions per particle; with one lane each, a few
+ * thousand particles are a few wavefronts that leave most SIMDs idle and
+ * have nothing to hide an interaction's latency behind. */
+template <int ctrl>
+__device__ __forceinline__ double dpp_f64(double v)
+{
+	const uint64_t u = (uint64_t)__double_as_longlong(v);
+	const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, ctrl, 0xf,
+			0xf, false);
+	const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), ctrl, 0xf,
+			0xf, false);
+	return __longlong_as_double((long long)((uint64_t)(uint32_t)hi << 32
+			| (uint32_t)lo));
+}
+
+/* the value of the team's lane S: quad_perm(S, S, S, S) in teams of 4,
+ * row_newbcast S in teams of 16 (a DPP row) */
+template <int L, int S>
+__device__ __forceinline__ double team_lane(double v)
+{
+	return dpp_f64<L == 4 ? S * 0x55 : 0x150 + S>(v);
+}
+
+/* a += the contributions of the team's lanes S .. S + 3, in lane order (a
+ * lane without one holds zeros, which change no sum) */
+template <int L, int S>
+__device__ __forceinline__ void team_add4(Acc &a, double x, double y, double z)
+{
+	a.x += team_lane<L, S>(x);
+	a.y += team_lane<L, S>(y);
+	a.z += team_lane<L, S>(z);
+	a.x += team_lane<L, S + 1>(x);
+	a.y += team_lane<L, S + 1>(y);
+	a.z += team_lane<L, S + 1>(z);
+	a.x += team_lane<L, S + 2>(x);
+	a.y += team_lane<L, S + 2>(y);
+	a.z += team_lane<L, S + 2>(z);
+	a.x += team_lane<L, S + 3>(x);
+	a.y += team_lane<L, S + 3>(y);
+	a.z += team_lane<L, S + 3>(z);
+}
+
+/* a += the first `count` (uniform) of the team's contributions */
+template <int L>
+__device__ __forceinline__ void team_add(Acc &a, double x, double y, double z,
+		bool hit, int count)
+{
+	team_add4<L, 0>(a, x, y, z);
+	if constexpr (L == 16) {
+		if (count > 4)
+			team_add4<L, 4>(a, x, y, z);
+		if (count > 8)
+			team_add4<L, 8>(a, x, y, z);
+		if (count > 12)
+			team_add4<L, 12>(a, x, y, z);
+	}
+	const uint64_t hits = __ballot(hit) >> (threadIdx.x & 63 & ~(L - 1));
+	a.cost += __popcll(hits & ((1ull << L) - 1));
+}
+
+/* P-P with U particles of a uniform range, in the reference's order.  Where
+ * no pair is inside the softening length (and none is the particle itself)
+ * the U roots and divisions, which are most of an interaction, are
+ * independent chains. */
+template <int U>
+__device__ __forceinline__ void pp_batch(Acc &a, const double4 (&q)[U],
+		double px, double py, double pz, const WalkParams &w)
+{
+	double dx[U], dy[U], dz[U], r2[U];
+	bool near = false;
+#pragma unroll
+	for (int u = 0; u < U; u++) {
+		dx[u] = wrap(q[u].x - px, w);
+		dy[u] = wrap(q[u].y - py, w);
+		dz[u] = wrap(q[u].z - pz, w);
+		r2[u] = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u];
+		near = near || !(r2[u] >= w.eps2 && r2[u] > 0);
+	}
+	if (near) {
+#pragma unroll
+		for (int u = 0; u < U; u++)
+			if (r2[u] != 0)
+				interact(a, q[u].w, dx[u], dy[u], dz[u], r2[u], w);
+		return;
+	}
+	double fac[U];
+#pragma unroll
+	for (int u = 0; u < U; u++) {
+		const double r_inv = 1 / sqrt(r2[u]);
+		fac[u] = w.G * q[u].w;
+		fac[u] *= r_inv * r_inv * r_inv;
+	}
+#pragma unroll
+	for (int u = 0; u < U; u++) {
+		a.x += fac[u] * dx[u];
+		a.y += fac[u] * dy[u];
+		a.z += fac[u] * dz[u];
+	}
+	a.cost += U;
+}
+
+/* P-P with the particles [first, last) for the lanes with `on` (a team's
+ * alike), in the reference's order; the range is the wavefront's, so one
+ * lane per particle loads uniformly */
+template <int L>
 __device__ __forceinline__ void pp_range_on(Acc &a, const double4 *pm,
 		int first, int last, double px, double py, double pz, bool on,
 		const WalkParams &w)
 {
-	for (int j = first; j < last; j++) {
-		const double4 q = pm[j];
-		if (!on)
-			continue;
-		const double dx = wrap(q.x - px, w), dy = wrap(q.y - py, w),
-				dz = wrap(q.z - pz, w);
-		const double r2 = dx * dx + dy * dy + dz * dz;
-		if (r2 != 0)
-			interact(a, q.w, dx, dy, dz, r2, w);
+	if constexpr (L == 1) {
+		int j = first;
+		for (; j + 4 <= last; j += 4) {
+			const double4 q[4] = { pm[j], pm[j + 1], pm[j + 2], pm[j + 3] };
+			if (on)
+				pp_batch<4>(a, q, px, py, pz, w);
+		}
+		for (; j < last; j++) {
+			const double4 q[1] = { pm[j] };
+			if (on)
+				pp_batch<1>(a, q, px, py, pz, w);
+		}
+	} else {
+		const int sub = threadIdx.x & (L - 1);
+		double4 n = pm[first + sub < last ? first + sub : last - 1];
+		for (int j = first; j < last; j += L) {
+			const double4 q = n;
+			const int kn = j + L + sub;
+			n = pm[kn < last ? kn : last - 1];
+			if (!on)
+				continue;
+			const double dx = wrap(q.x - px, w), dy = wrap(q.y - py, w),
+					dz = wrap(q.z - pz, w);
+			const double r2 = dx * dx + dy * dy + dz * dz;
+			const bool hit = j + sub < last && r2 != 0;
+			const double fac = hit ? kernel_fac(q.w, r2, w) : 0.0;
+			team_add<L>(a, hit ? fac * dx : 0.0, hit ? fac * dy : 0.0,
+					hit ? fac * dz : 0.0, hit, last - j);
+		}
 	}
 }
 
-/* the smallest value over the wavefront, as a wave-uniform value */
 /* min of v and the value DPP control `ctrl` moves into this lane (INT_MAX
  * where nothing arrives) */
 template <int ctrl, int rows>
@@ -112,7 +248,7 @@ __device__ __forceinline__ int wave_min(int v)
 	return __builtin_amdgcn_readlane(v, 63);
 }
 
-/* One lane per active particle, every lane taking exactly the reference's
+/* A team of L lanes per active particle, taking exactly the reference's
  * walk: its own decisions, its own interactions in its own order.  The
  * wavefront walks in lockstep: each lane keeps the next node of its walk,
  * the wavefront takes the smallest of them (walks only move forward in
@@ -121,6 +257,7 @@ __device__ __forceinline__ int wave_min(int v)
  * neighbours' walks share most nodes, so the wavefront visits little more
  * than one walk's nodes, without the per-lane gathers and divergent
  * branches of independent loops. */
+template <int L>
 __global__ void __launch_bounds__(256) k_walk64(int nact,
 		const int *__restrict__ active, const double4 *__restrict__ pm,
 		const double *__restrict__ last_acc, TopNodes T,
@@ -131,7 +268,7 @@ __global__ void __launch_bounds__(256) k_walk64(int nact,
 		double *__restrict__ gz, double *__restrict__ cost, int npart_total,
 		unsigned *err, unsigned long long *counter)
 {
-	const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+	const int gid = (int)((blockIdx.x * blockDim.x + threadIdx.x) / L);
 	const bool live = gid < nact;
 	const int ip = live ? active[gid] : 0;
 	const double4 p = pm[ip];
@@ -173,7 +310,7 @@ __global__ void __launch_bounds__(256) k_walk64(int nact,
 					atomicOr(err, TDV_EBIT_RANGE);
 				continue;
 			}
-			pp_range_on(a, pm, f, f + T.npart[j], p.x, p.y, p.z, walk, w);
+			pp_range_on<L>(a, pm, f, f + T.npart[j], p.x, p.y, p.z, walk, w);
 			continue;
 		}
 		/* gravity_tree_walk(_BH), Gravity/tree_accel.c:211-353 */
@@ -202,7 +339,7 @@ __global__ void __launch_bounds__(256) k_walk64(int nact,
 					atomicOr(err, TDV_EBIT_RANGE);
 					break;
 				}
-				pp_range_on(a, pm, f, f + c.y, p.x, p.y, p.z, mine, w);
+				pp_range_on<L>(a, pm, f, f + c.y, p.x, p.y, p.z, mine, w);
 				if (mine)
 					next = node + 1;
 				continue;
@@ -237,45 +374,95 @@ __global__ void __launch_bounds__(256) k_walk64(int nact,
 		}
 	}
 	/* add_recv_to, Gravity/tree_accel.c:110-129 */
-	if (live) {
+	const bool mine = live && (threadIdx.x & (L - 1)) == 0;
+	if (mine) {
 		ax[ip] = ax[ip] + a.x;
 		ay[ip] = ay[ip] + a.y;
 		az[ip] = az[ip] + a.z;
 		gx[ip] = a.x;
 		gy[ip] = a.y;
 		gz[ip] = a.z;
-		cost[ip] = a.cost;
+		cost[ip] = (double)a.cost;
 	}
-	count_interactions(a.cost, counter);
+	count_interactions(mine ? a.cost : 0, counter);
 }
 
 __device__ __forceinline__ void ewald_cube(Acc &a, const double *tab,
 		double dx, double dy, double dz, double m, const WalkParams &w)
 {
 	double f[3];
-	ewald_corr(tab, dx, dy, dz, w.box2ewald, f);
+	ewald_corr_rows(tab, dx, dy, dz, w.box2ewald, f);
 	a.x += w.G * m * f[0];
 	a.y += w.G * m * f[1];
 	a.z += w.G * m * f[2];
-	a.cost += 1;
+	a.cost++;
 }
 
+/* as pp_range_on, with the Ewald correction of each pair; one lane per
+ * particle takes two at a time, both gathers in flight */
+template <int L>
 __device__ __forceinline__ void ewald_pp_range_on(Acc &a, const double *tab,
 		const double4 *pm, int first, int last, double px, double py,
 		double pz, bool on, const WalkParams &w)
 {
-	for (int j = first; j < last; j++) {
-		const double4 q = pm[j];
-		if (!on)
-			continue;
-		const double dx = wrap(q.x - px, w), dy = wrap(q.y - py, w),
-				dz = wrap(q.z - pz, w);
-		if (dx != 0 && dy != 0 && dz != 0)
-			ewald_cube(a, tab, dx, dy, dz, q.w, w);
+	constexpr int U = 2;
+	const int sub = threadIdx.x & (L - 1);
+	if constexpr (L == 1) {
+		int j = first;
+		for (; j + U <= last; j += U) {
+			const double4 q[U] = { pm[j], pm[j + 1] };
+			if (!on)
+				continue;
+			double f[U][3];
+			bool hit[U];
+#pragma unroll
+			for (int u = 0; u < U; u++) {
+				const double dx = wrap(q[u].x - px, w),
+						dy = wrap(q[u].y - py, w), dz = wrap(q[u].z - pz, w);
+				hit[u] = dx != 0 && dy != 0 && dz != 0;
+				ewald_corr_rows(tab, dx, dy, dz, w.box2ewald, f[u]);
+			}
+#pragma unroll
+			for (int u = 0; u < U; u++) {
+				if (hit[u]) {
+					a.x += w.G * q[u].w * f[u][0];
+					a.y += w.G * q[u].w * f[u][1];
+					a.z += w.G * q[u].w * f[u][2];
+					a.cost++;
+				}
+			}
+		}
+		for (; j < last; j++) {
+			const double4 q = pm[j];
+			if (!on)
+				continue;
+			const double dx = wrap(q.x - px, w), dy = wrap(q.y - py, w),
+					dz = wrap(q.z - pz, w);
+			if (dx != 0 && dy != 0 && dz != 0)
+				ewald_cube(a, tab, dx, dy, dz, q.w, w);
+		}
+	} else {
+		double4 n = pm[first + sub < last ? first + sub : last - 1];
+		for (int j = first; j < last; j += L) {
+			const double4 q = n;
+			const int kn = j + L + sub;
+			n = pm[kn < last ? kn : last - 1];
+			if (!on)
+				continue;
+			const double dx = wrap(q.x - px, w), dy = wrap(q.y - py, w),
+					dz = wrap(q.z - pz, w);
+			const bool hit = j + sub < last && dx != 0 && dy != 0 && dz != 0;
+			double f[3];
+			ewald_corr_rows(tab, dx, dy, dz, w.box2ewald, f);
+			team_add<L>(a, hit ? w.G * q.w * f[0] : 0.0,
+					hit ? w.G * q.w * f[1] : 0.0,
+					hit ? w.G * q.w * f[2] : 0.0, hit, last - j);
+		}
 	}
 }
 
-/* Gravity_Tree_Periodic per lane, in lockstep as k_walk64 */
+/* Gravity_Tree_Periodic by lane teams, in lockstep as k_walk64 */
+template <int L>
 __global__ void __launch_bounds__(256) k_walk64_ewald(int nact,
 		const int *__restrict__ active, const double4 *__restrict__ pm,
 		const double *__restrict__ last_acc, TopNodes T,
@@ -287,7 +474,7 @@ __global__ void __launch_bounds__(256) k_walk64_ewald(int nact,
 		double *__restrict__ cost, int npart_total, unsigned *err,
 		unsigned long long *counter)
 {
-	const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+	const int gid = (int)((blockIdx.x * blockDim.x + threadIdx.x) / L);
 	const bool live = gid < nact;
 	const int ip = live ? active[gid] : 0;
 	const double4 p = pm[ip];
@@ -336,7 +523,7 @@ __global__ void __launch_bounds__(256) k_walk64_ewald(int nact,
 					atomicOr(err, TDV_EBIT_RANGE);
 				continue;
 			}
-			ewald_pp_range_on(a, tab, pm, f, f + T.npart[j], p.x, p.y, p.z,
+			ewald_pp_range_on<L>(a, tab, pm, f, f + T.npart[j], p.x, p.y, p.z,
 					walk, w);
 			continue;
 		}
@@ -365,7 +552,7 @@ __global__ void __launch_bounds__(256) k_walk64_ewald(int nact,
 					atomicOr(err, TDV_EBIT_RANGE);
 					break;
 				}
-				ewald_pp_range_on(a, tab, pm, f, f + c.y, p.x, p.y, p.z, mine,
+				ewald_pp_range_on<L>(a, tab, pm, f, f + c.y, p.x, p.y, p.z, mine,
 						w);
 				if (mine)
 					next = node + 1 == end ? INT_MAX : node + 1;
@@ -405,16 +592,17 @@ __global__ void __launch_bounds__(256) k_walk64_ewald(int nact,
 		}
 	}
 	/* add_recv_to, Gravity/tree_periodic.c:91-110 */
-	if (live) {
+	const bool mine = live && (threadIdx.x & (L - 1)) == 0;
+	if (mine) {
 		ax[ip] = ax[ip] + a.x;
 		ay[ip] = ay[ip] + a.y;
 		az[ip] = az[ip] + a.z;
 		gx[ip] = gx[ip] + a.x;
 		gy[ip] = gy[ip] + a.y;
 		gz[ip] = gz[ip] + a.z;
-		cost[ip] = cost[ip] + a.cost;
+		cost[ip] = cost[ip] + (double)a.cost;
 	}
-	count_interactions(a.cost, counter);
+	count_interactions(mine ? a.cost : 0, counter);
 }
 
 static WalkParams walk_params(const tdv_context *c, int use_bh)
@@ -438,13 +626,51 @@ static WalkParams walk_params(const tdv_context *c, int use_bh)
 	return w;
 }
 
+/* Lanes per particle and threads per workgroup, from the active count.
+ * Teams buy wavefronts and idle less in the lockstep (fewer particles per
+ * wavefront to wait for); they pay with L instead of one addition per
+ * component for each of the wavefront's pairs, a quarter of the Newton
+ * walk's time with teams of 4 and 1.5 times it with 16, little beside the
+ * Ewald walk's gathers.  Measured in ms for teams of 1, 4 and 16, the walk
+ * with one lane per particle in workgroups of 256 before them in brackets:
+ *   Newton, Hernquist  8192: 1.63, 1.05, 0.88 [2.26]; 14000: 2.56, 1.64,
+ *     1.74 [3.52]; 65536: 4.30, 3.79, 5.23 [5.91]; 10^6: 24.4, 24.0 [30.1]
+ *   Newton, periodic box 24^3: 4.36, 2.21, 2.72 [5.72]; 40^3: 18.8, 19.6,
+ *     38.3 [23.8]; 64^3: 157, 221, 452 [169]
+ *   Ewald, periodic box 24^3: 6.52, 3.47, 3.57 [10.4]; 40^3: 20.2, 19.4,
+ *     23.3 [28.8]; 64^3: 225, 223, 230 [310]; 80^3: 87, 51 [94]
+ * So the Newton walk takes teams of 4 while one lane each would be less
+ * than a wavefront per SIMD (65536 particles), the Ewald walk always, both
+ * teams of 16 up to 10240 particles.  A wavefront per workgroup spreads few
+ * of them over more CUs; the large Newton walks keep four neighbours on one
+ * CU, which share its scalar cache (64^3: 182 ms apart, 157 together). */
+struct Walk64Shape {
+	int team, block;
+};
+
+#define TDV_W64_TEAM16 10240
+#define TDV_W64_TEAM4 65536
+#define TDV_W64_TEAM_MAX (1 << 28)       /* thread numbers within 32 bits */
+
+static Walk64Shape walk64_shape(int nact, bool ewald)
+{
+	if (nact <= TDV_W64_TEAM16)
+		return { 16, 64 };
+	if (nact <= (ewald ? TDV_W64_TEAM_MAX : TDV_W64_TEAM4))
+		return { 4, 64 };
+	return { 1, 256 };
+}
+
 int tdv_walk64(tdv_context *c, int use_bh)
 {
 	if (!c->nactive)
 		return 0;
 	const WalkParams w = walk_params(c, use_bh);
-	hipLaunchKernelGGL(k_walk64, dim3(tdv_blocks((size_t)c->nactive, 256)),
-			dim3(256), 0, c->stream, c->nactive, c->active, c->pm, c->last_acc,
+	const Walk64Shape sh = walk64_shape(c->nactive, false);
+	const int L = sh.team;
+	auto kern = L == 16 ? k_walk64<16> : L == 4 ? k_walk64<4> : k_walk64<1>;
+	hipLaunchKernelGGL(kern, dim3(tdv_blocks((size_t)c->nactive * L, sh.block)),
+			dim3(sh.block), 0, c->stream, c->nactive, c->active, c->pm, c->last_acc,
 			c->top, c->node_a, c->node_b, c->node_c, w, c->acc[0], c->acc[1],
 			c->acc[2], c->gacc[0], c->gacc[1], c->gacc[2], c->cost, (int)c->n,
 			c->d_err, c->d_count);
@@ -458,12 +684,15 @@ int tdv_walk64_ewald(tdv_context *c, int use_bh)
 	if (!c->have_ewald)
 		return tdv_fail(c, TDV_ERR_ARG, "periodic walk without an Ewald table");
 	const WalkParams w = walk_params(c, use_bh);
-	hipLaunchKernelGGL(k_walk64_ewald,
-			dim3(tdv_blocks((size_t)c->nactive, 256)), dim3(256), 0, c->stream,
-			c->nactive, c->active, c->pm, c->last_acc, c->top, c->node_a,
-			c->node_b, c->node_c, c->ewald, w, c->acc[0], c->acc[1], c->acc[2],
-			c->gacc[0], c->gacc[1], c->gacc[2], c->cost, (int)c->n, c->d_err,
-			c->d_count + 1);
+	const Walk64Shape sh = walk64_shape(c->nactive, true);
+	const int L = sh.team;
+	auto kern = L == 16 ? k_walk64_ewald<16> : L == 4 ? k_walk64_ewald<4>
+			: k_walk64_ewald<1>;
+	hipLaunchKernelGGL(kern, dim3(tdv_blocks((size_t)c->nactive * L, sh.block)),
+			dim3(sh.block), 0, c->stream, c->nactive, c->active, c->pm, c->last_acc,
+			c->top, c->node_a, c->node_b, c->node_c, c->ewald_rows, w,
+			c->acc[0], c->acc[1], c->acc[2], c->gacc[0], c->gacc[1],
+			c->gacc[2], c->cost, (int)c->n, c->d_err, c->d_count + 1);
 	return tdv_check(c, hipGetLastError(), "k_walk64_ewald");
 }
 
@@ -499,7 +728,7 @@ __global__ void k_ewald_correction_batch(size_t n, const double *__restrict__ dr
 	if (i >= n)
 		return;
 	double r[3];
-	ewald_corr(tab, dr[3 * i], dr[3 * i + 1], dr[3 * i + 2], b2e, r);
+	ewald_corr_rows(tab, dr[3 * i], dr[3 * i + 1], dr[3 * i + 2], b2e, r);
 	f[3 * i] = r[0];
 	f[3 * i + 1] = r[1];
 	f[3 * i + 2] = r[2];
@@ -509,6 +738,6 @@ void tdv_launch_ewald_correction(tdv_context *c, size_t n, const double *dr,
 		double *f)
 {
 	hipLaunchKernelGGL(k_ewald_correction_batch, dim3(tdv_blocks(n, 256)),
-			dim3(256), 0, c->stream, n, dr, f, c->ewald,
+			dim3(256), 0, c->stream, n, dr, f, c->ewald_rows,
 			2 * TDV_NE / c->par.boxsize);
 }

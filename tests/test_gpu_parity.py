@@ -225,3 +225,39 @@ def test_set_domain_and_sort_particles():
     perm = oracle.qsort_index(keys, nthreads=4)
     np.testing.assert_array_equal(got["id"], perm.astype(np.uint32))
     np.testing.assert_array_equal(got["pos"], pos[perm])
+
+
+@pytest.mark.parametrize("periodic", [False, True])
+def test_lane_teams_leave_the_same_bits(periodic, ewald):
+    """The FP64 walks with 1, 4 and 16 lanes per particle (by the number of
+    active particles): every particle's sums round alike."""
+    n = 65536 + 77
+    if periodic:
+        pos, _, m = ics.clustered_box(n, nhalo=16, seed=11)
+        kw = dict(ewald_table=ewald, softening=1e-3)
+    else:
+        pos, _, m = ics.hernquist_sphere(n, seed=1)
+        kw = dict(softening=0.05)        # many pairs inside it
+    e = Engine(periodic=periodic, alpha_rel=0.02, **kw)
+    e.set_particles(pos, m)
+    e.setup_domain()
+    e.domain_decomposition()
+    e.compute_acceleration(True)
+    ref = e.get("pos", "last_acc_mag")
+
+    def walk(sub):
+        e.set_active(sub)
+        e.update_particles(ref["pos"], acc=np.zeros((n, 3)),
+                           last_acc_mag=ref["last_acc_mag"])
+        e.tree_acceleration(False)
+        got = e.get("acc", "cost")
+        return got["acc"][sub], got["cost"][sub], e.interaction_counts()
+
+    acc, cost, _ = walk(np.arange(n, dtype=np.int32))
+    for k in (65536, 65535, 10241, 10240, 129, 1):
+        sub = np.sort(np.random.Generator(np.random.Philox(k)).choice(
+            n, k, replace=False)).astype(np.int32)
+        a, c, counts = walk(sub)
+        np.testing.assert_array_equal(a, acc[sub], err_msg=str(k))
+        np.testing.assert_array_equal(c, cost[sub], err_msg=str(k))
+        assert sum(counts) == int(c.sum())
