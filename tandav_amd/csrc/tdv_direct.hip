@@ -4,12 +4,22 @@
  * over every other particle of the path's own pairwise kernel (K1 with the
  * negative softening length, Gravity/tree_accel.c:362-394), plus, on
  * periodic runs, the tabulated Ewald correction of every pair (nearest image
- * + Ewald_Correction, Gravity/periodic.c:35-113).  One workgroup per target;
- * lanes stride over the sources and the partial sums meet in a block
- * reduction.  Used to state the acceleration error of the walks.
+ * + Ewald_Correction, Gravity/periodic.c:35-113).  The sources are cut into
+ * parts, one workgroup per target and part; lanes stride over a part's
+ * sources, the sums meet in a block reduction and the parts' sums are added
+ * in part order.  Used to state the acceleration error of the walks.
  */
 #include "tdv_internal.h"
 #include "tdv_device.h"
+#include <algorithm>
+
+/* Two workgroups per CU keep the table's gathers busy, which bound a pair
+ * (more of them only spread the sources' separations over more of the table:
+ * 512 targets in 64^3 particles take 3.4 ms in one part each, 3.7 in four);
+ * with fewer targets than that the sources are cut into parts of at least
+ * TDV_DIRECT_MIN (16 targets 1.56 -> 0.15 ms, 100 targets 1.72 -> 0.95 ms). */
+#define TDV_DIRECT_BLOCKS 512
+#define TDV_DIRECT_MIN 2048
 
 __device__ __forceinline__ double dwrap(double d, int periodic, double box,
 		double half)
@@ -26,17 +36,21 @@ __device__ __forceinline__ double dwrap(double d, int periodic, double box,
 __global__ void __launch_bounds__(256) k_direct(int nt,
 		const int *__restrict__ idx, const double4 *__restrict__ pm, int n,
 		int periodic, double box, double G, double eps2, double eps3,
-		const double *__restrict__ tab, double b2e, double *__restrict__ out)
+		const double *__restrict__ tab, double b2e, int chunk,
+		double *__restrict__ out)
 {
 	__shared__ double red[3][256];
 	const int t = blockIdx.x;
 	if (t >= nt)
 		return;
+	/* this part's sources; its sums go to row blockIdx.y of out */
+	const int first = (int)blockIdx.y * chunk;
+	const int last = n - first < chunk ? n : first + chunk;
 	const int i = idx[t];
 	const double4 p = pm[i];
 	const double half = box / 2.0;
 	double ax = 0, ay = 0, az = 0;
-	for (int j = threadIdx.x; j < n; j += blockDim.x) {
+	for (int j = first + threadIdx.x; j < last; j += blockDim.x) {
 		if (j == i)
 			continue;
 		const double4 q = pm[j];
@@ -77,7 +91,19 @@ __global__ void __launch_bounds__(256) k_direct(int nt,
 	}
 	if (threadIdx.x == 0)
 		for (int d = 0; d < 3; d++)
-			out[3 * t + d] = red[d][0];
+			out[3 * ((size_t)blockIdx.y * nt + t) + d] = red[d][0];
+}
+
+__global__ void k_direct_parts(int n3, int nparts,
+		const double *__restrict__ part, double *__restrict__ out)
+{
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i >= n3)
+		return;
+	double s = part[i];
+	for (int k = 1; k < nparts; k++)
+		s += part[(size_t)k * n3 + i];
+	out[i] = s;
 }
 
 int tdv_direct_sum(tdv_context *c, int nt, const int *idx_dev, double *out_dev)
@@ -86,9 +112,23 @@ int tdv_direct_sum(tdv_context *c, int nt, const int *idx_dev, double *out_dev)
 		return 0;
 	if (c->par.periodic && !c->have_ewald)
 		return tdv_fail(c, TDV_ERR_ARG, "direct sum without an Ewald table");
-	hipLaunchKernelGGL(k_direct, dim3(nt), dim3(256), 0, c->stream, nt,
-			idx_dev, c->pm, (int)c->n, c->par.periodic, c->par.boxsize,
-			c->par.gravity, c->Epsilon2, c->Epsilon3, c->ewald,
-			2 * TDV_NE / (c->par.periodic ? c->par.boxsize : 1.0), out_dev);
+	/* parts, their sums in the sort's scratch (cap words, free here) */
+	const size_t n = c->n;
+	size_t parts = std::min({ (size_t)(TDV_DIRECT_BLOCKS / nt),
+		n / TDV_DIRECT_MIN, c->cap / (3 * (size_t)nt) });
+	if (parts < 1)
+		parts = 1;
+	const int chunk = (int)((n + parts - 1) / parts);
+	parts = (n + chunk - 1) / chunk;
+	double *sums = parts > 1 ? reinterpret_cast<double *>(c->sk[0]) : out_dev;
+	hipLaunchKernelGGL(k_direct, dim3(nt, (unsigned)parts), dim3(256), 0,
+			c->stream, nt, idx_dev, c->pm, (int)n, c->par.periodic,
+			c->par.boxsize, c->par.gravity, c->Epsilon2, c->Epsilon3,
+			c->ewald, 2 * TDV_NE / (c->par.periodic ? c->par.boxsize : 1.0),
+			chunk, sums);
+	if (parts > 1)
+		hipLaunchKernelGGL(k_direct_parts, dim3(tdv_blocks(3 * (size_t)nt,
+				256)), dim3(256), 0, c->stream, 3 * nt, (int)parts, sums,
+				out_dev);
 	return tdv_check(c, hipGetLastError(), "k_direct");
 }

@@ -272,3 +272,16 @@ def test_fp32_bundles_taken_whole():
     from tandav_amd import TDVError
     with pytest.raises(TDVError):
         Engine(precision="fp32", compat=False, fp32_bundle_min=65)
+
+
+@pytest.mark.parametrize("nt", [1, 5, 256, 257])
+def test_forcetest_in_parts_matches_whole(nt):
+    """Few targets have their sources cut into parts; many are summed whole:
+    the same terms, summed in another order."""
+    pos, _, m = ics.zeldovich_box(24, seed=7)
+    e = Engine(periodic=True, softening=1 / 960.)
+    e.set_particles(pos, m)
+    e.setup_domain()
+    many = e.forcetest(np.arange(600))
+    got = e.forcetest(np.arange(nt))
+    assert rel_err(got, many[:nt]).max() < 1e-11
