@@ -356,7 +356,7 @@ int tdv_create(const tdv_params *p, tdv_context **out)
 	if (!r)
 		r = dalloc(c, &c->long_count, 2);
 	if (!r)
-		r = dalloc(c, &c->q_arrived, 192);
+		r = dalloc(c, &c->lvl, TDV_LVL_WORDS);
 	if (!r)
 		r = tdv_check(c, hipMemset(c->d_err, 0, sizeof(unsigned)), "memset");
 	if (!r)
@@ -397,7 +397,7 @@ void tdv_destroy(tdv_context *c)
 	dfree(c->ctr32);
 	dfree(c->q32);
 	dfree(c->q_s6);
-	dfree(c->q_arrived);
+	dfree(c->lvl);
 	dfree(c->lvl_nodes);
 	dfree(c->tq32);
 	dfree(c->top32);
@@ -987,14 +987,16 @@ int tdv_launch_step(tdv_context *c)
 	(void)hipEventRecord(c->ev[EV_KEYS0], c->stream);
 	TDV_HIP(c, hipGraphLaunch(c->step_exec, c->stream));
 	(void)hipEventRecord(c->ev[EV_KICK1], c->stream);
+	/* the level counts are this tree's from now on */
 	int h[2];
 	TDV_HIP(c, hipMemcpyAsync(&h[0], c->top.ntop, sizeof(int),
 			hipMemcpyDeviceToHost, c->stream));
-	TDV_HIP(c, hipMemcpyAsync(&h[1], c->top.nnodes, sizeof(int),
+	TDV_HIP(c, hipMemcpyAsync(c->lvl_host, c->lvl, sizeof(c->lvl_host),
 			hipMemcpyDeviceToHost, c->stream));
 	TDV_HIP(c, hipMemcpyAsync(c->count, c->d_count, sizeof(c->count),
 			hipMemcpyDeviceToHost, c->stream));
 	TDV_HIP(c, hipStreamSynchronize(c->stream));
+	h[1] = (int)c->lvl_host[TDV_LVL_NODES];
 	float ms = 0.f;
 	(void)hipEventElapsedTime(&ms, c->ev[EV_KEYS0], c->ev[EV_KICK1]);
 	for (int k = 0; k < 8; k++)

@@ -232,59 +232,90 @@ __global__ void __launch_bounds__(256) k_tree_marks(size_t n,
 __global__ void __launch_bounds__(256) k_tree_counts(size_t n,
 		const uint64_t *__restrict__ key, TopNodes T, int vs,
 		const uint32_t *__restrict__ minpack, uint32_t *__restrict__ cnt,
-		int *__restrict__ lohi)
+		int *__restrict__ lohi, unsigned *__restrict__ lvl_cnt)
 {
+	/* nodes per level, gathered per block first */
+	__shared__ unsigned h[64];
+	if (threadIdx.x < 64)
+		h[threadIdx.x] = 0;
+	__syncthreads();
 	const size_t gi = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (gi >= n)
-		return;
-	const int i = (int)gi;
-	const TopRange r = top_of(key, gi, T, vs);
-	if (!r.tree) {
-		cnt[i] = 0;
-		lohi[i] = 0;
-		return;
+	if (gi < n) {
+		const int i = (int)gi;
+		const TopRange r = top_of(key, gi, T, vs);
+		const int lo = r.tree ? dprev_of(key, i, r.first, r.level) : TDV_NT;
+		int c = 0, pack = 0;
+		if (lo < TDV_NT) {               /* else no subtree, or dumped: no
+		                                    node of its own */
+			const int dn = (i == r.last) ? -1 : div_level(load_key(key, i),
+					load_key(key, i + 1));
+			const int lf = lo > dn ? lo : dn;
+			const uint32_t mp = minpack[i];
+			const int ml = (mp == NOCOLLAPSE) ? 99 : (int)(mp >> 24);
+			const int hi = lf < ml ? lf : ml;
+			c = hi >= lo ? hi - lo + 1 : 0;
+			pack = lo | (hi << 8) | ((ml <= lf) ? (1 << 16) : 0);
+			for (int lv = lo; lv <= hi; lv++)
+				atomicAdd(&h[lv], 1u);
+		}
+		cnt[i] = (uint32_t)c;
+		lohi[i] = pack;
 	}
-	const int lo = dprev_of(key, i, r.first, r.level);
-	if (lo >= TDV_NT) {              /* dumped: no node of its own */
-		cnt[i] = 0;
-		lohi[i] = 0;
-		return;
-	}
-	const int dn = (i == r.last) ? -1 : div_level(load_key(key, i),
-			load_key(key, i + 1));
-	const int lf = lo > dn ? lo : dn;
-	const uint32_t mp = minpack[i];
-	const int ml = (mp == NOCOLLAPSE) ? 99 : (int)(mp >> 24);
-	const int hi = lf < ml ? lf : ml;
-	const int c = hi >= lo ? hi - lo + 1 : 0;
-	cnt[i] = (uint32_t)c;
-	lohi[i] = lo | (hi << 8) | ((ml <= lf) ? (1 << 16) : 0);
+	__syncthreads();
+	if (threadIdx.x < 64 && h[threadIdx.x])
+		atomicAdd(&lvl_cnt[threadIdx.x], h[threadIdx.x]);
 }
 
-/* the node ranges of the top nodes' subtrees; more nodes than `cap` (a
- * captured step's arrays) set the node count to -1, which every later
- * kernel of the step reads as "do nothing", and raise TDV_EBIT_RANGE */
+/* the node ranges of the top nodes' subtrees, one wavefront (a scan over 64
+ * top nodes at a time: a single lane's loads in turn took 31 us of 64 top
+ * nodes, this 4); more nodes than `cap` (a captured step's arrays) set the
+ * node count to -1, which every later kernel of the step reads as "do
+ * nothing", and raise TDV_EBIT_RANGE.  Also the levels' list offsets and
+ * fill counters, and the node count and error flags for the host beside the
+ * level counts. */
 __global__ void __launch_bounds__(64) k_tree_targets(TopNodes T, int vs,
-		const uint32_t *__restrict__ off, long long cap, unsigned *err)
+		const uint32_t *__restrict__ off, long long cap, unsigned *err,
+		unsigned *__restrict__ lvl)
 {
-	if (threadIdx.x != 0)
-		return;
+	const int lane = threadIdx.x;
 	const int ntop = *T.ntop;
 	long long run = 0;
-	for (int t = 0; t < ntop; t++) {
+	for (int t0 = 0; t0 < ntop; t0 += 64) {
+		const int t = t0 + lane;
 		long long sz = 0;
-		if (T.npart[t] > vs)
+		if (t < ntop && T.npart[t] > vs)
 			sz = (long long)(off[T.first[t] + T.npart[t]]
 					- off[T.first[t]]) + 1;
-		T.target[t] = (int)run;      /* reserve_tree_memory(nNeeded) */
-		T.term[t] = (int)(run + sz - 1);
-		run += sz;
+		long long inc = sz;
+		for (int d = 1; d < 64; d <<= 1) {
+			const long long o = __shfl_up(inc, d, 64);
+			if (lane >= d)
+				inc += o;
+		}
+		if (t < ntop) {
+			T.target[t] = (int)(run + inc - sz);  /* reserve_tree_memory */
+			T.term[t] = (int)(run + inc - 1);
+		}
+		run += __shfl(inc, 63, 64);
 	}
-	if (run > cap) {
-		atomicOr(err, TDV_EBIT_RANGE);
-		*T.nnodes = -1;
-	} else {
-		*T.nnodes = (int)run;
+	int lv = (int)lvl[lane];
+	for (int d = 1; d < 64; d <<= 1) {
+		const int o = __shfl_up(lv, d, 64);
+		if (lane >= d)
+			lv += o;
+	}
+	lvl[TDV_LVL_OFF + lane] = (unsigned)lv - lvl[lane];
+	lvl[TDV_LVL_FILL + lane] = 0;
+	const bool over = run > cap;
+	if (over)
+		lvl[lane] = 0;                   /* no nodes, no lists */
+	if (lane == 0) {
+		if (over)
+			atomicOr(err, TDV_EBIT_RANGE);
+		const int nn = over ? -1 : (int)run;
+		*T.nnodes = nn;
+		lvl[TDV_LVL_NODES] = (unsigned)nn;
+		lvl[TDV_LVL_ERR] = atomicOr(err, 0u);
 	}
 }
 
@@ -300,11 +331,15 @@ __global__ void k_clear_nodes(size_t bound, const TopNodes T,
 	}
 }
 
-__global__ void k_fill_u32_val(size_t n, uint32_t *__restrict__ p, uint32_t v)
+/* no particle collapsed yet, no node in any level */
+__global__ void k_build_clear(size_t n, uint32_t *__restrict__ minpack,
+		unsigned *__restrict__ lvl_cnt)
 {
 	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	if (i < n)
-		p[i] = v;
+		minpack[i] = NOCOLLAPSE;
+	if (i < 64)
+		lvl_cnt[i] = 0;
 }
 
 __device__ __forceinline__ int node_index(const TopNodes &T, int t, int first,
@@ -618,7 +653,7 @@ __global__ void __launch_bounds__(64) k_tree_nodes_long(
  * key shares the cell with key_i); the head's own parent (a level-(lo-1)
  * cell, owned by the particle that starts it) is found the same way
  * backwards.  The centres of mass come afterwards, bottom-up over the
- * levels (k_com_level): a sum in tree order instead of the reference's
+ * levels (k_com_levels): a sum in tree order instead of the reference's
  * insertion order, which the FP64 walk keeps bit for bit and the FP32 walk
  * does not need. */
 
@@ -723,16 +758,19 @@ __device__ __forceinline__ void com_add_strided(const double *__restrict__ x,
 	}
 }
 
-/* Centres of mass and masses of one level's nodes, eight lanes per node,
- * from the children (one level deeper, done by the launch before) and the
- * particles no child covers; a fixed grid strides over the level's list. */
-__global__ void __launch_bounds__(256) k_com_level(int lv,
-		const unsigned *__restrict__ lcnt, const int *__restrict__ loff,
+/* Centres of mass and masses of the nodes of levels lv0 down to lv1, eight
+ * lanes per node, from the children (one level deeper, done before) and the
+ * particles no child covers; the grid strides over a level's list.  Several
+ * levels only in one workgroup, whose barrier orders them (tdv_level_runs). */
+__global__ void __launch_bounds__(TDV_LVL_THREADS) k_com_levels(int lv0,
+		int lv1, const unsigned *__restrict__ lcnt,
+		const int *__restrict__ loff,
 		const int *__restrict__ list, const int4 *__restrict__ nc,
 		const double *__restrict__ x, const double *__restrict__ y,
 		const double *__restrict__ z, const double *__restrict__ m,
-		double4 *__restrict__ na)
+		double4 *na)
 {
+	for (int lv = lv0; lv >= lv1; lv--, __syncthreads()) {
 	const int count = (int)lcnt[lv];
 	const int base = loff[lv];
 	for (int t0 = (blockIdx.x * blockDim.x) >> 3; t0 < count;
@@ -771,6 +809,7 @@ __global__ void __launch_bounds__(256) k_com_level(int lv,
 				s[k] += __shfl_xor(s[k], d, 8);
 		if (on && sub == 0)
 			na[j] = make_double4(s[1] / s[0], s[2] / s[0], s[3] / s[0], s[0]);
+	}
 	}
 }
 
@@ -886,6 +925,43 @@ __global__ void __launch_bounds__(256) k_tree_centres(size_t bound,
 	nb[j] = make_double4(cx, cy, cz, dom_size / (double)(1ull << lv));
 }
 
+/* The launches of a pass over the levels, deepest first.  A level is a
+ * kernel of its own, so that the next finds its results; most of the 43
+ * hold no or few nodes, and a launch costs more than their work (43 of each
+ * of the two passes took 0.34 ms and their gaps of a 65,536-particle step).
+ * Runs of levels of up to TDV_LVL_FEW nodes are taken by one workgroup in
+ * one launch, and what the counts of the last eager build call empty above
+ * and below is part of such runs.  In a captured step those counts are a
+ * guess: any plan is right for any tree, only slower. */
+std::vector<LevelRun> tdv_level_runs(const tdv_context *c, size_t bound)
+{
+	std::vector<LevelRun> runs;
+	int first = -1, last = -1;
+	for (int lv = 0; lv <= TDV_NT; lv++)
+		if (c->lvl_host[lv]) {
+			if (first < 0)
+				first = lv;
+			last = lv;
+		}
+	if (c->graph_mode) {             /* levels the guess says are empty too */
+		first = 0;
+		last = TDV_NT;
+	}
+	for (int lv = last; lv >= first && lv >= 0; lv--) {
+		const unsigned cnt = c->lvl_host[lv];
+		if (cnt > TDV_LVL_FEW) {
+			const size_t nodes = c->graph_mode ? bound : (size_t)cnt;
+			runs.push_back({ lv, lv, (unsigned)std::min(
+					(size_t)tdv_blocks(8 * nodes, 256), (size_t)2048), 256 });
+		} else if (!runs.empty() && runs.back().threads == TDV_LVL_THREADS) {
+			runs.back().lv1 = lv;
+		} else {
+			runs.push_back({ lv, lv, 1, TDV_LVL_THREADS });
+		}
+	}
+	return runs;
+}
+
 /* The build.  Eagerly it reads the node count back to size the node
  * arrays; in a captured step (c->graph_mode) the arrays keep the capacity
  * of the last eager build and every kernel takes the counts from device
@@ -896,25 +972,26 @@ int tdv_build_tree(tdv_context *c)
 	const int vs = c->par.vector_size;
 	const bool graph = c->graph_mode != 0;
 	c->lvl_ok = 0;                       /* the FP32 walk's level lists */
-	hipLaunchKernelGGL(k_fill_u32_val, dim3(tdv_blocks(n, 256)), dim3(256), 0,
-			c->stream, n, c->minpack, 0xFFFFFFFFu);
+	hipLaunchKernelGGL(k_build_clear, dim3(tdv_blocks(n, 256)), dim3(256), 0,
+			c->stream, n, c->minpack, c->lvl);
 	hipLaunchKernelGGL(k_tree_marks, dim3(tdv_blocks(n, 256)), dim3(256), 0,
 			c->stream, n, c->key, c->top, vs, c->minpack, c->d_err);
 	hipLaunchKernelGGL(k_tree_counts, dim3(tdv_blocks(n, 256)), dim3(256), 0,
 			c->stream, n, c->key, c->top, vs, c->minpack,
-			reinterpret_cast<uint32_t *>(c->cnt), c->lohi);
+			reinterpret_cast<uint32_t *>(c->cnt), c->lohi, c->lvl);
 	TDV_TRY(tdv_scan_u32(c, reinterpret_cast<uint32_t *>(c->cnt), c->off, n));
 	hipLaunchKernelGGL(k_tree_targets, dim3(1), dim3(64), 0, c->stream, c->top,
 			vs, c->off, graph ? (long long)c->node_cap : (1ll << 62),
-			c->d_err);
+			c->d_err, c->lvl);
 	TDV_HIP(c, hipGetLastError());
 	size_t bound = c->node_cap;          /* nodes the kernels may touch */
 	if (!graph) {
-		int nn = 0;
-		TDV_HIP(c, hipMemcpyAsync(&nn, c->top.nnodes, sizeof(int),
+		TDV_HIP(c, hipMemcpyAsync(c->lvl_host, c->lvl, sizeof(c->lvl_host),
 				hipMemcpyDeviceToHost, c->stream));
 		TDV_HIP(c, hipStreamSynchronize(c->stream));
-		TDV_TRY(tdv_check_err_flags(c));
+		if (c->lvl_host[TDV_LVL_ERR])
+			TDV_TRY(tdv_check_err_flags(c));
+		const int nn = (int)c->lvl_host[TDV_LVL_NODES];
 		TDV_TRY(tdv_ensure_nodes(c, (size_t)nn));
 		c->nnodes = (size_t)nn;
 		bound = (size_t)nn;
@@ -946,12 +1023,10 @@ int tdv_build_tree(tdv_context *c)
 				c->node_c, c->node_up);
 		if (bound > 0) {
 			TDV_TRY(tdv_level_lists(c, bound));
-			const unsigned grid = (unsigned)std::min(
-					(size_t)tdv_blocks(8 * bound, 256), (size_t)2048);
-			for (int lv = TDV_NT; lv >= 0; lv--)
-				hipLaunchKernelGGL(k_com_level, dim3(grid), dim3(256), 0,
-						c->stream, lv, c->q_arrived,
-						reinterpret_cast<const int *>(c->q_arrived + 128),
+			for (const LevelRun &r : tdv_level_runs(c, bound))
+				hipLaunchKernelGGL(k_com_levels, dim3(r.grid),
+						dim3(r.threads), 0, c->stream, r.lv0, r.lv1, c->lvl,
+						reinterpret_cast<const int *>(c->lvl + TDV_LVL_OFF),
 						c->lvl_nodes, c->node_c, c->pos[0], c->pos[1],
 						c->pos[2], c->mass, c->node_a);
 		}

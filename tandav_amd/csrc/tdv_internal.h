@@ -36,6 +36,16 @@
                                    24 (longer runs per digit store better;
                                    the LDS staging fits two blocks per CU) */
 
+/* the words of tdv_context::lvl: nodes per level in [0, 64), then */
+#define TDV_LVL_FILL 64      /* their lists' fill counters, */
+#define TDV_LVL_OFF 128      /* the lists' offsets, */
+#define TDV_LVL_NODES 192    /* the node count (-1: over capacity) and */
+#define TDV_LVL_ERR 193      /* the error flags after the node count */
+#define TDV_LVL_WORDS 194
+#define TDV_LVL_FEW 512      /* levels of up to this many nodes share a
+                                launch of one workgroup */
+#define TDV_LVL_THREADS 1024
+
 /* stage events of a context (stage_ms: keys, sort, reorder, top nodes,
  * build, walk, Ewald walk, kick/drift) */
 enum { EV_KEYS0, EV_KEYS1, EV_SORT1, EV_REORDER1, EV_TOP1, EV_BUILD0,
@@ -89,12 +99,11 @@ struct tdv_context {
 	uint32_t *gorder;                /* groups by descending expected cost */
 	size_t gcap;                     /* groups gkey and gorder hold */
 	double *q_s6;                    /* nodes' FP64 second moments, 6 each */
-	unsigned *q_arrived;             /* per level: counts [0, 64), fill
-	                                    counters [64, 128), list offsets
-	                                    [128, 192) */
+	unsigned *lvl;                   /* TDV_LVL_WORDS: nodes per level, ... */
 	int *lvl_nodes;                  /* node indices grouped by level */
 	size_t lvl_cap;                  /* nodes lvl_nodes holds */
 	int lvl_ok;                      /* the lists match the tree */
+	unsigned lvl_host[TDV_LVL_WORDS];    /* lvl of the last eager build */
 	int substep_prep;                /* capturing a substep walk: the
 	                                    quadrupoles and cell centres kept */
 	hipGraph_t graph;                /* captured regular-step walk */
@@ -201,8 +210,14 @@ int tdv_build_top_nodes(tdv_context *c);
 int tdv_assign_top(tdv_context *c);
 int tdv_build_tree(tdv_context *c);
 /* the tree's per-level node lists (lvl_nodes, counts and offsets in
- * q_arrived), on the device; sets lvl_ok */
+ * lvl), on the device; sets lvl_ok */
 int tdv_level_lists(tdv_context *c, size_t bound);
+/* launches of a bottom-up pass over the levels lv0 .. lv1 */
+struct LevelRun {
+	int lv0, lv1;
+	unsigned grid, threads;
+};
+std::vector<LevelRun> tdv_level_runs(const tdv_context *c, size_t bound);
 
 /* ---- launchers (tdv_walk64.hip, tdv_ewald.hip) ---- */
 int tdv_walk64(tdv_context *c, int use_bh);

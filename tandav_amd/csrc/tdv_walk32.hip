@@ -262,7 +262,7 @@ __global__ void k_prep32_particles(size_t n, const double4 *__restrict__ pm,
  * S^2 masses, fixed lengths) as {Txx, Tyy, Txy, Txz}, {Tyz, 0, 0, 0}; Tzz =
  * -Txx - Tyy.
  *
- * Bottom-up in O(nodes + particles), one launch per tree level from the
+ * Bottom-up in O(nodes + particles), level by level from the
  * deepest: every node covers the contiguous particle range [first, first +
  * Npart) and its children (one level deeper: the nodes from j + 1 below
  * j + DNext, siblings linked by DNext, bundles by + 1) cover sub-ranges of
@@ -327,14 +327,17 @@ __device__ __forceinline__ void moments_add_strided(
  * child covers and every eighth child term, then the eight partial sums
  * meet in a fixed butterfly (the same order on every run; every lane ends
  * with the same sums, addition being commutative). */
-__global__ void __launch_bounds__(256) k_moments_level(int lv,
-		const unsigned *__restrict__ lcnt, const int *__restrict__ loff,
+__global__ void __launch_bounds__(TDV_LVL_THREADS) k_moments_levels(int lv0,
+		int lv1, const unsigned *__restrict__ lcnt,
+		const int *__restrict__ loff,
 		const int *__restrict__ list, const int4 *__restrict__ nc,
 		const double4 *__restrict__ na, const double4 *__restrict__ pm,
-		double *__restrict__ s6, double scale, float4 *__restrict__ q)
+		double *s6, double scale, float4 *__restrict__ q)
 {
-	/* the level's nodes, count and list offset on the device; a fixed grid
-	 * strides over them */
+	/* a level's nodes, count and list offset on the device; a fixed grid
+	 * strides over them.  Several levels only in one workgroup, whose
+	 * barrier orders them (tdv_level_runs) */
+	for (int lv = lv0; lv >= lv1; lv--, __syncthreads()) {
 	const int count = (int)lcnt[lv];
 	const int base = loff[lv];
 	for (int t0 = (blockIdx.x * blockDim.x) >> 3; t0 < count;
@@ -384,46 +387,11 @@ __global__ void __launch_bounds__(256) k_moments_level(int lv,
 		moments_store(m6, scale, q + 2 * j);
 	}
 	}
-}
-
-/* exclusive offsets of the per-level counts, and the fill counters
- * cleared (one lane) */
-__global__ void k_level_offsets(const unsigned *__restrict__ cnt,
-		int *__restrict__ off, unsigned *__restrict__ fill)
-{
-	if (threadIdx.x != 0)
-		return;
-	int run = 0;
-	for (int lv = 0; lv < 64; lv++) {
-		off[lv] = run;
-		run += (int)cnt[lv];
-		fill[lv] = 0;
 	}
 }
 
-/* per-level node lists (terminators left out); counts are gathered per
- * block in LDS first, so the device-wide counters take one atomic per level
- * and block */
-__global__ void __launch_bounds__(256) k_level_count(int bound,
-		const int *__restrict__ nnd, const int4 *__restrict__ nc,
-		unsigned *__restrict__ cnt)
-{
-	__shared__ unsigned h[64];
-	const int nn = min(bound, *nnd);
-	const int j = blockIdx.x * blockDim.x + threadIdx.x;
-	if (threadIdx.x < 64)
-		h[threadIdx.x] = 0;
-	__syncthreads();
-	if (j < nn) {
-		const int4 c = nc[j];
-		if (c.w >= 0)
-			atomicAdd(&h[c.z & 63], 1u);
-	}
-	__syncthreads();
-	if (threadIdx.x < 64 && h[threadIdx.x])
-		atomicAdd(&cnt[threadIdx.x], h[threadIdx.x]);
-}
-
+/* the per-level node lists (terminators left out), each block's places
+ * taken with one atomic per level */
 __global__ void __launch_bounds__(256) k_level_fill(int bound,
 		const int *__restrict__ nnd, const int4 *__restrict__ nc,
 		const int *__restrict__ off, unsigned *__restrict__ fill,
@@ -1435,13 +1403,6 @@ __global__ void __launch_bounds__(256) k_group_keys(
 	}
 }
 
-__global__ void k_fill_u32(int n, unsigned *__restrict__ p)
-{
-	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < n)
-		p[i] = 0;
-}
-
 __global__ void k_walk32_queue_reset(unsigned *__restrict__ queue,
 		unsigned long long *__restrict__ counter)
 {
@@ -1451,9 +1412,8 @@ __global__ void k_walk32_queue_reset(unsigned *__restrict__ queue,
 		counter[threadIdx.x] = 0;
 }
 
-/* The per-level node lists, once per build: counts, offsets, fill, all on
- * the device (the node count is read there too, so a captured step can
- * rebuild them). */
+/* The per-level node lists, once per build, from the counts and offsets the
+ * build leaves in lvl (on the device, so a captured step can rebuild them) */
 int tdv_level_lists(tdv_context *c, size_t bound)
 {
 	if (c->lvl_cap < c->node_cap) {
@@ -1468,18 +1428,10 @@ int tdv_level_lists(tdv_context *c, size_t bound)
 				c->node_cap * sizeof(int)));
 		c->lvl_cap = c->node_cap;
 	}
-	unsigned *cnt = c->q_arrived, *fill = c->q_arrived + 64;
-	int *off = reinterpret_cast<int *>(c->q_arrived + 128);
-	hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(128), 0, c->stream, 128,
-			c->q_arrived);
-	hipLaunchKernelGGL(k_level_count, dim3(tdv_blocks(bound, 256)),
-			dim3(256), 0, c->stream, (int)bound, c->top.nnodes, c->node_c,
-			cnt);
-	hipLaunchKernelGGL(k_level_offsets, dim3(1), dim3(64), 0, c->stream, cnt,
-			off, fill);
 	hipLaunchKernelGGL(k_level_fill, dim3(tdv_blocks(bound, 256)), dim3(256),
-			0, c->stream, (int)bound, c->top.nnodes, c->node_c, off, fill,
-			c->lvl_nodes);
+			0, c->stream, (int)bound, c->top.nnodes, c->node_c,
+			reinterpret_cast<const int *>(c->lvl + TDV_LVL_OFF),
+			c->lvl + TDV_LVL_FILL, c->lvl_nodes);
 	TDV_HIP(c, hipGetLastError());
 	c->lvl_ok = 1;
 	return 0;
@@ -1598,12 +1550,10 @@ int tdv_walk32(tdv_context *c, int use_bh)
 			TDV_TRY(tdv_level_lists(c, bound));
 		/* bottom-up: a level's nodes take their children's moments */
 		if (bound) {
-			const unsigned grid = (unsigned)std::min(
-					(size_t)tdv_blocks(8 * bound, 256), (size_t)2048);
-			for (int lv = TDV_NT; lv >= 0; lv--)
-				hipLaunchKernelGGL(k_moments_level, dim3(grid), dim3(256), 0,
-						c->stream, lv, c->q_arrived,
-						reinterpret_cast<const int *>(c->q_arrived + 128),
+			for (const LevelRun &r : tdv_level_runs(c, bound))
+				hipLaunchKernelGGL(k_moments_levels, dim3(r.grid),
+						dim3(r.threads), 0, c->stream, r.lv0, r.lv1, c->lvl,
+						reinterpret_cast<const int *>(c->lvl + TDV_LVL_OFF),
 						c->lvl_nodes, c->node_c, c->node_a, c->pm, c->q_s6,
 						qscale, c->q32);
 		}
