@@ -347,6 +347,8 @@ int tdv_create(const tdv_params *p, tdv_context **out)
 		r = tdv_check(c, hipEventCreate(&c->ev[e]), "hipEventCreate");
 	if (!r)
 		r = dalloc(c, &c->d_err, 1);
+	if (!r && !p->periodic)
+		r = dalloc(c, &c->select, 1);
 	if (!r)
 		r = dalloc(c, &c->d_count, 4);
 	if (!r)
@@ -402,6 +404,7 @@ void tdv_destroy(tdv_context *c)
 	dfree(c->tq32);
 	dfree(c->top32);
 	tdv_graph_drop(c);
+	dfree(c->select);
 	dfree(c->d_err);
 	dfree(c->d_count);
 	dfree(c->d_nactive);

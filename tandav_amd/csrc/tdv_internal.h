@@ -57,6 +57,15 @@ enum { EV_KEYS0, EV_KEYS1, EV_SORT1, EV_REORDER1, EV_TOP1, EV_BUILD0,
 #define TDV_EBIT_RANGE 4u
 #define TDV_EBIT_TIES 8u
 
+#define TDV_SELECT_BINS 2048 /* bins of the median selection's digit */
+struct SelectState {         /* the selection of the three medians, device */
+	uint64_t prefix[3];      /* the key's digits found so far */
+	unsigned long long maxd; /* largest distance from the centre, as bits */
+	uint64_t k[3];           /* rank among the keys with that prefix */
+	unsigned done;           /* workgroups that have counted */
+	unsigned hist[3 * TDV_SELECT_BINS];
+};
+
 struct TopNodes {            /* device arrays, top_cap entries each */
 	int *first, *npart, *level, *target, *term;
 	uint64_t *key;
@@ -166,6 +175,7 @@ struct tdv_context {
 	                                    {E, J, S} in kernel units */
 	int ewald16_ok;                  /* ewald16 matches ewald */
 
+	SelectState *select;             /* non-periodic domain */
 	unsigned *d_err;
 	unsigned long long *d_count;     /* [4] interactions: tree, Ewald;
 	                                    FP32 walk: of which multipole nodes,

@@ -15,6 +15,8 @@
 #include "tdv_internal.h"
 #include "tdv_device.h"
 
+#include <algorithm>
+#include <cstddef>
 #include <cstring>
 #include <mutex>
 
@@ -706,33 +708,136 @@ void tdv_launch_pack_pm(tdv_context *c)
 /* non-periodic domain (domain.c:751-847, select.c:19-80)                    */
 /* ------------------------------------------------------------------------ */
 
-/* order-preserving u64 image of a double */
-__global__ void k_f64_orderkey(size_t n, const double *__restrict__ x,
-		uint64_t *__restrict__ out)
+/* order-preserving u64 image of a double, and back */
+__device__ __forceinline__ uint64_t f64_orderkey(double x)
 {
-	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	const uint64_t u = (uint64_t)__double_as_longlong(x[i]);
-	out[i] = (u >> 63) ? ~u : (u | (1ull << 63));
+	const uint64_t u = (uint64_t)__double_as_longlong(x);
+	return (u >> 63) ? ~u : (u | (1ull << 63));
 }
 
-__global__ void k_max_dist(size_t n, const double *__restrict__ x,
-		const double *__restrict__ y, const double *__restrict__ z, double cx,
-		double cy, double cz, unsigned long long *out)
+__host__ __device__ inline uint64_t f64_from_orderkey(uint64_t u)
 {
-	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	double v = 0;
-	if (i < n)
-		v = fmax(fmax(fabs(x[i] - cx), fabs(y[i] - cy)), fabs(z[i] - cz));
+	return (u >> 63) ? (u & ~(1ull << 63)) : ~u;
+}
+
+/* The k-th smallest of each of the three coordinates by radix selection: a
+ * pass counts the next digit of the keys that share the prefix found so
+ * far, and the last workgroup to finish extends the prefix by the digit
+ * whose bin holds the k-th.  Six passes over 24 bytes per particle and one
+ * launch each for all three; sorting each coordinate to read one element
+ * took 24 radix passes of five launches, 1.1 ms of a 65,536-particle step.
+ * Leaves the counters cleared for the next pass. */
+#define SEL_BITS 11
+#define SEL_BINS TDV_SELECT_BINS
+#define SEL_THREADS 256
+static_assert(SEL_BINS == 1 << SEL_BITS, "bins of a digit");
+
+__global__ void k_select_init(SelectState *st, uint64_t k)
+{
+	for (int i = threadIdx.x; i < 3 * SEL_BINS; i += blockDim.x)
+		st->hist[i] = 0;
+	if (threadIdx.x < 3) {
+		st->prefix[threadIdx.x] = 0;
+		st->k[threadIdx.x] = k;
+	}
+	if (threadIdx.x == 0) {
+		st->done = 0;
+		st->maxd = 0;
+	}
+}
+
+__global__ void __launch_bounds__(SEL_THREADS) k_select_pass(size_t n,
+		const double *__restrict__ x, const double *__restrict__ y,
+		const double *__restrict__ z, int shift, int bits, SelectState *st)
+{
+	__shared__ unsigned h[3 * SEL_BINS];
+	__shared__ unsigned wsum[SEL_THREADS / 64];
+	__shared__ unsigned last;
+	const int tid = threadIdx.x;
+	for (int i = tid; i < 3 * SEL_BINS; i += SEL_THREADS)
+		h[i] = 0;
+	const double *col[3] = { x, y, z };
+	uint64_t prefix[3];
+	for (int d = 0; d < 3; d++)
+		prefix[d] = st->prefix[d];
+	__syncthreads();
+	const int above = shift + bits;      /* the prefix's lowest bit */
+	const unsigned mask = (1u << bits) - 1;
+	for (size_t i = (size_t)blockIdx.x * SEL_THREADS + tid; i < n;
+			i += (size_t)gridDim.x * SEL_THREADS)
+#pragma unroll
+		for (int d = 0; d < 3; d++) {
+			const uint64_t u = f64_orderkey(col[d][i]);
+			if (above >= 64 || (u >> above) == prefix[d])
+				atomicAdd(&h[d * SEL_BINS + ((unsigned)(u >> shift) & mask)],
+						1u);
+		}
+	__syncthreads();
+	for (int i = tid; i < 3 * SEL_BINS; i += SEL_THREADS)
+		if (h[i])
+			atomicAdd(&st->hist[i], h[i]);
+	__threadfence();                     /* the counts before the ticket */
+	__syncthreads();
+	if (tid == 0)
+		last = atomicAdd(&st->done, 1u) == gridDim.x - 1;
+	__syncthreads();
+	if (!last)
+		return;
+	/* the last workgroup: every count is in; read past this XCD's L2 */
+	constexpr int PER = SEL_BINS / SEL_THREADS;
+	for (int d = 0; d < 3; d++) {
+		unsigned c[PER], sum = 0;
+#pragma unroll
+		for (int u = 0; u < PER; u++) {
+			unsigned *p = &st->hist[d * SEL_BINS + tid * PER + u];
+			c[u] = __hip_atomic_load(p, __ATOMIC_RELAXED,
+					__HIP_MEMORY_SCOPE_AGENT);
+			sum += c[u];
+		}
+		unsigned tot;
+		const unsigned before = block_excl_scan(sum, &tot, wsum);
+		const uint64_t k = st->k[d];
+		__syncthreads();                 /* k read by all before it changes */
+		if (k >= before && k < (uint64_t)before + sum) {
+			unsigned b = before;
+			int u = 0;
+			while (k >= (uint64_t)b + c[u])
+				b += c[u++];
+			st->k[d] = k - b;
+			st->prefix[d] = prefix[d] << bits | (unsigned)(tid * PER + u);
+		}
+	}
+	__syncthreads();
+	for (int i = tid; i < 3 * SEL_BINS; i += SEL_THREADS)
+		st->hist[i] = 0;
+	if (tid == 0)
+		st->done = 0;
+}
+
+/* the largest distance on an axis from the centre just found */
+__global__ void k_max_dist(size_t n, const double *__restrict__ x,
+		const double *__restrict__ y, const double *__restrict__ z,
+		SelectState *st)
+{
+	double c[3];
+	for (int d = 0; d < 3; d++)
+		c[d] = __longlong_as_double((long long)f64_from_orderkey(
+				st->prefix[d]));
 	/* non-negative doubles order like their bit patterns */
-	unsigned long long b = (unsigned long long)__double_as_longlong(v);
+	unsigned long long b = 0;
+	for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+			i += (size_t)gridDim.x * blockDim.x) {
+		const unsigned long long v = (unsigned long long)__double_as_longlong(
+				fmax(fmax(fabs(x[i] - c[0]), fabs(y[i] - c[1])),
+				fabs(z[i] - c[2])));
+		b = v > b ? v : b;
+	}
 	for (int d = 32; d >= 1; d >>= 1) {
 		unsigned long long o = __shfl_xor(b, d, 64);
 		b = o > b ? o : b;
 	}
 	if ((threadIdx.x & 63) == 0)
-		atomicMax(out, b);
+		atomicMax(&st->maxd, b);
 }
 
 int tdv_domain_nonperiodic(tdv_context *c)
@@ -743,32 +848,31 @@ int tdv_domain_nonperiodic(tdv_context *c)
 	/* Select(n>>1, n, data) orders data[1..n-1] and returns position n>>1 of
 	 * that 1-based range, i.e. the ((n>>1)-1)-th smallest of data[1..n-1] */
 	const size_t m = n - 1, k = (n >> 1) - 1;
-	uint64_t *tmp = c->key_tmp;
-	for (int d = 0; d < 3; d++) {
-		hipLaunchKernelGGL(k_f64_orderkey, dim3(tdv_blocks(m, 256)), dim3(256),
-				0, c->stream, m, c->pos[d] + 1, tmp);
-		int res;
-		TDV_TRY(radix_sort_u64(c, context_work(c, nullptr), m, tmp, 1, 0,
-				nullptr, &res));
-		uint64_t u;
-		TDV_HIP(c, hipMemcpyAsync(&u, c->sk[res] + k, 8, hipMemcpyDeviceToHost,
-				c->stream));
-		TDV_HIP(c, hipStreamSynchronize(c->stream));
-		u = (u >> 63) ? (u & ~(1ull << 63)) : ~u;
-		double v;
-		memcpy(&v, &u, 8);
-		c->dom_center[d] = v;
+	SelectState *st = c->select;
+	const unsigned grid = (unsigned)std::min((size_t)tdv_blocks(m, 1024),
+			(size_t)512);
+	hipLaunchKernelGGL(k_select_init, dim3(1), dim3(1024), 0, c->stream, st,
+			(uint64_t)k);
+	for (int above = 64; above > 0; ) {
+		const int bits = above < SEL_BITS ? above : SEL_BITS;
+		above -= bits;
+		hipLaunchKernelGGL(k_select_pass, dim3(grid), dim3(SEL_THREADS), 0,
+				c->stream, m, c->pos[0] + 1, c->pos[1] + 1, c->pos[2] + 1,
+				above, bits, st);
 	}
-	unsigned long long *dmax = reinterpret_cast<unsigned long long *>(tmp);
-	TDV_HIP(c, hipMemsetAsync(dmax, 0, 8, c->stream));
-	hipLaunchKernelGGL(k_max_dist, dim3(tdv_blocks(n, 256)), dim3(256), 0,
-			c->stream, n, c->pos[0], c->pos[1], c->pos[2], c->dom_center[0],
-			c->dom_center[1], c->dom_center[2], dmax);
-	unsigned long long b;
-	TDV_HIP(c, hipMemcpyAsync(&b, dmax, 8, hipMemcpyDeviceToHost, c->stream));
+	hipLaunchKernelGGL(k_max_dist, dim3(grid), dim3(SEL_THREADS), 0,
+			c->stream, n, c->pos[0], c->pos[1], c->pos[2], st);
+	TDV_HIP(c, hipGetLastError());
+	SelectState h;
+	TDV_HIP(c, hipMemcpyAsync(&h, st, offsetof(SelectState, k),
+			hipMemcpyDeviceToHost, c->stream));
 	TDV_HIP(c, hipStreamSynchronize(c->stream));
+	for (int d = 0; d < 3; d++) {
+		const uint64_t u = f64_from_orderkey(h.prefix[d]);
+		memcpy(&c->dom_center[d], &u, 8);
+	}
 	double maxd;
-	memcpy(&maxd, &b, 8);
+	memcpy(&maxd, &h.maxd, 8);
 	c->dom_size = 2.001 * maxd;
 	for (int d = 0; d < 3; d++)
 		c->dom_origin[d] = c->dom_center[d] - 0.5 * c->dom_size;

@@ -261,3 +261,29 @@ def test_lane_teams_leave_the_same_bits(periodic, ewald):
         np.testing.assert_array_equal(a, acc[sub], err_msg=str(k))
         np.testing.assert_array_equal(c, cost[sub], err_msg=str(k))
         assert sum(counts) == int(c.sum())
+
+
+@pytest.mark.parametrize("n", [3, 4, 5, 257, 1025, 70001])
+@pytest.mark.parametrize("kind", ["signed", "ties", "spread"])
+def test_medians_by_selection_match_oracle(n, kind):
+    """The non-periodic domain's centre (order statistics of data[1..n-1])
+    and size, bit for bit: both signs, many equal coordinates, exponents
+    over the whole range of the radix selection's digits."""
+    g = np.random.Generator(np.random.Philox(n))
+    if kind == "signed":
+        pos = g.normal(0.0, 1.0, (n, 3))
+    elif kind == "ties":
+        pos = g.integers(-2, 3, (n, 3)) * 0.25
+        pos[-1] = (3.0, -5.0, 7.0)       # a domain of nonzero size
+    else:
+        pos = g.choice([-1.0, 1.0], (n, 3)) * 10.0 ** g.uniform(-200, 100,
+                                                               (n, 3))
+    e = Engine(periodic=False)
+    e.set_particles(pos, np.full(n, 1.0 / n))
+    e.setup_domain()
+    size, origin, center = e.domain
+    c, s, o = oracle.domain_nonperiodic(*(np.ascontiguousarray(pos[:, d])
+                                          for d in range(3)))
+    np.testing.assert_array_equal(center, c)
+    assert size == s
+    np.testing.assert_array_equal(origin, o)
