@@ -7,7 +7,8 @@
  *
  * Sort: LSD radix sort, 8-bit digits, over the high 64 key bits with a
  * 32-bit payload (the original index), 8 passes of histogram -> scan ->
- * stable scatter.  Runs of equal high words are then ordered by the low
+ * stable scatter (few tiles: the scatter sums the histograms itself; one
+ * tile: all passes in one workgroup's LDS).  Runs of equal high words are then ordered by the low
  * word; equal full keys raise TDV_ERR_DUP_KEYS (the reference's quicksort
  * is unstable, sort.c:253-341, so only unique keys have a defined order).
  * Traffic per pass: 12 B read (histogram) + 12 B read + 12 B written.
@@ -225,6 +226,9 @@ __device__ __forceinline__ unsigned rs_tile(unsigned b, unsigned nb)
 	return x < r ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
 }
 
+/* BY_TILE: the counts of a tile side by side (the scatter sums them), else
+ * digit-major for the device-wide scan */
+template <bool BY_TILE>
 __global__ void __launch_bounds__(RS_THREADS) k_rs_hist(
 		const uint64_t *__restrict__ keys, int stride, int off, size_t n,
 		int shift, uint32_t *__restrict__ hist, unsigned nblocks)
@@ -249,39 +253,121 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_hist(
 			atomicAdd(&h[(unsigned)(kk[it] >> shift) & 255u], 1u);
 	}
 	__syncthreads();
-	hist[(size_t)threadIdx.x * nblocks + tile] = h[threadIdx.x];
+	hist[BY_TILE ? (size_t)tile * RS_BINS + threadIdx.x
+			: (size_t)threadIdx.x * nblocks + tile] = h[threadIdx.x];
 }
 
-/* One LSD pass's scatter of a tile of RS_TILE keys: every key's rank
- * among the tile's keys of its digit (stable: waves, items and lanes in
- * input order), the tile sorted by digit in LDS, then written out in that
- * order, so consecutive threads store consecutive positions of a digit's
- * run (one run of ~16 keys per digit and tile) instead of every lane a
- * key of its own digit somewhere else. */
+/* exclusive prefix sum over the 256 digits of the first four waves' v
+ * (thread d holds digit d's), every thread of the workgroup taking part */
+__device__ __forceinline__ uint32_t rs_digit_scan(uint32_t v,
+		uint32_t *wsum)
+{
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+	uint32_t x = v;
+#pragma unroll
+	for (int o = 1; o < 64; o <<= 1) {
+		const uint32_t y = __shfl_up(x, o, 64);
+		if (lane >= o)
+			x += y;
+	}
+	if (lane == 63 && w < 4)
+		wsum[w] = x;
+	__syncthreads();
+	uint32_t before = 0;
+	for (int q = 0; q < w && q < 4; q++)
+		before += wsum[q];
+	return before + x - v;
+}
+
+/* A workgroup's tile of THREADS x ITEMS keys in LDS */
+template <int THREADS, int ITEMS>
+struct RsShared {
+	uint32_t wcnt[THREADS / 64][RS_BINS];
+	uint32_t dstart[RS_BINS];            /* digit's first slot in the tile */
+	uint32_t wsum[4];
+	uint64_t skey[THREADS * ITEMS];
+	uint32_t sval[THREADS * ITEMS];
+};
+
+/* The tile's keys sorted by one digit into LDS: every key's rank among the
+ * tile's keys of its digit (stable: waves, items and lanes in input order),
+ * then the digits' runs one after the other.  Wave w's item it of lane l is
+ * the tile's key (w ITEMS + it) 64 + l; the first nvalid keys count. */
+template <int THREADS, int ITEMS>
+__device__ __forceinline__ void rs_sort_tile(RsShared<THREADS, ITEMS> &sh,
+		const uint64_t (&kk)[ITEMS], const uint32_t (&vv)[ITEMS], int nvalid,
+		int shift)
+{
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+	for (int q = threadIdx.x; q < THREADS / 64 * RS_BINS; q += THREADS)
+		sh.wcnt[q / RS_BINS][q % RS_BINS] = 0;
+	__syncthreads();
+	uint32_t rk[ITEMS];
+	const uint64_t lt = (1ull << lane) - 1;
+#pragma unroll
+	for (int it = 0; it < ITEMS; it++) {
+		const bool valid = (w * ITEMS + it) * 64 + lane < nvalid;
+		const unsigned d = (unsigned)(kk[it] >> shift) & 255u;
+		uint64_t peers = __ballot(valid);
+#pragma unroll
+		for (int b = 0; b < 8; b++) {
+			const uint64_t bal = __ballot((d >> b) & 1u);
+			peers &= ((d >> b) & 1u) ? bal : ~bal;
+		}
+		const uint32_t below = (uint32_t)__popcll(peers & lt);
+		const int leader = peers ? (__ffsll((unsigned long long)peers) - 1) : 0;
+		uint32_t old = 0;
+		if (valid && below == 0)
+			old = atomicAdd(&sh.wcnt[w][d], (uint32_t)__popcll(peers));
+		old = __shfl(old, leader, 64);
+		rk[it] = old + below;
+	}
+	__syncthreads();
+	/* per digit: the waves' exclusive prefix, and the tile's count, whose
+	 * exclusive scan over the digits places each digit's run in the tile */
+	uint32_t cnt = 0;
+	if (threadIdx.x < RS_BINS)
+		for (int q = 0; q < THREADS / 64; q++) {
+			const uint32_t t = sh.wcnt[q][threadIdx.x];
+			sh.wcnt[q][threadIdx.x] = cnt;
+			cnt += t;
+		}
+	const uint32_t start = rs_digit_scan(cnt, sh.wsum);
+	if (threadIdx.x < RS_BINS)
+		sh.dstart[threadIdx.x] = start;
+	__syncthreads();
+#pragma unroll
+	for (int it = 0; it < ITEMS; it++)
+		if ((w * ITEMS + it) * 64 + lane < nvalid) {
+			const unsigned d = (unsigned)(kk[it] >> shift) & 255u;
+			const uint32_t slot = sh.dstart[d] + sh.wcnt[w][d] + rk[it];
+			sh.skey[slot] = kk[it];
+			sh.sval[slot] = vv[it];
+		}
+	__syncthreads();
+}
+
+/* One LSD pass's scatter of a tile of RS_TILE keys: the tile sorted by
+ * digit in LDS, then written out in that order, so consecutive threads
+ * store consecutive positions of a digit's run (one run of ~16 keys per
+ * digit and tile) instead of every lane a key of its own digit somewhere
+ * else.  BY_TILE: where a tile's runs go is summed here from all tiles'
+ * counts (thread d digit d's), else read from the scanned histogram. */
+template <bool BY_TILE>
 __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(
 		const uint64_t *__restrict__ kin, int stride, int off,
 		const uint32_t *__restrict__ vin, uint64_t *__restrict__ kout,
 		uint32_t *__restrict__ vout, size_t n, int shift,
 		const uint32_t *__restrict__ hscan, unsigned nblocks)
 {
-	__shared__ uint32_t wcnt[RS_WAVES][RS_BINS];
+	__shared__ RsShared<RS_THREADS, RS_ITEMS> sh;
 	__shared__ uint32_t binoff[RS_BINS];
-	__shared__ uint32_t dstart[RS_BINS];     /* digit's first slot in tile */
-	__shared__ uint32_t wsum[RS_WAVES];
-	__shared__ uint64_t skey[RS_TILE];
-	__shared__ uint32_t sval[RS_TILE];
 	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-	for (int q = 0; q < RS_WAVES; q++)
-		wcnt[q][threadIdx.x] = 0;
 	const unsigned tile = rs_tile(blockIdx.x, nblocks);
-	binoff[threadIdx.x] = hscan[(size_t)threadIdx.x * nblocks + tile];
-	__syncthreads();
-
-	const size_t base = (size_t)tile * RS_TILE + (size_t)w * 64 * RS_ITEMS;
+	const size_t tile0 = (size_t)tile * RS_TILE;
+	const size_t base = tile0 + (size_t)w * 64 * RS_ITEMS;
 	uint64_t kk[RS_ITEMS];
 	uint32_t vv[RS_ITEMS];
-	uint32_t rk[RS_ITEMS];
-	const uint64_t lt = (1ull << lane) - 1;
 	/* all of the wave's loads in flight at once: unconditional, at an
 	 * index clamped into [0, n) (n >= 1); what lies past n is not used */
 #pragma unroll
@@ -300,70 +386,72 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(
 		for (int it = 0; it < RS_ITEMS; it++)
 			vv[it] = (uint32_t)(base + (size_t)it * 64 + lane);
 	}
-#pragma unroll
-	for (int it = 0; it < RS_ITEMS; it++) {
-		const size_t i = base + (size_t)it * 64 + lane;
-		const bool valid = i < n;
-		const unsigned d = (unsigned)(kk[it] >> shift) & 255u;
-		uint64_t peers = __ballot(valid);
-#pragma unroll
-		for (int b = 0; b < 8; b++) {
-			const uint64_t bal = __ballot((d >> b) & 1u);
-			peers &= ((d >> b) & 1u) ? bal : ~bal;
+	if (BY_TILE) {
+		uint32_t before = 0, all = 0;
+#pragma unroll 8
+		for (unsigned t = 0; t < nblocks; t++) {
+			const uint32_t h = hscan[(size_t)t * RS_BINS + threadIdx.x];
+			before += t < tile ? h : 0;
+			all += h;
 		}
-		const uint32_t below = (uint32_t)__popcll(peers & lt);
-		const int leader = peers ? (__ffsll((unsigned long long)peers) - 1) : 0;
-		uint32_t old = 0;
-		if (valid && below == 0)
-			old = atomicAdd(&wcnt[w][d], (uint32_t)__popcll(peers));
-		old = __shfl(old, leader, 64);
-		rk[it] = old + below;
+		binoff[threadIdx.x] = rs_digit_scan(all, sh.wsum) + before;
+	} else {
+		binoff[threadIdx.x] = hscan[(size_t)threadIdx.x * nblocks + tile];
 	}
-	__syncthreads();
-	/* per digit: the waves' exclusive prefix, and the tile's count, whose
-	 * exclusive scan over the digits places each digit's run in the tile */
-	uint32_t cnt = 0;
-	for (int q = 0; q < RS_WAVES; q++) {
-		const uint32_t t = wcnt[q][threadIdx.x];
-		wcnt[q][threadIdx.x] = cnt;
-		cnt += t;
-	}
-	uint32_t x = cnt;
-#pragma unroll
-	for (int o = 1; o < 64; o <<= 1) {
-		const uint32_t y = __shfl_up(x, o, 64);
-		if (lane >= o)
-			x += y;
-	}
-	if (lane == 63)
-		wsum[w] = x;
-	__syncthreads();
-	uint32_t before = 0;
-	for (int q = 0; q < w; q++)
-		before += wsum[q];
-	dstart[threadIdx.x] = before + x - cnt;
-	__syncthreads();
-#pragma unroll
-	for (int it = 0; it < RS_ITEMS; it++) {
-		const size_t i = base + (size_t)it * 64 + lane;
-		if (i < n) {
-			const unsigned d = (unsigned)(kk[it] >> shift) & 255u;
-			const uint32_t slot = dstart[d] + wcnt[w][d] + rk[it];
-			skey[slot] = kk[it];
-			sval[slot] = vv[it];
-		}
-	}
-	__syncthreads();
-	const size_t tile0 = (size_t)tile * RS_TILE;
 	const int nvalid = n - tile0 < (size_t)RS_TILE ? (int)(n - tile0)
 			: RS_TILE;
+	__syncthreads();
+	rs_sort_tile<RS_THREADS, RS_ITEMS>(sh, kk, vv, nvalid, shift);
 	for (int j = threadIdx.x; j < nvalid; j += RS_THREADS) {
-		const uint64_t k = skey[j];
+		const uint64_t k = sh.skey[j];
 		const unsigned d = (unsigned)(k >> shift) & 255u;
-		const uint32_t pos = binoff[d] + ((uint32_t)j - dstart[d]);
+		const uint32_t pos = binoff[d] + ((uint32_t)j - sh.dstart[d]);
 		if (pos < n) {                       /* always, by construction */
 			kout[pos] = k;
-			vout[pos] = sval[j];
+			vout[pos] = sh.sval[j];
+		}
+	}
+}
+
+/* All passes of up to RS_TILE keys in one workgroup: each pass sorts the
+ * tile by its digit in LDS and reads it back in that order.  A launch costs
+ * more than a pass of so few keys (a 4096-particle step 1.11 -> 0.95 ms). */
+#define RS1_THREADS 1024
+#define RS1_ITEMS (RS_TILE / RS1_THREADS)
+static_assert(RS1_THREADS * RS1_ITEMS == RS_TILE, "one tile");
+
+__global__ void __launch_bounds__(RS1_THREADS) k_rs_one_tile(
+		const uint64_t *__restrict__ kin, int stride, int off,
+		const uint32_t *__restrict__ vin, uint64_t *__restrict__ kout,
+		uint32_t *__restrict__ vout, int n)
+{
+	__shared__ RsShared<RS1_THREADS, RS1_ITEMS> sh;
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+	const int base = w * 64 * RS1_ITEMS + lane;
+	uint64_t kk[RS1_ITEMS];
+	uint32_t vv[RS1_ITEMS];
+#pragma unroll
+	for (int it = 0; it < RS1_ITEMS; it++) {
+		const int i = base + it * 64;
+		kk[it] = rs_load(kin, (size_t)(i < n ? i : n - 1), stride, off);
+		vv[it] = vin ? vin[i < n ? i : n - 1] : (uint32_t)i;
+	}
+	for (int shift = 0; shift < 64; shift += 8) {
+		rs_sort_tile<RS1_THREADS, RS1_ITEMS>(sh, kk, vv, n, shift);
+#pragma unroll
+		for (int it = 0; it < RS1_ITEMS; it++) {
+			const int i = base + it * 64;
+			kk[it] = sh.skey[i < n ? i : n - 1];
+			vv[it] = sh.sval[i < n ? i : n - 1];
+		}
+		__syncthreads();
+	}
+#pragma unroll
+	for (int it = 0; it < RS1_ITEMS; it++) {
+		const int i = base + it * 64;
+		if (i < n) {
+			kout[i] = kk[it];
+			vout[i] = vv[it];
 		}
 	}
 }
@@ -380,6 +468,7 @@ struct SortWork {
 	unsigned *d_err;             /* TDV_EBIT_* flags */
 	uint64_t *hi_tmp;            /* n words: the tie fallback's high words */
 	uint32_t *p_tmp;             /* n: the tie fallback's first order */
+	uint32_t *order;             /* n: the order while the keys are read */
 	bool no_sync;                /* captured: no read back, no fallback (the
 	                                tie flag stays in d_err for the caller) */
 };
@@ -399,32 +488,54 @@ static SortWork context_work(tdv_context *c, const uint32_t *perm_out)
 	w.hi_tmp = reinterpret_cast<uint64_t *>(c->tmp_f64);
 	w.p_tmp = c->perm == perm_out ? reinterpret_cast<uint32_t *>(c->lohi)
 			: c->perm;
+	w.order = c->perm == perm_out ? c->perm : c->sv[1];
 	w.no_sync = c->graph_mode != 0;
 	return w;
 }
 
+/* Up to this many tiles the scatter sums the tiles' counts itself: two
+ * launches a pass instead of five.  The sum reads 1 KiB per tile and
+ * workgroup; with more tiles the scan's three launches are cheaper. */
+#define RS_SUM_TILES 64
+
 /* sorts n u64 keys (read with stride/offset, e.g. the high words of 128-bit
- * keys) carrying payload vin (NULL = original index) into w.sk/sv; returns
- * the buffer index holding the result */
+ * keys) carrying payload vin (NULL = original index): the sorted keys into
+ * w.sk[*res], the payload into vout */
 static int radix_sort_u64(tdv_context *c, const SortWork &w, size_t n,
 		const uint64_t *keys, int stride, int off, const uint32_t *vin,
-		int *res)
+		uint32_t *vout, int *res)
 {
 	const unsigned nb = (unsigned)((n + RS_TILE - 1) / RS_TILE);
 	const size_t hn = (size_t)nb * RS_BINS;
 	if (hn + 1 > w.hist_cap)
 		return tdv_fail(c, TDV_ERR_ARG, "radix sort histogram too small");
+	if (nb == 1) {
+		hipLaunchKernelGGL(k_rs_one_tile, dim3(1), dim3(RS1_THREADS), 0,
+				w.stream, keys, stride, off, vin, w.sk[0], vout, (int)n);
+		*res = 0;
+		return tdv_check(c, hipGetLastError(), "radix sort");
+	}
+	const bool by_tile = nb <= RS_SUM_TILES;
 	const uint64_t *kin = keys;
 	const uint32_t *vi = vin;
 	int s = stride, o = off, cur = 0;
 	for (int pass = 0; pass < 8; pass++) {
 		const int shift = 8 * pass;
-		hipLaunchKernelGGL(k_rs_hist, dim3(nb), dim3(RS_THREADS), 0, w.stream,
-				kin, s, o, n, shift, w.hist, nb);
-		TDV_TRY(scan_u32(c, w.stream, w.scan_part, w.hist, w.hist, hn));
-		hipLaunchKernelGGL(k_rs_scatter, dim3(nb), dim3(RS_THREADS), 0,
-				w.stream, kin, s, o, vi, w.sk[cur], w.sv[cur], n, shift,
-				w.hist, nb);
+		uint32_t *vo = pass == 7 ? vout : w.sv[cur];
+		if (by_tile) {
+			hipLaunchKernelGGL(k_rs_hist<true>, dim3(nb), dim3(RS_THREADS), 0,
+					w.stream, kin, s, o, n, shift, w.hist, nb);
+			hipLaunchKernelGGL(k_rs_scatter<true>, dim3(nb),
+					dim3(RS_THREADS), 0, w.stream, kin, s, o, vi, w.sk[cur],
+					vo, n, shift, w.hist, nb);
+		} else {
+			hipLaunchKernelGGL(k_rs_hist<false>, dim3(nb), dim3(RS_THREADS),
+					0, w.stream, kin, s, o, n, shift, w.hist, nb);
+			TDV_TRY(scan_u32(c, w.stream, w.scan_part, w.hist, w.hist, hn));
+			hipLaunchKernelGGL(k_rs_scatter<false>, dim3(nb),
+					dim3(RS_THREADS), 0, w.stream, kin, s, o, vi, w.sk[cur],
+					vo, n, shift, w.hist, nb);
+		}
 		kin = w.sk[cur];
 		vi = w.sv[cur];
 		s = 1;
@@ -445,10 +556,9 @@ int tdv_radix_pass8(tdv_context *c, size_t n, const uint64_t *keys,
 	const size_t hn = (size_t)nb * RS_BINS;
 	if (hn + 1 > c->hist_cap)
 		return tdv_fail(c, TDV_ERR_ARG, "radix pass histogram too small");
-	hipLaunchKernelGGL(k_rs_hist, dim3(nb), dim3(RS_THREADS), 0, c->stream,
-			keys, 1, 0, n, 0, c->hist, nb);
-	TDV_TRY(scan_u32(c, c->stream, c->scan_part, c->hist, c->hist, hn));
-	hipLaunchKernelGGL(k_rs_scatter, dim3(nb), dim3(RS_THREADS), 0,
+	hipLaunchKernelGGL(k_rs_hist<true>, dim3(nb), dim3(RS_THREADS), 0,
+			c->stream, keys, 1, 0, n, 0, c->hist, nb);
+	hipLaunchKernelGGL(k_rs_scatter<true>, dim3(nb), dim3(RS_THREADS), 0,
 			c->stream, keys, 1, 0, nullptr, kout, order, n, 0, c->hist, nb);
 	return tdv_check(c, hipGetLastError(), "radix pass");
 }
@@ -519,12 +629,13 @@ static int sort_keys_work(tdv_context *c, const SortWork &w, size_t n,
 	if (n == 0)
 		return 0;
 	int res;
-	TDV_TRY(radix_sort_u64(c, w, n, keys, 2, 1, nullptr, &res));
+	TDV_TRY(radix_sort_u64(c, w, n, keys, 2, 1, nullptr, w.order, &res));
 	hipLaunchKernelGGL(k_fix_ties, dim3(tdv_blocks(n, 256)), dim3(256), 0,
-			w.stream, n, w.sk[res], w.sv[res], keys, w.d_err);
+			w.stream, n, w.sk[res], w.order, keys, w.d_err);
 	if (w.no_sync) {
-		TDV_HIP(c, hipMemcpyAsync(perm_out, w.sv[res], n * sizeof(uint32_t),
-				hipMemcpyDeviceToDevice, w.stream));
+		if (w.order != perm_out)
+			TDV_HIP(c, hipMemcpyAsync(perm_out, w.order,
+					n * sizeof(uint32_t), hipMemcpyDeviceToDevice, w.stream));
 		return tdv_check(c, hipGetLastError(), "sort");
 	}
 	unsigned e = 0;
@@ -536,17 +647,17 @@ static int sort_keys_work(tdv_context *c, const SortWork &w, size_t n,
 		 * first (8 passes), then the high words in that order (8 passes) */
 		TDV_HIP(c, hipMemsetAsync(w.d_err, 0, sizeof(unsigned), w.stream));
 		int r1;
-		TDV_TRY(radix_sort_u64(c, w, n, keys, 2, 0, nullptr, &r1));
-		TDV_HIP(c, hipMemcpyAsync(w.p_tmp, w.sv[r1], n * sizeof(uint32_t),
-				hipMemcpyDeviceToDevice, w.stream));
+		TDV_TRY(radix_sort_u64(c, w, n, keys, 2, 0, nullptr, w.p_tmp, &r1));
 		hipLaunchKernelGGL(k_gather_hi, dim3(tdv_blocks(n, 256)), dim3(256), 0,
 				w.stream, n, w.p_tmp, keys, w.hi_tmp);
-		TDV_TRY(radix_sort_u64(c, w, n, w.hi_tmp, 1, 0, w.p_tmp, &res));
+		TDV_TRY(radix_sort_u64(c, w, n, w.hi_tmp, 1, 0, w.p_tmp, w.order,
+				&res));
 		hipLaunchKernelGGL(k_check_dups, dim3(tdv_blocks(n, 256)), dim3(256), 0,
-				w.stream, n, w.sv[res], keys, w.d_err);
+				w.stream, n, w.order, keys, w.d_err);
 	}
-	TDV_HIP(c, hipMemcpyAsync(perm_out, w.sv[res], n * sizeof(uint32_t),
-			hipMemcpyDeviceToDevice, w.stream));
+	if (w.order != perm_out)
+		TDV_HIP(c, hipMemcpyAsync(perm_out, w.order, n * sizeof(uint32_t),
+				hipMemcpyDeviceToDevice, w.stream));
 	return tdv_check(c, hipGetLastError(), "sort");
 }
 
@@ -627,6 +738,7 @@ extern "C" int tdv_sort_keys_noalloc(size_t n, const uint64_t *keys,
 	w.sv[1] = reinterpret_cast<uint32_t *>(base + NA_SV1);
 	w.hi_tmp = reinterpret_cast<uint64_t *>(base + NA_HI);
 	w.p_tmp = reinterpret_cast<uint32_t *>(base + NA_PT);
+	w.order = w.sv[1];
 	w.hist = reinterpret_cast<uint32_t *>(base + NA_HIST);
 	w.hist_cap = NA_HIST_CAP;
 	w.scan_part = reinterpret_cast<uint32_t *>(base + NA_PART);

@@ -287,3 +287,19 @@ def test_medians_by_selection_match_oracle(n, kind):
     np.testing.assert_array_equal(center, c)
     assert size == s
     np.testing.assert_array_equal(origin, o)
+
+
+@pytest.mark.parametrize("n", [63, 1024, 6143, 6144, 6145, 64 * 6144,
+                               64 * 6144 + 1])
+def test_sort_paths_match_stable_order(n):
+    """One workgroup's tile, tiles summed by the scatter, the device-wide
+    scan: keys with few distinct high digits, runs of equal high words
+    ordered by the low word."""
+    g = np.random.Generator(np.random.Philox(n))
+    keys = np.empty((n, 2), np.uint64)
+    keys[:, 0] = g.permutation(n).astype(np.uint64) * np.uint64(7)
+    keys[:, 1] = (g.integers(0, max(2, n // 3), n).astype(np.uint64)
+                  << np.uint64(g.integers(0, 40)))
+    e = Engine(periodic=False)
+    want = np.lexsort((keys[:, 0], keys[:, 1]))
+    np.testing.assert_array_equal(e.sort_keys(keys).astype(np.int64), want)
