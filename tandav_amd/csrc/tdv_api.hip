@@ -564,29 +564,20 @@ static int computational_domain(tdv_context *c)
 	return tdv_domain_nonperiodic(c);
 }
 
-__global__ void k_iota(int n, int *__restrict__ a)
+/* every particle active: the list and its count */
+__global__ void k_all_active(int n, int *__restrict__ a, int *__restrict__ na)
 {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i < n)
 		a[i] = i;
+	if (i == 0)
+		*na = n;
 }
 
 /* Sort_Particles_By_Peano_Key (peano.c:20-48) with the current domain:
  * keys, sort, reorder of every column.  The active list's indices belong to
  * the old order, so it is reset to every particle (a sync point, as at every
  * domain decomposition of the reference); tdv_set_active narrows it. */
-__global__ void k_set_int(int *p, int v)
-{
-	if (threadIdx.x == 0)
-		*p = v;
-}
-
-__global__ void k_clear_err_bits(unsigned *err, unsigned bits)
-{
-	if (threadIdx.x == 0)
-		*err &= ~bits;
-}
-
 static int keys_sort_reorder(tdv_context *c)
 {
 	const size_t n = c->n;
@@ -597,57 +588,24 @@ static int keys_sort_reorder(tdv_context *c)
 			c->dom_size, c->key_tmp, 0);
 	rec(c, EV_KEYS1);
 	TDV_TRY(tdv_sort_device(c, n, c->key_tmp, c->perm));
+	rec(c, EV_SORT1);
 	/* equal keys (particles within Domain.Size / 2^42 on every axis) stay in
 	 * their input order: the reference's quicksort leaves them in an order
-	 * of its own (sort.c:253-341), the build dumps them all the same */
-	hipLaunchKernelGGL(k_clear_err_bits, dim3(1), dim3(64), 0, c->stream,
-			c->d_err, TDV_EBIT_DUP);
-	rec(c, EV_SORT1);
-	/* reorder_collisionless_particles (peano.c:50-82) as gathers */
-	tdv_launch_gather_key(c, n, c->perm, c->key_tmp, c->key);
-	double **cols[] = { &c->pos[0], &c->pos[1], &c->pos[2], &c->vel[0],
-		&c->vel[1], &c->vel[2], &c->acc[0], &c->acc[1], &c->acc[2],
-		&c->gacc[0], &c->gacc[1], &c->gacc[2], &c->mass, &c->last_acc,
-		&c->cost };
-	for (double **col : cols) {
-		tdv_launch_gather_f64(c, n, c->perm, *col, c->tmp_f64);
-		if (c->graph_mode) {
-			/* a captured step keeps every column where it is, so each
-			 * replay finds its buffers: copy back instead of swapping */
-			TDV_HIP(c, hipMemcpyAsync(*col, c->tmp_f64, n * sizeof(double),
-					hipMemcpyDeviceToDevice, c->stream));
-			continue;
-		}
-		double *t = *col;
-		*col = c->tmp_f64;
-		c->tmp_f64 = t;
-	}
-	int *icols[] = { c->tree_parent, c->time_bin,
-		reinterpret_cast<int *>(c->id), reinterpret_cast<int *>(c->it_drift),
-		reinterpret_cast<int *>(c->it_kick) };
-	for (int *col : icols) {
-		tdv_launch_gather_i32(c, n, c->perm, col, c->lohi);
-		TDV_HIP(c, hipMemcpyAsync(col, c->lohi, n * sizeof(int),
-				hipMemcpyDeviceToDevice, c->stream));
-	}
-	tdv_launch_pack_pm(c);
-	if (c->graph_mode) {
-		/* every particle active after the sort, the count on the device */
-		hipLaunchKernelGGL(k_iota, dim3(tdv_blocks(n, 256)), dim3(256), 0,
-				c->stream, (int)n, c->active);
-		hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, c->stream,
-				c->d_nactive, (int)n);
-		TDV_HIP(c, hipGetLastError());
+	 * of its own (sort.c:253-341), the build dumps them all the same, and
+	 * the sort's duplicate flag is dropped */
+	tdv_launch_reorder(c, TDV_EBIT_DUP);
+	if (c->graph_mode || (size_t)c->nactive != n) {
+		/* the count on the device: a captured step's replays read it */
+		hipLaunchKernelGGL(k_all_active, dim3(tdv_blocks(n, 256)), dim3(256),
+				0, c->stream, (int)n, c->active, c->d_nactive);
 		c->nactive = (int)n;
+	}
+	if (c->graph_mode) {
+		TDV_HIP(c, hipGetLastError());
 		c->have_domain = 1;
 		c->have_tree = 0;
 		c->have_top = 0;
 		return 0;
-	}
-	if ((size_t)c->nactive != n) {
-		hipLaunchKernelGGL(k_iota, dim3(tdv_blocks(n, 256)), dim3(256), 0,
-				c->stream, (int)n, c->active);
-		TDV_TRY(set_nactive(c, (int)n));
 	}
 	tdv_graph_drop(c);               /* columns were swapped */
 	(void)hipEventRecord(c->ev[EV_REORDER1], c->stream);

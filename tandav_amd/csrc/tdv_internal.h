@@ -204,8 +204,7 @@ void tdv_launch_gather_f64(tdv_context *c, size_t n, const uint32_t *perm,
 		const double *in, double *out);
 void tdv_launch_gather_i32(tdv_context *c, size_t n, const uint32_t *perm,
 		const int *in, int *out);
-void tdv_launch_gather_key(tdv_context *c, size_t n, const uint32_t *perm,
-		const uint64_t *in, uint64_t *out);
+void tdv_launch_reorder(tdv_context *c, unsigned clear);
 void tdv_launch_reverse_keys(tdv_context *c, size_t n, const uint64_t *in,
 		uint64_t *out);
 void tdv_launch_pack_pm(tdv_context *c);

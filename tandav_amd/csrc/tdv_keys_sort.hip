@@ -790,13 +790,143 @@ void tdv_launch_gather_i32(tdv_context *c, size_t n, const uint32_t *perm,
 			c->stream, n, perm, in, out);
 }
 
-void tdv_launch_gather_key(tdv_context *c, size_t n, const uint32_t *perm,
-		const uint64_t *in, uint64_t *out)
+/* ---- the reorder (reorder_collisionless_particles, peano.c:50-82) --------
+ *
+ * Every column gathered by the sort's order.  A kernel takes several columns
+ * per pass over the order, each into a spare buffer of its size that then
+ * changes places with the column; the first also writes the walk's packed
+ * records.  One kernel per column, the 32-bit ones copied back, took 28
+ * launches and 40% more traffic. */
+struct Cols3 {
+	double *in[3], *out[3];
+};
+
+struct Cols5 {
+	int *in[5], *out[5];
+};
+
+__global__ void k_reorder_pos(size_t n, const uint32_t *__restrict__ perm,
+		const ulonglong2 *__restrict__ kin, ulonglong2 *__restrict__ kout,
+		Cols3 c, const double *__restrict__ m, double4 *__restrict__ pm,
+		unsigned *__restrict__ err, unsigned clear)
 {
-	hipLaunchKernelGGL(k_gather<ulonglong2>, dim3(tdv_blocks(n, 256)),
-			dim3(256), 0, c->stream, n, perm,
-			reinterpret_cast<const ulonglong2 *>(in),
-			reinterpret_cast<ulonglong2 *>(out));
+	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (i == 0)
+		*err &= ~clear;
+	if (i >= n)
+		return;
+	const uint32_t p = perm[i];
+	const ulonglong2 k = kin[p];
+	const double4 q = make_double4(c.in[0][p], c.in[1][p], c.in[2][p], m[p]);
+	kout[i] = k;
+	c.out[0][i] = q.x;
+	c.out[1][i] = q.y;
+	c.out[2][i] = q.z;
+	pm[i] = q;
+}
+
+/* perm NULL: copied in place order (a captured step's way back) */
+__global__ void k_reorder_f64(size_t n, const uint32_t *__restrict__ perm,
+		Cols3 c)
+{
+	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (i >= n)
+		return;
+	const size_t p = perm ? perm[i] : i;
+	const double a = c.in[0][p], b = c.in[1][p], d = c.in[2][p];
+	c.out[0][i] = a;
+	c.out[1][i] = b;
+	c.out[2][i] = d;
+}
+
+__global__ void k_reorder_i32(size_t n, const uint32_t *__restrict__ perm,
+		Cols5 c)
+{
+	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (i >= n)
+		return;
+	const size_t p = perm ? perm[i] : i;
+	int v[5];
+#pragma unroll
+	for (int q = 0; q < 5; q++)
+		v[q] = c.in[q][p];
+#pragma unroll
+	for (int q = 0; q < 5; q++)
+		c.out[q][i] = v[q];
+}
+
+/* The particle columns, the key (key_tmp -> key) and pm in the order perm;
+ * the error bits `clear` are dropped.  The spare buffers are the sort's and
+ * the build's scratch, free here and of the columns' size.  A captured step
+ * copies back instead of changing places, so each replay finds its columns
+ * where they were. */
+void tdv_launch_reorder(tdv_context *c, unsigned clear)
+{
+	const size_t n = c->n;
+	const dim3 grid(tdv_blocks(n, 256)), block(256);
+	double *spare[3] = { c->tmp_f64, reinterpret_cast<double *>(c->sk[0]),
+		reinterpret_cast<double *>(c->sk[1]) };
+	double **cols[5][3] = { { &c->pos[0], &c->pos[1], &c->pos[2] },
+		{ &c->vel[0], &c->vel[1], &c->vel[2] },
+		{ &c->acc[0], &c->acc[1], &c->acc[2] },
+		{ &c->gacc[0], &c->gacc[1], &c->gacc[2] },
+		{ &c->mass, &c->last_acc, &c->cost } };
+	for (int g = 0; g < 5; g++) {
+		Cols3 k;
+		for (int q = 0; q < 3; q++) {
+			k.in[q] = *cols[g][q];
+			k.out[q] = spare[q];
+		}
+		if (g == 0)
+			hipLaunchKernelGGL(k_reorder_pos, grid, block, 0, c->stream, n,
+					c->perm, reinterpret_cast<const ulonglong2 *>(c->key_tmp),
+					reinterpret_cast<ulonglong2 *>(c->key), k, c->mass, c->pm,
+					c->d_err, clear);
+		else
+			hipLaunchKernelGGL(k_reorder_f64, grid, block, 0, c->stream, n,
+					c->perm, k);
+		for (int q = 0; q < 3; q++)
+			if (c->graph_mode) {
+				std::swap(k.in[q], k.out[q]);
+			} else {
+				*cols[g][q] = k.out[q];
+				spare[q] = k.in[q];
+			}
+		if (c->graph_mode)
+			hipLaunchKernelGGL(k_reorder_f64, grid, block, 0, c->stream, n,
+					(const uint32_t *)nullptr, k);
+	}
+	c->tmp_f64 = spare[0];
+	c->sk[0] = reinterpret_cast<uint64_t *>(spare[1]);
+	c->sk[1] = reinterpret_cast<uint64_t *>(spare[2]);
+	const Cols5 g = { { c->tree_parent, c->time_bin,
+		reinterpret_cast<int *>(c->id), reinterpret_cast<int *>(c->it_drift),
+		reinterpret_cast<int *>(c->it_kick) },
+		{ c->cnt, c->lohi, reinterpret_cast<int *>(c->minpack),
+		reinterpret_cast<int *>(c->sv[0]),
+		reinterpret_cast<int *>(c->sv[1]) } };
+	hipLaunchKernelGGL(k_reorder_i32, grid, block, 0, c->stream, n, c->perm,
+			g);
+	if (c->graph_mode) {
+		Cols5 k;
+		for (int q = 0; q < 5; q++) {
+			k.in[q] = g.out[q];
+			k.out[q] = g.in[q];
+		}
+		hipLaunchKernelGGL(k_reorder_i32, grid, block, 0, c->stream, n,
+				(const uint32_t *)nullptr, k);
+		return;
+	}
+	c->tree_parent = g.out[0];
+	c->time_bin = g.out[1];
+	c->id = reinterpret_cast<uint32_t *>(g.out[2]);
+	c->it_drift = reinterpret_cast<uint32_t *>(g.out[3]);
+	c->it_kick = reinterpret_cast<uint32_t *>(g.out[4]);
+	c->cnt = g.in[0];
+	c->lohi = g.in[1];
+	c->minpack = reinterpret_cast<uint32_t *>(g.in[2]);
+	c->sv[0] = reinterpret_cast<uint32_t *>(g.in[3]);
+	c->sv[1] = reinterpret_cast<uint32_t *>(g.in[4]);
 }
 
 __global__ void k_pack_pm(size_t n, const double *__restrict__ x,
