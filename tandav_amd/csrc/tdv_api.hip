@@ -41,12 +41,34 @@ int tdv_check(tdv_context *c, hipError_t e, const char *what)
 			std::string(what) + ": " + hipGetErrorString(e));
 }
 
-int tdv_check_err_flags(tdv_context *c)
+__global__ void __launch_bounds__(256) k_report(HostReport *rep,
+		const unsigned *__restrict__ err, const int *__restrict__ ntop,
+		const int *__restrict__ nactive,
+		const unsigned long long *__restrict__ count,
+		const unsigned *__restrict__ lvl)
 {
-	unsigned e = 0;
-	TDV_HIP(c, hipMemcpyAsync(&e, c->d_err, sizeof(e), hipMemcpyDeviceToHost,
-			c->stream));
-	TDV_HIP(c, hipStreamSynchronize(c->stream));
+	const int i = threadIdx.x;
+	if (i < TDV_LVL_WORDS)
+		rep->lvl[i] = lvl[i];
+	if (i < 4)
+		rep->count[i] = count[i];
+	if (i == 0) {
+		rep->err = *err;
+		rep->ntop = *ntop;
+		rep->nactive = *nactive;
+	}
+}
+
+int tdv_report(tdv_context *c)
+{
+	hipLaunchKernelGGL(k_report, dim3(1), dim3(256), 0, c->stream, c->rep,
+			c->d_err, c->top.ntop, c->d_nactive, c->d_count, c->lvl);
+	TDV_HIP(c, hipGetLastError());
+	return tdv_check(c, hipStreamSynchronize(c->stream), "sync");
+}
+
+int tdv_flags_error(tdv_context *c, unsigned e)
+{
 	if (!e)
 		return 0;
 	TDV_HIP(c, hipMemsetAsync(c->d_err, 0, sizeof(unsigned), c->stream));
@@ -60,6 +82,12 @@ int tdv_check_err_flags(tdv_context *c)
 		return tdv_fail(c, TDV_ERR_TIES, "run of equal 64-bit key prefixes");
 	return tdv_fail(c, TDV_ERR_RANGE,
 			"a small top node's particle range leaves the particle arrays");
+}
+
+int tdv_check_err_flags(tdv_context *c)
+{
+	TDV_TRY(tdv_report(c));
+	return tdv_flags_error(c, c->rep->err);
 }
 
 template <typename T>
@@ -360,6 +388,9 @@ int tdv_create(const tdv_params *p, tdv_context **out)
 	if (!r)
 		r = dalloc(c, &c->lvl, TDV_LVL_WORDS);
 	if (!r)
+		r = tdv_check(c, hipHostMalloc((void **)&c->rep, sizeof(HostReport)),
+				"hipHostMalloc");
+	if (!r)
 		r = tdv_check(c, hipMemset(c->d_err, 0, sizeof(unsigned)), "memset");
 	if (!r)
 		r = alloc_top(c, 64);
@@ -405,6 +436,8 @@ void tdv_destroy(tdv_context *c)
 	dfree(c->top32);
 	tdv_graph_drop(c);
 	dfree(c->select);
+	if (c->rep)
+		(void)hipHostFree(c->rep);
 	dfree(c->d_err);
 	dfree(c->d_count);
 	dfree(c->d_nactive);
@@ -578,7 +611,7 @@ __global__ void k_all_active(int n, int *__restrict__ a, int *__restrict__ na)
  * keys, sort, reorder of every column.  The active list's indices belong to
  * the old order, so it is reset to every particle (a sync point, as at every
  * domain decomposition of the reference); tdv_set_active narrows it. */
-static int keys_sort_reorder(tdv_context *c)
+static int launch_sort_reorder(tdv_context *c, bool defer)
 {
 	const size_t n = c->n;
 	if (!n)
@@ -587,7 +620,7 @@ static int keys_sort_reorder(tdv_context *c)
 	tdv_launch_keys(c, n, c->pos[0], c->pos[1], c->pos[2], c->dom_origin,
 			c->dom_size, c->key_tmp, 0);
 	rec(c, EV_KEYS1);
-	TDV_TRY(tdv_sort_device(c, n, c->key_tmp, c->perm));
+	TDV_TRY(tdv_sort_device(c, n, c->key_tmp, c->perm, defer));
 	rec(c, EV_SORT1);
 	/* equal keys (particles within Domain.Size / 2^42 on every axis) stay in
 	 * their input order: the reference's quicksort leaves them in an order
@@ -600,21 +633,42 @@ static int keys_sort_reorder(tdv_context *c)
 				0, c->stream, (int)n, c->active, c->d_nactive);
 		c->nactive = (int)n;
 	}
-	if (c->graph_mode) {
-		TDV_HIP(c, hipGetLastError());
-		c->have_domain = 1;
-		c->have_tree = 0;
-		c->have_top = 0;
-		return 0;
+	if (!c->graph_mode) {
+		tdv_graph_drop(c);           /* columns were swapped */
+		(void)hipEventRecord(c->ev[EV_REORDER1], c->stream);
 	}
-	tdv_graph_drop(c);               /* columns were swapped */
-	(void)hipEventRecord(c->ev[EV_REORDER1], c->stream);
 	TDV_HIP(c, hipGetLastError());
-	TDV_TRY(tdv_check_err_flags(c));
 	c->have_domain = 1;
 	c->have_tree = 0;
 	c->have_top = 0;
 	return 0;
+}
+
+/* The sort and the reorder do not wait for the sort's tie flag: where a run
+ * of equal 64-bit prefixes was too long to be ordered by the low words, the
+ * columns are in an order that is right but for such runs, equal prefixes
+ * in input order.  This, once the flag is on the host, sorts them again
+ * with the 128-bit fallback and leaves the two orders' product in perm;
+ * `again` says so. */
+static int finish_sort_reorder(tdv_context *c, bool *again)
+{
+	*again = (c->rep->err & TDV_EBIT_TIES) != 0;
+	if (!*again)
+		return tdv_flags_error(c, c->rep->err);
+	TDV_HIP(c, hipMemsetAsync(c->d_err, 0, sizeof(unsigned), c->stream));
+	TDV_HIP(c, hipMemcpyAsync(c->off, c->perm, c->n * sizeof(uint32_t),
+			hipMemcpyDeviceToDevice, c->stream));
+	TDV_TRY(launch_sort_reorder(c, false));
+	tdv_launch_compose(c, c->n, c->off, c->perm);
+	return tdv_check_err_flags(c);
+}
+
+static int keys_sort_reorder(tdv_context *c)
+{
+	bool again;
+	TDV_TRY(launch_sort_reorder(c, true));
+	TDV_TRY(tdv_report(c));
+	return finish_sort_reorder(c, &again);
 }
 
 int tdv_set_domain(tdv_context *c, double size, const double origin[3])
@@ -702,11 +756,19 @@ int tdv_domain_decomposition(tdv_context *c)
 		return TDV_ERR_ARG;
 	TDV_TRY(computational_domain(c));
 	c->have_domain_set = 1;
-	TDV_TRY(keys_sort_reorder(c));
+	TDV_TRY(launch_sort_reorder(c, true));
 	TDV_TRY(tdv_build_top_nodes(c));
-	c->have_top = 1;
 	(void)hipEventRecord(c->ev[EV_TOP1], c->stream);
-	TDV_HIP(c, hipStreamSynchronize(c->stream));
+	TDV_TRY(tdv_report(c));
+	bool again;
+	TDV_TRY(finish_sort_reorder(c, &again));
+	if (again) {
+		TDV_TRY(tdv_build_top_nodes(c));
+		(void)hipEventRecord(c->ev[EV_TOP1], c->stream);
+		TDV_TRY(tdv_report(c));
+	}
+	c->ntop = c->rep->ntop;
+	c->have_top = 1;
 	float ms;
 	(void)hipEventElapsedTime(&ms, c->ev[EV_KEYS0], c->ev[EV_KEYS1]);
 	c->stage_ms[0] = ms;
@@ -769,9 +831,9 @@ int tdv_tree_build(tdv_context *c)
 	(void)hipEventRecord(c->ev[EV_BUILD0], c->stream);
 	TDV_TRY(tdv_build_tree(c));
 	(void)hipEventRecord(c->ev[EV_BUILD1], c->stream);
-	TDV_HIP(c, hipStreamSynchronize(c->stream));
+	TDV_TRY(tdv_report(c));
 	(void)hipEventElapsedTime(&c->stage_ms[4], c->ev[EV_BUILD0], c->ev[EV_BUILD1]);
-	return tdv_check_err_flags(c);
+	return tdv_flags_error(c, c->rep->err);
 }
 
 int tdv_tree_acceleration(tdv_context *c, int use_bh)
@@ -791,12 +853,11 @@ int tdv_tree_acceleration(tdv_context *c, int use_bh)
 			TDV_TRY(tdv_walk64_ewald(c, use_bh));
 	}
 	(void)hipEventRecord(c->ev[EV_EWALD1], c->stream);
-	TDV_HIP(c, hipStreamSynchronize(c->stream));
+	TDV_TRY(tdv_report(c));
 	(void)hipEventElapsedTime(&c->stage_ms[5], c->ev[EV_WALK0], c->ev[EV_WALK1]);
 	(void)hipEventElapsedTime(&c->stage_ms[6], c->ev[EV_WALK1], c->ev[EV_EWALD1]);
-	TDV_HIP(c, hipMemcpy(c->count, c->d_count, sizeof(c->count),
-			hipMemcpyDeviceToHost));
-	return tdv_check_err_flags(c);
+	memcpy(c->count, c->rep->count, sizeof(c->count));
+	return tdv_flags_error(c, c->rep->err);
 }
 
 int tdv_compute_acceleration(tdv_context *c, int prepare_step)
@@ -864,12 +925,11 @@ int tdv_launch_walk(tdv_context *c)
 	(void)hipEventRecord(c->ev[EV_WALK0], c->stream);
 	TDV_HIP(c, hipGraphLaunch(c->graph_exec, c->stream));
 	(void)hipEventRecord(c->ev[EV_WALK1], c->stream);
-	TDV_HIP(c, hipStreamSynchronize(c->stream));
+	TDV_TRY(tdv_report(c));
 	(void)hipEventElapsedTime(&c->stage_ms[5], c->ev[EV_WALK0], c->ev[EV_WALK1]);
 	c->stage_ms[6] = 0.f;
-	TDV_HIP(c, hipMemcpy(c->count, c->d_count, sizeof(c->count),
-			hipMemcpyDeviceToHost));
-	return tdv_check_err_flags(c);
+	memcpy(c->count, c->rep->count, sizeof(c->count));
+	return tdv_flags_error(c, c->rep->err);
 }
 
 /* The whole regular step of a periodic FP32 run as one HIP graph: the
@@ -905,7 +965,7 @@ int tdv_capture_step(tdv_context *c, double kick, double drift)
 	c->capturing = 1;
 	int r = computational_domain(c);
 	if (!r)
-		r = keys_sort_reorder(c);
+		r = launch_sort_reorder(c, true);
 	if (!r)
 		r = tdv_build_top_nodes(c);
 	if (!r) {
@@ -948,30 +1008,24 @@ int tdv_launch_step(tdv_context *c)
 	(void)hipEventRecord(c->ev[EV_KEYS0], c->stream);
 	TDV_HIP(c, hipGraphLaunch(c->step_exec, c->stream));
 	(void)hipEventRecord(c->ev[EV_KICK1], c->stream);
+	TDV_TRY(tdv_report(c));
 	/* the level counts are this tree's from now on */
-	int h[2];
-	TDV_HIP(c, hipMemcpyAsync(&h[0], c->top.ntop, sizeof(int),
-			hipMemcpyDeviceToHost, c->stream));
-	TDV_HIP(c, hipMemcpyAsync(c->lvl_host, c->lvl, sizeof(c->lvl_host),
-			hipMemcpyDeviceToHost, c->stream));
-	TDV_HIP(c, hipMemcpyAsync(c->count, c->d_count, sizeof(c->count),
-			hipMemcpyDeviceToHost, c->stream));
-	TDV_HIP(c, hipStreamSynchronize(c->stream));
-	h[1] = (int)c->lvl_host[TDV_LVL_NODES];
+	memcpy(c->lvl_host, c->rep->lvl, sizeof(c->lvl_host));
+	memcpy(c->count, c->rep->count, sizeof(c->count));
+	const int nn = (int)c->lvl_host[TDV_LVL_NODES];
+	const unsigned err = c->rep->err;
 	float ms = 0.f;
 	(void)hipEventElapsedTime(&ms, c->ev[EV_KEYS0], c->ev[EV_KICK1]);
 	for (int k = 0; k < 8; k++)
 		c->stage_ms[k] = 0.f;
 	c->stage_ms[5] = ms;                 /* the whole step */
-	c->ntop = h[0];
+	c->ntop = c->rep->ntop;
 	c->nactive = (int)c->n;
 	c->have_domain = 1;
 	c->have_top = 1;
-	c->have_tree = h[1] >= 0;
-	c->lvl_ok = h[1] >= 0;
-	c->nnodes = h[1] >= 0 ? (size_t)h[1] : 0;
-	unsigned err = 0;
-	TDV_HIP(c, hipMemcpy(&err, c->d_err, sizeof(err), hipMemcpyDeviceToHost));
+	c->have_tree = nn >= 0;
+	c->lvl_ok = nn >= 0;
+	c->nnodes = nn >= 0 ? (size_t)nn : 0;
 	if (err & TDV_EBIT_TIES) {
 		TDV_HIP(c, hipMemset(c->d_err, 0, sizeof(unsigned)));
 		c->have_tree = 0;
@@ -980,13 +1034,13 @@ int tdv_launch_step(tdv_context *c)
 				"fallback, which a captured step does not take: run the step "
 				"eagerly");
 	}
-	if (h[1] < 0) {
+	if (nn < 0) {
 		TDV_HIP(c, hipMemset(c->d_err, 0, sizeof(unsigned)));
 		return tdv_fail(c, TDV_ERR_RANGE, "tdv_launch_step: the tree needs "
 				"more nodes than the captured step holds: run the step "
 				"eagerly and capture again");
 	}
-	return tdv_check_err_flags(c);
+	return tdv_flags_error(c, err);
 }
 
 enum { FT_TABLE, FT_EXACT_SPLIT, FT_EXACT_PAIRS };
@@ -1103,7 +1157,7 @@ int tdv_sort_keys(tdv_context *c, size_t n, const uint64_t *keys,
 	}
 	TDV_HIP(c, hipMemcpyAsync(c->key_tmp, keys, 16 * n, hipMemcpyHostToDevice,
 			c->stream));
-	TDV_TRY(tdv_sort_device(c, n, c->key_tmp, c->perm));
+	TDV_TRY(tdv_sort_device(c, n, c->key_tmp, c->perm, false));
 	TDV_HIP(c, hipMemcpyAsync(perm_out, c->perm, 4 * n, hipMemcpyDeviceToHost,
 			c->stream));
 	TDV_HIP(c, hipStreamSynchronize(c->stream));
@@ -1525,10 +1579,8 @@ int tdv_make_active_list(tdv_context *c, int max_active_bin,
 	hipLaunchKernelGGL(k_active_scatter, dim3(tdv_blocks(n, 256)), dim3(256),
 			0, c->stream, n, flag, c->off, c->active, c->d_nactive);
 	TDV_HIP(c, hipGetLastError());
-	int nact = 0;
-	TDV_HIP(c, hipMemcpyAsync(&nact, c->d_nactive, sizeof(int),
-			hipMemcpyDeviceToHost, c->stream));
-	TDV_HIP(c, hipStreamSynchronize(c->stream));
+	TDV_TRY(tdv_report(c));
+	const int nact = c->rep->nactive;
 	c->nactive = nact;
 	if (nact <= 0)                   /* timestep.c:296-297 */
 		return tdv_fail(c, TDV_ERR_ARG, "tdv_make_active_list: no active "

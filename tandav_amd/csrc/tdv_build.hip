@@ -27,6 +27,7 @@
 #include "tdv_internal.h"
 #include "tdv_device.h"
 #include <algorithm>
+#include <cstring>
 
 #define NOCOLLAPSE 0xFFFFFFFFu
 
@@ -114,11 +115,6 @@ int tdv_build_top_nodes(tdv_context *c)
 			c->key, c->pos[0], c->pos[1], c->pos[2], c->dom_origin[0],
 			c->dom_origin[1], c->dom_origin[2], c->dom_size, c->top);
 	TDV_HIP(c, hipGetLastError());
-	if (!c->graph_mode) {            /* a captured step keeps it on the device */
-		TDV_HIP(c, hipMemcpyAsync(&c->ntop, c->top.ntop, sizeof(int),
-				hipMemcpyDeviceToHost, c->stream));
-		TDV_HIP(c, hipStreamSynchronize(c->stream));
-	}
 	return tdv_assign_top(c);
 }
 
@@ -271,8 +267,7 @@ __global__ void __launch_bounds__(256) k_tree_counts(size_t n,
  * nodes, this 4); more nodes than `cap` (a captured step's arrays) set the
  * node count to -1, which every later kernel of the step reads as "do
  * nothing", and raise TDV_EBIT_RANGE.  Also the levels' list offsets and
- * fill counters, and the node count and error flags for the host beside the
- * level counts. */
+ * fill counters, and the node count for the host beside the level counts. */
 __global__ void __launch_bounds__(64) k_tree_targets(TopNodes T, int vs,
 		const uint32_t *__restrict__ off, long long cap, unsigned *err,
 		unsigned *__restrict__ lvl)
@@ -315,7 +310,6 @@ __global__ void __launch_bounds__(64) k_tree_targets(TopNodes T, int vs,
 		const int nn = over ? -1 : (int)run;
 		*T.nnodes = nn;
 		lvl[TDV_LVL_NODES] = (unsigned)nn;
-		lvl[TDV_LVL_ERR] = atomicOr(err, 0u);
 	}
 }
 
@@ -986,11 +980,8 @@ int tdv_build_tree(tdv_context *c)
 	TDV_HIP(c, hipGetLastError());
 	size_t bound = c->node_cap;          /* nodes the kernels may touch */
 	if (!graph) {
-		TDV_HIP(c, hipMemcpyAsync(c->lvl_host, c->lvl, sizeof(c->lvl_host),
-				hipMemcpyDeviceToHost, c->stream));
-		TDV_HIP(c, hipStreamSynchronize(c->stream));
-		if (c->lvl_host[TDV_LVL_ERR])
-			TDV_TRY(tdv_check_err_flags(c));
+		TDV_TRY(tdv_check_err_flags(c));
+		memcpy(c->lvl_host, c->rep->lvl, sizeof(c->lvl_host));
 		const int nn = (int)c->lvl_host[TDV_LVL_NODES];
 		TDV_TRY(tdv_ensure_nodes(c, (size_t)nn));
 		c->nnodes = (size_t)nn;

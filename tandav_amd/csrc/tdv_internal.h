@@ -39,9 +39,8 @@
 /* the words of tdv_context::lvl: nodes per level in [0, 64), then */
 #define TDV_LVL_FILL 64      /* their lists' fill counters, */
 #define TDV_LVL_OFF 128      /* the lists' offsets, */
-#define TDV_LVL_NODES 192    /* the node count (-1: over capacity) and */
-#define TDV_LVL_ERR 193      /* the error flags after the node count */
-#define TDV_LVL_WORDS 194
+#define TDV_LVL_NODES 192    /* the node count (-1: over capacity) */
+#define TDV_LVL_WORDS 193
 #define TDV_LVL_FEW 512      /* levels of up to this many nodes share a
                                 launch of one workgroup */
 #define TDV_LVL_THREADS 1024
@@ -64,6 +63,16 @@ struct SelectState {         /* the selection of the three medians, device */
 	uint64_t k[3];           /* rank among the keys with that prefix */
 	unsigned done;           /* workgroups that have counted */
 	unsigned hist[3 * TDV_SELECT_BINS];
+};
+
+/* What the host reads of the device's counts and flags after a call's
+ * kernels, in page-locked host memory that k_report writes: one launch and
+ * one wait where each item was a copy and a wait of its own. */
+struct HostReport {
+	unsigned err;            /* TDV_EBIT_* */
+	int ntop, nactive, pad;
+	unsigned long long count[4];
+	unsigned lvl[TDV_LVL_WORDS];
 };
 
 struct TopNodes {            /* device arrays, top_cap entries each */
@@ -176,6 +185,7 @@ struct tdv_context {
 	int ewald16_ok;                  /* ewald16 matches ewald */
 
 	SelectState *select;             /* non-periodic domain */
+	HostReport *rep;                 /* host memory, see tdv_report */
 	unsigned *d_err;
 	unsigned long long *d_count;     /* [4] interactions: tree, Ewald;
 	                                    FP32 walk: of which multipole nodes,
@@ -199,7 +209,9 @@ void tdv_launch_keys(tdv_context *c, size_t n, const double *x,
 		const double *y, const double *z, const double o[3], double size,
 		uint64_t *out, int reversed);
 int tdv_sort_device(tdv_context *c, size_t n, const uint64_t *keys,
-		uint32_t *perm_out);
+		uint32_t *perm_out, bool defer);
+void tdv_launch_compose(tdv_context *c, size_t n, const uint32_t *first,
+		uint32_t *perm);
 void tdv_launch_gather_f64(tdv_context *c, size_t n, const uint32_t *perm,
 		const double *in, double *out);
 void tdv_launch_gather_i32(tdv_context *c, size_t n, const uint32_t *perm,
@@ -285,6 +297,11 @@ int tdv_domain_refine(tdv_context *c, int ntarget, double part_alloc_factor,
 /* ---- helpers (tdv_api.hip) ---- */
 int tdv_fail(tdv_context *c, int code, const std::string &msg);
 int tdv_check(tdv_context *c, hipError_t e, const char *what);
+/* wait for the stream with c->rep brought up to date */
+int tdv_report(tdv_context *c);
+/* the error that the flags stand for (0 for none), which are cleared */
+int tdv_flags_error(tdv_context *c, unsigned flags);
+/* both */
 int tdv_check_err_flags(tdv_context *c);
 int tdv_ensure_nodes(tdv_context *c, size_t nodes);
 

@@ -469,8 +469,8 @@ struct SortWork {
 	uint64_t *hi_tmp;            /* n words: the tie fallback's high words */
 	uint32_t *p_tmp;             /* n: the tie fallback's first order */
 	uint32_t *order;             /* n: the order while the keys are read */
-	bool no_sync;                /* captured: no read back, no fallback (the
-	                                tie flag stays in d_err for the caller) */
+	bool no_sync;                /* no read back, no fallback (the tie flag
+	                                stays in d_err for the caller) */
 };
 
 static SortWork context_work(tdv_context *c, const uint32_t *perm_out)
@@ -489,7 +489,7 @@ static SortWork context_work(tdv_context *c, const uint32_t *perm_out)
 	w.p_tmp = c->perm == perm_out ? reinterpret_cast<uint32_t *>(c->lohi)
 			: c->perm;
 	w.order = c->perm == perm_out ? c->perm : c->sv[1];
-	w.no_sync = c->graph_mode != 0;
+	w.no_sync = false;
 	return w;
 }
 
@@ -661,10 +661,29 @@ static int sort_keys_work(tdv_context *c, const SortWork &w, size_t n,
 	return tdv_check(c, hipGetLastError(), "sort");
 }
 
+/* defer: the tie flag stays in d_err for the caller, no fallback */
 int tdv_sort_device(tdv_context *c, size_t n, const uint64_t *keys,
-		uint32_t *perm_out)
+		uint32_t *perm_out, bool defer)
 {
-	return sort_keys_work(c, context_work(c, perm_out), n, keys, perm_out);
+	SortWork w = context_work(c, perm_out);
+	w.no_sync = defer;
+	return sort_keys_work(c, w, n, keys, perm_out);
+}
+
+/* perm = first, then perm */
+__global__ void k_compose(size_t n, const uint32_t *__restrict__ first,
+		uint32_t *__restrict__ perm)
+{
+	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < n)
+		perm[i] = first[perm[i]];
+}
+
+void tdv_launch_compose(tdv_context *c, size_t n, const uint32_t *first,
+		uint32_t *perm)
+{
+	hipLaunchKernelGGL(k_compose, dim3(tdv_blocks(n, 256)), dim3(256), 0,
+			c->stream, n, first, perm);
 }
 
 /* ------------------------------------------------------------------------ */

@@ -303,3 +303,34 @@ def test_sort_paths_match_stable_order(n):
     e = Engine(periodic=False)
     want = np.lexsort((keys[:, 0], keys[:, 1]))
     np.testing.assert_array_equal(e.sort_keys(keys).astype(np.int64), want)
+
+
+@pytest.mark.parametrize("n,clump", [(20000, 6000), (9000, 4096), (5000, 5000)])
+def test_particle_sort_with_long_runs_of_equal_prefixes(n, clump):
+    """More than 4096 particles that share a 64-bit key prefix: the sort
+    takes its 128-bit form after the columns were reordered once, and the
+    order, the top nodes and the permutation of host columns are those of
+    one stable sort."""
+    g = np.random.Generator(np.random.Philox(n))
+    pos = g.uniform(0.0, 1.0, (n, 3))
+    where = g.permutation(n)[:clump]
+    pos[where] = 0.3 + 1e-9 * g.uniform(0.0, 1.0, (clump, 3))
+    e = Engine(periodic=True, softening=1e-3)
+    e.set_particles(pos, np.full(n, 1.0 / n))
+    e.setup_domain()
+    k = oracle.peano_keys(pos[:, 0], pos[:, 1], pos[:, 2], [0, 0, 0], 1.0,
+                          False)
+    want = np.lexsort((k[:, 0], k[:, 1]))
+    got = e.get("id", "pos")
+    np.testing.assert_array_equal(got["id"].astype(np.int64), want)
+    np.testing.assert_array_equal(got["pos"], pos[want])
+    col = np.arange(n, dtype=np.float64)
+    e.permute_columns(col)
+    np.testing.assert_array_equal(col.astype(np.int64), want)
+    e.domain_decomposition()
+    np.testing.assert_array_equal(e.get("id")["id"].astype(np.int64), want)
+    top = e.top_nodes()
+    assert int(top["Npart"].sum()) == n
+    cells = k[want][:, 1] >> np.uint64(58)
+    np.testing.assert_array_equal(top["First_Part"],
+                                  np.unique(cells, return_index=True)[1][::-1])
