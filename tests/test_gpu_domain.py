@@ -63,3 +63,27 @@ def test_domain_targets_rejects_too_few_bunches():
     e.set_particles(pos, m)
     with pytest.raises(TDVError):
         e.domain_decomposition_targets(2)
+
+
+@pytest.mark.parametrize("n,ntarget", [(1000, 2), (65537, 3), (400000, 16)])
+def test_domain_targets_of_long_cost_sums_match_oracle(n, ntarget):
+    """Bunches of up to a few hundred thousand particles: their float costs
+    in particle order, from the walk's own Cost, bit for bit the serial
+    sums (the refinement depends on every one of them)."""
+    pos, _, m = ics.clustered_box(n, nhalo=3, seed=9)
+    e = Engine(periodic=True, softening=1e-4, alpha_rel=0.005, compat=False,
+               precision="fp32", fp32_criterion=3, ewald_accuracy=1.0)
+    e.set_particles(pos, m)
+    e.setup_domain()
+    e.domain_decomposition()
+    e.compute_acceleration(True)
+    cost = e.get("cost")["cost"]
+    short = e.keys(reversed_=False)[:, 1].copy()
+    rec, it = oracle.domain_targets(short, cost, ntarget)
+    tasks, passes = e.domain_decomposition_targets(ntarget)
+    top = e.top_nodes()
+    assert passes == it
+    assert len(top) == len(rec)
+    for f in ("Key", "Level", "First_Part", "Npart"):
+        np.testing.assert_array_equal(top[f], rec[f], err_msg=f)
+    np.testing.assert_array_equal(tasks, -rec["Target"] - 1)
