@@ -212,11 +212,10 @@ __global__ void k_kick_bins(int nact, const int *__restrict__ active,
 	kick_dt[i] = dt;
 }
 
-/* lower bound of v in the sorted active list */
-__device__ __forceinline__ int active_lower(const int *__restrict__ a, int n,
-		int v)
+/* lower bound of v in the sorted active list's entries [lo, hi) */
+__device__ __forceinline__ int active_lower(const int *__restrict__ a, int lo,
+		int hi, int v)
 {
-	int lo = 0, hi = n;
 	while (lo < hi) {
 		const int mid = (lo + hi) >> 1;
 		if (a[mid] < v)
@@ -227,182 +226,326 @@ __device__ __forceinline__ int active_lower(const int *__restrict__ a, int n,
 	return lo;
 }
 
+/* The run of the sorted active list (n entries) that lies in the particles
+ * [first, first + count).  Its start is entry `first` itself where all
+ * particles up to it are active; its end is at most count entries on. */
+__device__ __forceinline__ int2 active_run(const int *__restrict__ a, int n,
+		int first, int count)
+{
+	const bool all = first < n && a[first] == first
+			&& (first == 0 || a[first - 1] < first);
+	const int lo = all ? first : active_lower(a, 0, n, first);
+	if (lo >= n || a[lo] >= first + count)
+		return make_int2(lo, lo);
+	return make_int2(lo, active_lower(a, lo + 1, min(n, lo + count),
+			first + count));
+}
+
 /* Gravity_Tree_Update_Kicks (tree_update.c:12-57) for every active
  * particle: each tree node on the particle's path below its subtree root
  * (the nodes whose particle range holds it) takes Dp += m dt a / M, marked
  * UPDATED; the node's particles in particle order, so the sums are the
  * reference's one-thread sums.
  *
- * One lane per node finds the node's run [lo, hi) of the sorted active list
- * and sums runs of up to KICK_LANE_RUN particles itself.  A longer run is a
- * chain of that many dependent additions, so what one lane can do about it
- * is to keep everything else (loads, products, the division) out of the
- * chain, which it cannot: such nodes go to a list, one wavefront each
- * (k_tree_kicks_long).  Nodes of more than 64 active particles are disjoint
- * within a level, so TDV_NT levels hold fewer than 42 / 65 n of them and the
- * list fits n entries.  With one lane for every node and top node a kick of
- * all particles of the clustered 2^20 box took 67 ms here and 88 ms for the
- * top nodes; now 0.06 ms here and 5.4 ms for the list and the top nodes. */
-#define KICK_LANE_RUN 64
+ * A team of 16 lanes per node finds the node's run [lo, hi) of the sorted
+ * active list and takes runs of up to KICK_TEAM_RUN particles, each lane
+ * forming one particle's quotients m dt a / M, which all of the team then
+ * add in particle order, from lane to lane by DPP.  Longer runs, chains of
+ * that many dependent additions, go to a list (k_tree_kicks_long).  Nodes of
+ * more than 64 active particles are disjoint within a level, so TDV_NT
+ * levels hold fewer than 42 / 65 n of them and the list fits n entries.
+ * With one lane for every node and top node a kick of all particles of the
+ * clustered 2^20 box took 67 ms here and 88 ms for the top nodes, now 0.09
+ * ms here and 1.3 ms for the list and the top nodes; of 65,000 particles, a
+ * few active, 17 and 17 us with a lane for the short runs and the chains
+ * added one by one, 7 and 16 us now. */
+#define KICK_TEAM_RUN 64
 
 struct KickList {                /* build scratch, n entries each */
 	int *node, *lo, *hi;
+	int2 *top;                   /* every top node's run */
 	unsigned *count;             /* [0] listed nodes, [1] their queue */
 };
 
-__global__ void k_tree_kicks(size_t nn, int4 *__restrict__ nc,
+/* the value of lane S of the 16 (row_newbcast) */
+template <int S>
+__device__ __forceinline__ double row_lane(double v)
+{
+	const uint64_t u = (uint64_t)__double_as_longlong(v);
+	const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u,
+			0x150 + S, 0xf, 0xf, false);
+	const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0,
+			(int)(u >> 32), 0x150 + S, 0xf, 0xf, false);
+	return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+
+/* d += the quotients of lanes S .. 15, in lane order */
+template <int S>
+__device__ __forceinline__ void row_add(double4 &d, double x, double y,
+		double z)
+{
+	if constexpr (S < 16) {
+		d.x = d.x + row_lane<S>(x);
+		d.y = d.y + row_lane<S>(y);
+		d.z = d.z + row_lane<S>(z);
+		row_add<S + 1>(d, x, y, z);
+	}
+}
+
+__global__ void __launch_bounds__(256) k_tree_kicks(size_t nn,
+		int4 *__restrict__ nc,
 		const double4 *__restrict__ na, double4 *__restrict__ dpn,
 		int nact, const int *__restrict__ active,
 		const double *__restrict__ m, const double *__restrict__ dtk,
 		const double *__restrict__ ax, const double *__restrict__ ay,
-		const double *__restrict__ az, KickList list)
+		const double *__restrict__ az, const TopNodes T, KickList list)
 {
-	const size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (j >= nn)
+	const size_t j = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
+	const int sub = threadIdx.x & 15;
+	if (j >= nn) {                       /* the top nodes' runs */
+		const size_t t = j - nn;
+		if (t < (size_t)*T.ntop && sub == 0)
+			list.top[t] = active_run(active, nact, T.first[t], T.npart[t]);
 		return;
+	}
 	const int4 c = nc[j];
 	if (c.w < 0 || ((c.z >> TDV_BIT_TOP) & 1))
 		return;                          /* terminator, subtree root */
-	const int lo = active_lower(active, nact, c.w);
-	const int hi = active_lower(active, nact, c.w + c.y);
+	const int2 run = active_run(active, nact, c.w, c.y);
+	const int lo = run.x, hi = run.y;
 	if (lo >= hi)
 		return;
-	nc[j].z = c.z | (1 << TDV_BIT_UPDATED);   /* only this node's own */
-	if (hi - lo > KICK_LANE_RUN) {
-		const unsigned slot = atomicAdd(&list.count[0], 1u);
-		list.node[slot] = (int)j;
-		list.lo[slot] = lo;
-		list.hi[slot] = hi;
+	if (sub == 0)
+		nc[j].z = c.z | (1 << TDV_BIT_UPDATED);   /* only this node's own */
+	if (hi - lo > KICK_TEAM_RUN) {
+		if (sub == 0) {
+			const unsigned slot = atomicAdd(&list.count[0], 1u);
+			list.node[slot] = (int)j;
+			list.lo[slot] = lo;
+			list.hi[slot] = hi;
+		}
 		return;
 	}
 	const double M = na[j].w;
 	double4 d = dpn[j];
-	/* four particles' loads and quotients at a time, then their additions
-	 * in order */
-	int g = lo;
-	for (; g + 4 <= hi; g += 4) {
-		double qx[4], qy[4], qz[4];
-#pragma unroll
-		for (int u = 0; u < 4; u++) {
-			const int i = active[g + u];
-			const double mdt = m[i] * dtk[i];
-			qx[u] = mdt * ax[i] / M;
-			qy[u] = mdt * ay[i] / M;
-			qz[u] = mdt * az[i] / M;
-		}
-#pragma unroll
-		for (int u = 0; u < 4; u++) {
-			d.x = d.x + qx[u];
-			d.y = d.y + qy[u];
-			d.z = d.z + qz[u];
-		}
-	}
-	for (; g < hi; g++) {
-		const int i = active[g];
+	for (int g = lo; g < hi; g += 16) {
+		/* past the run: its last particle's loads, zeros to add */
+		const bool on = g + sub < hi;
+		const int i = active[on ? g + sub : hi - 1];
 		const double mdt = m[i] * dtk[i];
-		d.x = d.x + mdt * ax[i] / M;
-		d.y = d.y + mdt * ay[i] / M;
-		d.z = d.z + mdt * az[i] / M;
+		const double qx = mdt * ax[i] / M, qy = mdt * ay[i] / M,
+				qz = mdt * az[i] / M;
+		row_add<0>(d, on ? qx : 0.0, on ? qy : 0.0, on ? qz : 0.0);
 	}
-	dpn[j] = d;
+	if (sub == 0)
+		dpn[j] = d;
 }
 
-/* The sum of one run [lo, hi) of the active list by one wavefront: the
- * lanes load 64 particles and form their quotients m dt a / M side by side,
- * the next 64 particles' loads in flight meanwhile; lane c of the first
- * three then adds component c in particle order from LDS, `step` making one
- * addition.  What is left of the chain is one dependent addition (and, for
- * the float top nodes, its two conversions) per particle. */
-template <typename Step>
-__device__ __forceinline__ double kick_run(int lo, int hi, double M,
-		const int *__restrict__ active, const double *__restrict__ m,
-		const double *__restrict__ dtk, const double *__restrict__ ax,
-		const double *__restrict__ ay, const double *__restrict__ az,
-		double start, double (*sh)[64], Step step)
+/* the value a DPP control moves into this lane, 0 where nothing arrives */
+template <int ctrl, int rows>
+__device__ __forceinline__ double dpp_add_f64(double v)
 {
+	const uint64_t u = (uint64_t)__double_as_longlong(v);
+	const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u, ctrl,
+			rows, 0xf, false);
+	const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0,
+			(int)(u >> 32), ctrl, rows, 0xf, false);
+	return v + __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+
+/* inclusive prefix sum over the wavefront (row_shr 1, 2, 4, 8, row_bcast 15
+ * and 31) */
+__device__ __forceinline__ double wave_prefix_add(double v)
+{
+	v = dpp_add_f64<0x111, 0xf>(v);
+	v = dpp_add_f64<0x112, 0xf>(v);
+	v = dpp_add_f64<0x114, 0xf>(v);
+	v = dpp_add_f64<0x118, 0xf>(v);
+	v = dpp_add_f64<0x142, 0xa>(v);
+	v = dpp_add_f64<0x143, 0xc>(v);
+	return v;
+}
+
+__device__ __forceinline__ double lane_f64(double v, int l)
+{
+	const uint64_t u = (uint64_t)__double_as_longlong(v);
+	const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)u, l);
+	const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(u >> 32),
+			l);
+	return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+
+/* one addition of a sum in double, or of a float's (its value in a double) */
+template <bool FLOAT>
+__device__ __forceinline__ double chain_step(double s, double q)
+{
+	return FLOAT ? (double)(float)(s + q) : s + q;
+}
+
+/* s after s = s + q (FLOAT: (float)(s + q)) for q[0 .. nb) in order, by one
+ * wavefront, with the serial chain's bits.  Lane l holds q[4 l .. 4 l + 4)
+ * in mine (0 past nb), sh all of them; s is the same in every lane.
+ *
+ * While |s| stays in one binade [2^e, 2^(e+1)), s = A u with u = 2^(e-P), P
+ * = 52 (23 for a float) and A a whole number, and an addition adds to A the
+ * whole number nearest to t = q / u, whatever A is, unless t lies halfway
+ * between two.  (A float's sum is rounded to a double first: t to multiples
+ * of 2^-29, whose unit is the same for every A of the binade.)  The lanes
+ * add up their four and a prefix sum, exact in whole numbers, gives every
+ * lane its A.  The lanes up to the first that meets a tie or may leave the
+ * binade (judged by the sum of its |k|) stand; that lane's four are added
+ * one by one and the rest go on in the new binade.  After CHAIN_ROUNDS such
+ * stops (s near zero) the rest of the 256 are added one by one. */
+#define CHAIN_PER_LANE 4
+#define CHAIN_LEN (64 * CHAIN_PER_LANE)
+#define CHAIN_ROUNDS 8
+
+template <bool FLOAT>
+__device__ __forceinline__ double chain_sum(double s,
+		const double (&mine)[CHAIN_PER_LANE], const double *sh, int nb)
+{
+	constexpr int P = FLOAT ? 23 : 52;
+	constexpr double lo = FLOAT ? 0x1p23 : 0x1p52, half = 0.5 * lo;
+	constexpr int emax = FLOAT ? 120 : 900;  /* clear of the type's ends */
 	const int lane = threadIdx.x;
-	const double *row = sh[lane < 3 ? lane : 0];
-	double s = start, nm = 0, nx = 0, ny = 0, nz = 0;
-	if (lo + lane < hi) {
-		const int i = active[lo + lane];
-		nm = m[i] * dtk[i];
-		nx = ax[i];
-		ny = ay[i];
-		nz = az[i];
-	}
-	for (int b0 = lo; b0 < hi; b0 += 64) {
-		const double qx = nm * nx / M, qy = nm * ny / M, qz = nm * nz / M;
-		if (b0 + 64 + lane < hi) {
-			const int i = active[b0 + 64 + lane];
-			nm = m[i] * dtk[i];
-			nx = ax[i];
-			ny = ay[i];
-			nz = az[i];
-		}
-		__syncthreads();                 /* the last block's row is read */
-		sh[0][lane] = qx;
-		sh[1][lane] = qy;
-		sh[2][lane] = qz;
-		__syncthreads();
-		const int nb = hi - b0 < 64 ? hi - b0 : 64;
-		int q = 0;
-		for (; q + 16 <= nb; q += 16) {
-			double t[16];
+	int base = 0;
+	for (int round = 0; base < nb; round++) {
+		const int e = (int)((uint64_t)__double_as_longlong(s) >> 52 & 0x7ff)
+				- 1023;
+		const bool chain = e >= -emax && e <= emax;
+		if (chain && round < CHAIN_ROUNDS) {
+			const double scale = __longlong_as_double(
+					(long long)(1023 + P - e) << 52);
+			const double A = fabs(s) * scale;
+			double sum = 0, range = 0;
+			bool ok = true;
 #pragma unroll
-			for (int u = 0; u < 16; u++)
-				t[u] = row[q + u];
-#pragma unroll
-			for (int u = 0; u < 16; u++)
-				s = step(s, t[u]);
+			for (int u = 0; u < CHAIN_PER_LANE; u++) {
+				double t = (s < 0 ? -mine[u] : mine[u]) * scale;
+				ok = ok && fabs(t) < half;
+				if (FLOAT)
+					t = (t + 0x1.8p23) - 0x1.8p23;
+				const double k = rint(t);
+				ok = ok && fabs(t - k) != 0.5;
+				sum += k;
+				range += fabs(k);
+			}
+			if (lane * CHAIN_PER_LANE < base) {  /* summed already */
+				sum = range = 0;
+				ok = true;
+			}
+			const double to = A + wave_prefix_add(sum);
+			const double from = to - sum;
+			const uint64_t stop = ~__ballot(ok && from - range > lo
+					&& from + range < 2 * lo);
+			const int first = stop ? __ffsll((long long)stop) - 1 : 64;
+			if (first * CHAIN_PER_LANE > base) {
+				const double m = lane_f64(to, first - 1) * __longlong_as_double(
+						(long long)(1023 - P + e) << 52);
+				s = s < 0 ? -m : m;
+				base = first * CHAIN_PER_LANE;
+			}
 		}
-		for (; q < nb; q++)
-			s = step(s, row[q]);
+		/* the lane's four, or everything left */
+		const int end = round < CHAIN_ROUNDS ? min(base + CHAIN_PER_LANE, nb)
+				: nb;
+		for (; base + 8 <= end; base += 8) {
+			double t[8];
+#pragma unroll
+			for (int u = 0; u < 8; u++)
+				t[u] = sh[base + u];
+#pragma unroll
+			for (int u = 0; u < 8; u++)
+				s = chain_step<FLOAT>(s, t[u]);
+		}
+		for (; base < end; base++)
+			s = chain_step<FLOAT>(s, sh[base]);
 	}
 	return s;
 }
 
-/* The listed nodes, a wavefront each, and before them the top nodes
- * (tree_update.c:43-55), whose runs are the longest: their Dp is a float in
- * D[].TNode, rounded after every addition, and the node is marked kicked.
- * Workgroup b < ntop takes top node b, then every workgroup takes listed
- * nodes from one counter. */
+/* one component of the sum of a run [lo, hi) of the active list's quotients
+ * m dt a / M, starting from s: 256 quotients at a time, formed side by
+ * side, the next 256 particles' loads in flight while they are summed */
+template <bool FLOAT>
+__device__ __forceinline__ double kick_run(int lo, int hi, double M,
+		const int *__restrict__ active, const double *__restrict__ m,
+		const double *__restrict__ dtk, const double *__restrict__ a,
+		double s, double *sh)
+{
+	constexpr int B = CHAIN_PER_LANE;
+	const int at = lo + (int)threadIdx.x * B;
+	double nm[B], na[B];
+#pragma unroll
+	for (int u = 0; u < B; u++) {
+		const int i = active[at + u < hi ? at + u : hi - 1];
+		nm[u] = m[i] * dtk[i];
+		na[u] = a[i];
+	}
+	for (int b0 = 0; lo + b0 < hi; b0 += CHAIN_LEN) {
+		double q[B];
+#pragma unroll
+		for (int u = 0; u < B; u++)
+			q[u] = at + b0 + u < hi ? nm[u] * na[u] / M : 0.0;
+#pragma unroll
+		for (int u = 0; u < B; u++) {
+			const int g = at + b0 + CHAIN_LEN + u;
+			const int i = active[g < hi ? g : hi - 1];
+			nm[u] = m[i] * dtk[i];
+			na[u] = a[i];
+		}
+		__syncthreads();                 /* the last block's are read */
+#pragma unroll
+		for (int u = 0; u < B; u++)
+			sh[threadIdx.x * B + u] = q[u];
+		__syncthreads();
+		const int left = hi - lo - b0;
+		s = chain_sum<FLOAT>(s, q, sh, left < CHAIN_LEN ? left : CHAIN_LEN);
+	}
+	return s;
+}
+
+/* A wavefront for each component of the top nodes (tree_update.c:43-55),
+ * whose runs are the longest and whose Dp is a float in D[].TNode, rounded
+ * after every addition (the node is marked kicked), and of the listed
+ * nodes.  Workgroup b < 3 ntop takes component b of the top nodes' Dp, then
+ * every workgroup takes components of listed nodes from one counter. */
 __global__ void __launch_bounds__(64) k_tree_kicks_long(const TopNodes T,
-		const double4 *__restrict__ na, double4 *__restrict__ dpn, int nact,
+		const double4 *__restrict__ na, double4 *__restrict__ dpn,
 		const int *__restrict__ active, const double *__restrict__ m,
 		const double *__restrict__ dtk, const double *__restrict__ ax,
 		const double *__restrict__ ay, const double *__restrict__ az,
 		KickList list)
 {
-	__shared__ double sh[3][64];
+	__shared__ double sh[CHAIN_LEN];
 	const int lane = threadIdx.x;
 	const int ntop = *T.ntop;
-	for (int t = blockIdx.x; t < ntop; t += gridDim.x) {
-		const int lo = active_lower(active, nact, T.first[t]);
-		const int hi = active_lower(active, nact, T.first[t] + T.npart[t]);
+	for (int w = blockIdx.x; w < 3 * ntop; w += gridDim.x) {
+		const int t = w / 3, d = w - 3 * t;
+		const int lo = list.top[t].x, hi = list.top[t].y;
 		if (lo >= hi)
 			continue;
-		const double s = kick_run(lo, hi, (double)T.mass[t], active, m, dtk,
-				ax, ay, az, lane < 3 ? (double)T.dp[3 * t + lane] : 0.0, sh,
-				[](double a, double q) { return (double)(float)(a + q); });
-		if (lane < 3)
-			T.dp[3 * t + lane] = (float)s;
-		if (lane == 0)
+		const double s = kick_run<true>(lo, hi, (double)T.mass[t], active, m,
+				dtk, d == 0 ? ax : d == 1 ? ay : az, (double)T.dp[w], sh);
+		if (lane == 0) {
+			T.dp[w] = (float)s;
 			T.kicked[t] = 1;
+		}
 	}
-	const int nl = (int)list.count[0];
+	const int items = 3 * (int)list.count[0];
 	for (;;) {
 		/* wave-uniform ticket, as in the walk's queue */
 		const unsigned tk = atomicAdd(&list.count[1], lane == 0 ? 1u : 0u);
 		const int item = __builtin_amdgcn_readfirstlane((int)tk);
-		if (item >= nl)
+		if (item >= items)
 			break;
-		const int j = list.node[item];
-		double *dp = reinterpret_cast<double *>(dpn + j);
-		const double s = kick_run(list.lo[item], list.hi[item], na[j].w,
-				active, m, dtk, ax, ay, az, lane < 3 ? dp[lane] : 0.0, sh,
-				[](double a, double q) { return a + q; });
-		if (lane < 3)
-			dp[lane] = s;
+		const int k = item / 3, d = item - 3 * k;
+		const int j = list.node[k];
+		double *dp = reinterpret_cast<double *>(dpn + j) + d;
+		const double s = kick_run<false>(list.lo[k], list.hi[k], na[j].w,
+				active, m, dtk, d == 0 ? ax : d == 1 ? ay : az, *dp, sh);
+		if (lane == 0)
+			*dp = s;
 	}
 }
 
@@ -659,19 +802,19 @@ int tdv_kick_halfstep(tdv_context *c, int update_tree)
 				c->long_count);
 	if (update_tree && c->nactive) {
 		const KickList list = { reinterpret_cast<int *>(c->minpack), c->cnt,
-			c->lohi, c->long_count };
-		if (c->nnodes)
-			hipLaunchKernelGGL(k_tree_kicks, dim3(tdv_blocks(c->nnodes, 256)),
-					dim3(256), 0, c->stream, c->nnodes, c->node_c, c->node_a,
-					c->node_dp, c->nactive, c->active, c->mass, c->kick_dt,
-					c->acc[0], c->acc[1], c->acc[2], list);
-		/* the top nodes first, then at most a wave per 65 active */
+			c->lohi, reinterpret_cast<int2 *>(c->sk[0]), c->long_count };
+		hipLaunchKernelGGL(k_tree_kicks, dim3(tdv_blocks(16 * (c->nnodes
+				+ (size_t)c->ntop), 256)), dim3(256), 0, c->stream, c->nnodes,
+				c->node_c, c->node_a, c->node_dp, c->nactive, c->active,
+				c->mass, c->kick_dt, c->acc[0], c->acc[1], c->acc[2], c->top,
+				list);
+		/* the top nodes first, then at most a node per 65 active and level */
 		const unsigned grid = (unsigned)std::min((size_t)TDV_LONG_GRID,
-				(size_t)c->ntop + (size_t)c->nactive / (KICK_LANE_RUN + 1));
+				3 * ((size_t)c->ntop
+				+ (size_t)c->nactive / (KICK_TEAM_RUN + 1)));
 		hipLaunchKernelGGL(k_tree_kicks_long, dim3(grid), dim3(64), 0,
-				c->stream, c->top, c->node_a, c->node_dp, c->nactive,
-				c->active, c->mass, c->kick_dt, c->acc[0], c->acc[1],
-				c->acc[2], list);
+				c->stream, c->top, c->node_a, c->node_dp, c->active, c->mass,
+				c->kick_dt, c->acc[0], c->acc[1], c->acc[2], list);
 	}
 	(void)hipEventRecord(c->ev[EV_KICK1], c->stream);
 	TDV_HIP(c, hipGetLastError());
