@@ -90,6 +90,12 @@ int tdv_check_err_flags(tdv_context *c)
 	return tdv_flags_error(c, c->rep->err);
 }
 
+int tdv_clear_counts(tdv_context *c)
+{
+	return tdv_check(c, hipMemsetAsync(c->d_count, 0,
+			4 * sizeof(unsigned long long), c->stream), "counters");
+}
+
 template <typename T>
 static int dalloc(tdv_context *c, T **p, size_t count)
 {
@@ -840,13 +846,12 @@ int tdv_tree_acceleration(tdv_context *c, int use_bh)
 {
 	if (!c || !c->have_tree)
 		return tdv_fail(c, TDV_ERR_ARG, "walk before a tree build");
-	TDV_HIP(c, hipMemsetAsync(c->d_count, 0, 4 * sizeof(unsigned long long),
-			c->stream));
 	(void)hipEventRecord(c->ev[EV_WALK0], c->stream);
 	if (c->par.precision == TDV_WALK_FP32) {
 		TDV_TRY(tdv_walk32(c, use_bh));     /* Newton + Ewald in one pass */
 		(void)hipEventRecord(c->ev[EV_WALK1], c->stream);
 	} else {
+		TDV_TRY(tdv_clear_counts(c));
 		TDV_TRY(tdv_walk64(c, use_bh));
 		(void)hipEventRecord(c->ev[EV_WALK1], c->stream);
 		if (c->par.periodic)

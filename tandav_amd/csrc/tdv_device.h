@@ -146,6 +146,16 @@ __host__ __device__ inline void peano_key_words(double x, double y, double z,
 	}
 }
 
+/* lane l's v (l wave-uniform) */
+__device__ __forceinline__ double lane_f64(double v, int l)
+{
+	const uint64_t u = (uint64_t)__double_as_longlong(v);
+	const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)u, l);
+	const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(u >> 32),
+			l);
+	return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+
 /* Ewald_Correction, Gravity/periodic.c:35-113 (table already / Box^2):
  * the table cell of a separation, its trilinear weights and the signs */
 struct EwaldCell {

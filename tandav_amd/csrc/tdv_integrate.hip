@@ -31,6 +31,7 @@
  * timestep.c:380-388), no longer than the largest active bin allows.
  */
 #include "tdv_internal.h"
+#include "tdv_device.h"
 
 #include <algorithm>
 #include <cmath>
@@ -364,15 +365,6 @@ __device__ __forceinline__ double wave_prefix_add(double v)
 	v = dpp_add_f64<0x142, 0xa>(v);
 	v = dpp_add_f64<0x143, 0xc>(v);
 	return v;
-}
-
-__device__ __forceinline__ double lane_f64(double v, int l)
-{
-	const uint64_t u = (uint64_t)__double_as_longlong(v);
-	const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)u, l);
-	const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(u >> 32),
-			l);
-	return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
 }
 
 /* one addition of a sum in double, or of a float's (its value in a double) */

@@ -244,6 +244,7 @@ std::vector<LevelRun> tdv_level_runs(const tdv_context *c, size_t bound);
 int tdv_walk64(tdv_context *c, int use_bh);
 int tdv_walk64_ewald(tdv_context *c, int use_bh);
 int tdv_walk32(tdv_context *c, int use_bh);
+int tdv_clear_counts(tdv_context *c);    /* the interaction counters */
 void tdv_launch_safe_last_accel_dev(tdv_context *c);
 void tdv_launch_kick_drift(tdv_context *c, double kick, double drift);
 void tdv_graph_drop(tdv_context *c);

@@ -273,16 +273,23 @@ __device__ __forceinline__ void moments_add_particles(
 		const double4 *__restrict__ pm, int first, int count, double cx,
 		double cy, double cz, double *m6)
 {
-	for (int p = first; p < first + count; p++) {
-		const double4 q = pm[p];
+	/* by one wavefront: 64 particles side by side, added in order */
+	for (int p = 0; p < count; p += 64) {
+		const double4 q = pm[first + min(p + (int)threadIdx.x, count - 1)];
 		const double dx = q.x - cx, dy = q.y - cy, dz = q.z - cz;
-		const double mx = q.w * dx, my = q.w * dy;
-		m6[0] = fma(mx, dx, m6[0]);
-		m6[1] = fma(my, dy, m6[1]);
-		m6[2] = fma(q.w * dz, dz, m6[2]);
-		m6[3] = fma(mx, dy, m6[3]);
-		m6[4] = fma(mx, dz, m6[4]);
-		m6[5] = fma(my, dz, m6[5]);
+		const double mx = q.w * dx, my = q.w * dy, mz = q.w * dz;
+		const int nb = min(count - p, 64);
+		for (int u = 0; u < nb; u++) {
+			const double lx = lane_f64(dx, u), ly = lane_f64(dy, u),
+					lz = lane_f64(dz, u), lmx = lane_f64(mx, u),
+					lmy = lane_f64(my, u), lmz = lane_f64(mz, u);
+			m6[0] = fma(lmx, lx, m6[0]);
+			m6[1] = fma(lmy, ly, m6[1]);
+			m6[2] = fma(lmz, lz, m6[2]);
+			m6[3] = fma(lmx, ly, m6[3]);
+			m6[4] = fma(lmx, lz, m6[4]);
+			m6[5] = fma(lmy, lz, m6[5]);
+		}
 	}
 }
 
@@ -424,11 +431,11 @@ __global__ void __launch_bounds__(256) k_level_fill(int bound,
 /* top nodes: from the subtree's root, shifted to the float centre of mass
  * (S about a point P = S_cm + M (c - P)(c - P)^T), or from the particles of
  * a top node without subtree */
-__global__ void k_moments_top(const TopNodes T, int vs,
+__global__ void __launch_bounds__(64) k_moments_top(const TopNodes T, int vs,
 		const double4 *__restrict__ na, const double4 *__restrict__ pm,
 		const double *__restrict__ s6, double scale, float4 *__restrict__ q)
 {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
+	const int t = blockIdx.x;        /* a wavefront per top node */
 	if (t >= *T.ntop || *T.nnodes < 0)
 		return;
 	const double cx = T.com[3 * t], cy = T.com[3 * t + 1],
@@ -449,7 +456,8 @@ __global__ void k_moments_top(const TopNodes T, int vs,
 	} else {
 		moments_add_particles(pm, T.first[t], T.npart[t], cx, cy, cz, m6);
 	}
-	moments_store(m6, scale, q + 2 * t);
+	if (threadIdx.x == 0)
+		moments_store(m6, scale, q + 2 * t);
 }
 
 /* ---- the walk ---------------------------------------------------------- */
@@ -1225,9 +1233,16 @@ __global__ void __launch_bounds__(64) k_walk32_want(
 		const int *__restrict__ active, const int4 *__restrict__ p32,
 		const double *__restrict__ last_acc, TopNodes T,
 		const int4 *__restrict__ top32, Walk32Params w,
-		unsigned long long *__restrict__ wmask)
+		unsigned long long *__restrict__ wmask, unsigned *__restrict__ queue,
+		unsigned long long *__restrict__ counter)
 {
 	const int group = blockIdx.x;
+	if (group == 0) {                    /* the walk's queue and counters */
+		if (threadIdx.x == 0)
+			queue[0] = 0;
+		if (threadIdx.x < 4)
+			counter[threadIdx.x] = 0;
+	}
 	const int nact = *nact_dev;
 	const int ngroups = (nact + 63) / 64;
 	if (group >= ngroups || walk32_parts(ngroups, split) == 1
@@ -1240,15 +1255,26 @@ __global__ void __launch_bounds__(64) k_walk32_want(
 	const int ip = gid < nact ? active[gid] : active[nact - 1];
 	const int4 me = p32[ip];
 	const float crit = (float)(last_acc[ip] * (double)w.alpha_rel);
+	const int live = min(64, nact - group * 64);
+	/* a lane per top node and the group's particles in turn, from lane to
+	 * lane: one load per top node, where a loop over the top nodes waited
+	 * for each one's (17 us for a few groups, this 6) */
 	for (int q = 0; q < TDV_WANT_WORDS && q * 64 < ntop; q++) {
-		unsigned long long bits = 0;
-		for (int b = 0; b < 64 && q * 64 + b < ntop; b++) {
-			const int j = q * 64 + b;
-			const float ts = ldexpf(w.dom_f, -T.level[j]);
+		const int j = q * 64 + (int)threadIdx.x;
+		const bool on = j < ntop;
+		const int4 tc = top32[on ? j : 0];
+		const float ts = ldexpf(w.dom_f, -T.level[on ? j : 0]);
+		bool want = false;
+		for (int i = 0; i < live; i++) {
+			const int4 p = make_int4(__builtin_amdgcn_readlane(me.x, i),
+					__builtin_amdgcn_readlane(me.y, i),
+					__builtin_amdgcn_readlane(me.z, i), 0);
+			const float c = __int_as_float(__builtin_amdgcn_readlane(
+					__float_as_int(crit), i));
 			float rx, ry, rz;
-			if (__any(top_want(top32[j], ts, me, crit, w, rx, ry, rz)))
-				bits |= 1ull << b;
+			want = top_want(tc, ts, p, c, w, rx, ry, rz) || want;
 		}
+		const unsigned long long bits = __ballot(on && want);
 		if (threadIdx.x == 0)
 			wmask[(size_t)group * TDV_WANT_WORDS + q] = bits;
 	}
@@ -1465,7 +1491,7 @@ __global__ void k_safe_last_accel_dev(const int *__restrict__ nact_dev,
 int tdv_walk32(tdv_context *c, int use_bh)
 {
 	if (!c->nactive && !c->capturing)
-		return 0;
+		return tdv_clear_counts(c);
 	const size_t n = c->n, nn = c->nnodes;
 	/* fixed-point frame: 2^32 per periodic box, 2^31 per domain otherwise */
 	const double S = c->par.periodic ? 4294967296.0 / c->par.boxsize
@@ -1558,8 +1584,7 @@ int tdv_walk32(tdv_context *c, int use_bh)
 						qscale, c->q32);
 		}
 		if (tgrid)
-			hipLaunchKernelGGL(k_moments_top, dim3(tdv_blocks((size_t)tgrid,
-					64)), dim3(64), 0, c->stream, c->top, c->par.vector_size,
+			hipLaunchKernelGGL(k_moments_top, dim3((unsigned)tgrid), dim3(64), 0, c->stream, c->top, c->par.vector_size,
 					c->node_a, c->pm, c->q_s6, qscale, c->tq32);
 	}
 	if (tgrid)
@@ -1663,7 +1688,8 @@ int tdv_walk32(tdv_context *c, int use_bh)
 		hipLaunchKernelGGL(k_walk32_want, dim3(c->capturing
 				? (unsigned)TDV_SPLIT_ITEMS / 2 : (unsigned)ngroups_h),
 				dim3(64), 0, c->stream, c->d_nactive, split, c->active,
-				c->p32, c->last_acc, c->top, c->top32, w, c->wmask);
+				c->p32, c->last_acc, c->top, c->top32, w, c->wmask,
+				c->d_queue, c->d_count);
 		TDV_TRY(tdv_check(c, hipGetLastError(), "k_walk32_want"));
 	}
 	if (!c->par.fp32_queue && (c->capturing || parts)) {
@@ -1673,8 +1699,6 @@ int tdv_walk32(tdv_context *c, int use_bh)
 				: (size_t)ngroups_h * nparts_h;
 		auto kern = c->par.fp32_waves == 6 ? k_walk32_items_w6
 				: c->par.fp32_waves == 8 ? k_walk32_items_w8 : k_walk32_items;
-		hipLaunchKernelGGL(k_walk32_queue_reset, dim3(1), dim3(64), 0,
-				c->stream, c->d_queue, c->d_count);
 		hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64), 0,
 				c->stream, c->d_nactive, split, c->partial, c->wmask, 0,
 				c->active,
@@ -1691,8 +1715,9 @@ int tdv_walk32(tdv_context *c, int use_bh)
 	}
 	if (c->par.fp32_queue || c->capturing || parts) {
 		/* grid: enough waves to fill every SIMD at the 8-wave budget */
-		hipLaunchKernelGGL(k_walk32_queue_reset, dim3(1), dim3(64), 0,
-				c->stream, c->d_queue, c->d_count);
+		if (!c->capturing && !parts)
+			hipLaunchKernelGGL(k_walk32_queue_reset, dim3(1), dim3(64), 0,
+					c->stream, c->d_queue, c->d_count);
 		hipLaunchKernelGGL(k_walk32_queue, dim3(TDV_QUEUE_GRID), dim3(64), 0,
 				c->stream, c->d_nactive, c->d_queue, split, c->partial,
 				c->wmask, 0,
@@ -1710,6 +1735,7 @@ int tdv_walk32(tdv_context *c, int use_bh)
 					c->gacc[1], c->gacc[2], c->cost);
 		return tdv_check(c, hipGetLastError(), "k_walk32_parts_sum");
 	}
+	TDV_TRY(tdv_clear_counts(c));
 	auto kern = c->par.fp32_waves == 6 ? k_walk32_w6
 			: c->par.fp32_waves == 8 ? k_walk32_w8 : k_walk32;
 	hipLaunchKernelGGL(kern, dim3(tdv_blocks((size_t)c->nactive, 64)),
