@@ -74,7 +74,7 @@ typedef struct {
 	                          the partial sums are carried into FP64
 	                          (0 = 16)                                        */
 	int fp32_waves;        /* FP32 walk: register budget for 6 or 8 waves per
-	                          SIMD (0 = the compiler's own allocation)        */
+	                          SIMD (0 = the kernel's own choice)              */
 	int fp32_queue;        /* FP32 walk: 1 = persistent work-queue kernel
 	                          (fixed grid, groups taken from a counter); 0 =
 	                          one wave per group, or per work item for

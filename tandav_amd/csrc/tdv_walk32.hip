@@ -466,9 +466,10 @@ struct Acc32 {
 	float x, y, z;
 	double X, Y, Z;
 	int since;
-	unsigned long long cost, ewald;  /* interactions, Ewald corrections */
-	unsigned nodes, ewq;             /* of which multipole nodes, and
-	                                    corrections with quadrupoles */
+	/* interactions and Ewald corrections of one particle (each node and
+	 * particle at most once), of which multipole nodes and corrections
+	 * with quadrupoles */
+	unsigned cost, ewald, nodes, ewq;
 };
 
 __device__ __forceinline__ void carry(Acc32 &a)
@@ -541,31 +542,37 @@ __device__ __forceinline__ void quad32(Acc32 &a, const float4 qa, float qyz,
 }
 
 /* The Ewald table node nearest to a separation d (fixed units) on the
- * positive octant, the offset from it in grid units (|offset| <= 1/2 per
- * axis) and the reflection signs (the correction is odd in each axis,
- * sign(0) = +1; Gravity/periodic.c:35-113). */
+ * positive octant, as its record's byte offset, and the offset from it in
+ * grid units (|offset| <= 1/2 per axis).  The correction is odd in each axis
+ * (sign(0) = +1: d is a converted integer, whose zero is positive;
+ * Gravity/periodic.c:35-113): d's sign bits turn it.  |d| is at most half
+ * the box (2^31), so the node is at most TDV_NE on each axis; its number,
+ * below 2^24, is formed in FP32 like the offsets: a third fewer instructions
+ * than with integer indices and 64-bit addresses. */
 struct EwaldNode {
-	int b;                           /* node (i, j, k) */
+	unsigned at;                     /* byte offset of the record */
 	float du, dv, dq;
-	float sx, sy, sz;
 };
 
 __device__ __forceinline__ EwaldNode ewald_node(float dx, float dy, float dz,
 		const Walk32Params &w)
 {
 	EwaldNode c;
-	c.sx = dx < 0.f ? -1.f : 1.f;
-	c.sy = dy < 0.f ? -1.f : 1.f;
-	c.sz = dz < 0.f ? -1.f : 1.f;
 	const float u = fabsf(dx) * w.u_scale, v = fabsf(dy) * w.u_scale,
 			q = fabsf(dz) * w.u_scale;
-	const int i = min((int)(u + 0.5f), TDV_NE), j = min((int)(v + 0.5f), TDV_NE),
-			k = min((int)(q + 0.5f), TDV_NE);
-	c.du = u - (float)i;
-	c.dv = v - (float)j;
-	c.dq = q - (float)k;
-	c.b = (i * TDV_NE1 + j) * TDV_NE1 + k;
+	const float i = floorf(u + 0.5f), j = floorf(v + 0.5f),
+			k = floorf(q + 0.5f);
+	c.du = u - i;
+	c.dv = v - j;
+	c.dq = q - k;
+	c.at = (unsigned)fmaf(fmaf(i, (float)TDV_NE1, j), (float)TDV_NE1, k) << 6;
 	return c;
+}
+
+/* v with its sign turned where s is negative */
+__device__ __forceinline__ float turn(float v, unsigned s)
+{
+	return __uint_as_float(__float_as_uint(v) ^ (s & 0x80000000u));
 }
 
 __device__ __forceinline__ float h2lo(float v)
@@ -578,6 +585,9 @@ __device__ __forceinline__ float h2hi(float v)
 	return (float)__builtin_bit_cast(half2_t, v).y;
 }
 
+typedef float vfloat4 __attribute__((ext_vector_type(4)));
+typedef float vfloat2 __attribute__((ext_vector_type(2)));
+
 /* The correction on the positive octant from the nearest node to second
  * order, E + J d + (1/2) S d d (d the offset in grid units; S fully
  * symmetric, the gradient's second derivatives), and the node's S / 6. */
@@ -589,8 +599,12 @@ struct EwaldLocal {
 __device__ __forceinline__ EwaldLocal ewald_local(const float4 *__restrict__ t,
 		const EwaldNode &c, const Walk32Params &w)
 {
-	const float4 *r = t + 4 * c.b;
-	const float4 r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3];
+	/* vector loads: as structs their fields were fetched in five pieces */
+	const char *r = reinterpret_cast<const char *>(t) + c.at;
+	const vfloat4 r0 = *reinterpret_cast<const vfloat4 *>(r);
+	const vfloat4 r1 = *reinterpret_cast<const vfloat4 *>(r + 16);
+	const vfloat4 r2 = *reinterpret_cast<const vfloat4 *>(r + 32);
+	const vfloat2 r3 = *reinterpret_cast<const vfloat2 *>(r + 48);
 	EwaldLocal e;
 	e.Sxxx = h2lo(r2.y);
 	e.Syyy = h2hi(r2.y);
@@ -629,9 +643,9 @@ __device__ __forceinline__ void ewald16(Acc32 &a, const float4 *__restrict__ t,
 {
 	const EwaldNode c = ewald_node(dx, dy, dz, w);
 	const EwaldLocal e = ewald_local(t, c, w);
-	a.x = fmaf(m * c.sx, e.ex, a.x);
-	a.y = fmaf(m * c.sy, e.ey, a.y);
-	a.z = fmaf(m * c.sz, e.ez, a.z);
+	a.x = fmaf(turn(m, __float_as_uint(dx)), e.ex, a.x);
+	a.y = fmaf(turn(m, __float_as_uint(dy)), e.ey, a.y);
+	a.z = fmaf(turn(m, __float_as_uint(dz)), e.ez, a.z);
 	a.ewald++;
 }
 
@@ -654,8 +668,10 @@ __device__ __forceinline__ void ewald16q(Acc32 &a, const float4 *__restrict__ t,
 			cyy = qa.y * w.inv_s2 * w.inv_s2_box4;
 	const float czz = -(cxx + cyy);
 	const float t2 = 2.f * w.inv_s2 * w.inv_s2_box4;
-	const float cxy = qa.z * t2 * (c.sx * c.sy), cxz = qa.w * t2 * (c.sx * c.sz),
-			cyz = qyz * t2 * (c.sy * c.sz);
+	const unsigned ux = __float_as_uint(dx), uy = __float_as_uint(dy),
+			uz = __float_as_uint(dz);
+	const float cxy = turn(qa.z * t2, ux ^ uy), cxz = turn(qa.w * t2, ux ^ uz),
+			cyz = turn(qyz * t2, uy ^ uz);
 	float vx = m * e.ex, vy = m * e.ey, vz = m * e.ez;
 	vx = fmaf(cxx, e.Sxxx, fmaf(cyy, e.Sxyy, fmaf(czz, e.Sxzz, vx)));
 	vx = fmaf(cxy, e.Sxxy, fmaf(cxz, e.Sxxz, fmaf(cyz, e.Sxyz, vx)));
@@ -663,9 +679,9 @@ __device__ __forceinline__ void ewald16q(Acc32 &a, const float4 *__restrict__ t,
 	vy = fmaf(cxy, e.Sxyy, fmaf(cxz, e.Sxyz, fmaf(cyz, e.Syyz, vy)));
 	vz = fmaf(cxx, e.Sxxz, fmaf(cyy, e.Syyz, fmaf(czz, e.Szzz, vz)));
 	vz = fmaf(cxy, e.Sxyz, fmaf(cxz, e.Sxzz, fmaf(cyz, e.Syzz, vz)));
-	a.x = fmaf(c.sx, vx, a.x);
-	a.y = fmaf(c.sy, vy, a.y);
-	a.z = fmaf(c.sz, vz, a.z);
+	a.x += turn(vx, ux);
+	a.y += turn(vy, uy);
+	a.z += turn(vz, uz);
 	a.ewald++;
 	a.ewq++;
 }
@@ -738,15 +754,14 @@ __device__ __forceinline__ bool node_opens_ri(float m, float s, float r2,
 		const Walk32Params &w)
 {
 	const float es = w.eps_abs + s;
-	if (r2 < es * es)
-		return true;
+	const bool near = r2 < es * es;
 	if (w.use_bh)
-		return s * s > r2 * w.theta_bh;
+		return near | (s * s > r2 * w.theta_bh);
 	const float ms2 = m * s * s;
 	const float lhs = w.crit3 ? ms2 * (s * ri) : ms2;
 	const float s6 = 0.6f * s;
-	return lhs > (r2 * crit) * r2 || (fabsf(sx) < s6 && fabsf(sy) < s6
-			&& fabsf(sz) < s6);
+	return near | (lhs > (r2 * crit) * r2) | ((fabsf(sx) < s6)
+			& (fabsf(sy) < s6) & (fabsf(sz) < s6));
 }
 
 /* An accepted node (r >= |eps| + s, outside the softening length): its
@@ -817,6 +832,11 @@ __device__ __forceinline__ void ewald_pp(Acc32 &a, const float4 *__restrict__ ta
 	}
 }
 
+/* The switches of Walk32Params that a walk's kernel has as constants: any
+ * (none of them), or the usual walk (relative criterion, quadrupoles) of a
+ * periodic or an isolated run */
+enum { WALK32_ANY, WALK32_PERIODIC, WALK32_ISOLATED };
+
 /* One wave walks `group` (64 active particles, one per lane) over part
  * `part` of `nparts`: every subtree the group walks is cut into nparts
  * contiguous node ranges and this wave takes range `part` of each, so
@@ -829,7 +849,7 @@ __device__ __forceinline__ void ewald_pp(Acc32 &a, const float4 *__restrict__ ta
  * subtree are dealt out over the parts.  With nparts == 1 the results go
  * to the particles; otherwise to partial[part * nslot + slot], summed in
  * part order by k_walk32_parts_sum. */
-template <bool SPLIT>
+template <bool SPLIT, int MODE>
 __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 		double4 *__restrict__ partial, int nslot, int nact,
 		const int *__restrict__ active, const int4 *__restrict__ p32,
@@ -843,6 +863,11 @@ __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 		const float4 *__restrict__ p32o,
 		const unsigned long long *__restrict__ wmask)
 {
+	if (MODE != WALK32_ANY) {            /* the switches as constants */
+		w.use_bh = 0;
+		w.quad = 1;
+		w.periodic = MODE == WALK32_PERIODIC;
+	}
 	if (*T.nnodes < 0)                   /* the build overflowed: no walk */
 		return;
 	const int ntop = *T.ntop;
@@ -853,7 +878,7 @@ __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 	/* relative criterion: open if M s^2 > r^4 |a| alpha / G; with masses
 	 * scaled by G S^2 and lengths in fixed units this is m s^2 > r^4 crit */
 	const float crit = (float)(last_acc[ip] * (double)w.alpha_rel);
-	Acc32 a = { 0.f, 0.f, 0.f, 0.0, 0.0, 0.0, 0, 0ull, 0ull, 0u, 0u };
+	Acc32 a = { 0.f, 0.f, 0.f, 0.0, 0.0, 0.0, 0, 0u, 0u, 0u, 0u };
 	const int every = w.carry_every;
 	const float inv_parts = 1.f / (float)nparts;
 
@@ -1135,7 +1160,7 @@ __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 	if (nparts > 1) {
 		if (live)
 			partial[(size_t)part * nslot + gid] = make_double4(a.X, a.Y, a.Z,
-					(double)(a.cost + a.ewald));
+					(double)((unsigned long long)a.cost + a.ewald));
 	} else if (live) {
 		ax[ip] = ax[ip] + a.X;
 		ay[ip] = ay[ip] + a.Y;
@@ -1143,7 +1168,7 @@ __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 		gx[ip] = a.X;
 		gy[ip] = a.Y;
 		gz[ip] = a.Z;
-		cost[ip] = (double)(a.cost + a.ewald);
+		cost[ip] = (double)((unsigned long long)a.cost + a.ewald);
 	}
 	unsigned long long v = live ? a.cost : 0ull, e = live ? a.ewald : 0ull,
 			nd = live ? a.nodes : 0ull, eq = live ? a.ewq : 0ull;
@@ -1177,32 +1202,39 @@ __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 		double *__restrict__ cost, unsigned long long *counter, \
 		const int4 *__restrict__ top32, const float4 *__restrict__ tq32, \
 		const float4 *__restrict__ p32o, const uint32_t *__restrict__ gorder
-#define TDV_WALK32_CALL_PARTW(g, part, nparts, partial, nslot, wmask) \
-		walk32_body<true>(g, part, nparts, partial, nslot, nact, active, p32, \
-		last_acc, T, rec, tab, w, ax, ay, az, gx, gy, gz, cost, \
+#define TDV_WALK32_CALL_PARTW(MODE, g, part, nparts, partial, nslot, wmask) \
+		walk32_body<true, MODE>(g, part, nparts, partial, nslot, nact, \
+		active, p32, last_acc, T, rec, tab, w, ax, ay, az, gx, gy, gz, cost, \
 		counter, top32, tq32, p32o, wmask)
-#define TDV_WALK32_CALL(g) \
-		walk32_body<false>(g, 0, 1, nullptr, 0, nact, active, p32, \
+#define TDV_WALK32_CALL(MODE, g) \
+		walk32_body<false, MODE>(g, 0, 1, nullptr, 0, nact, active, p32, \
 		last_acc, T, rec, tab, w, ax, ay, az, gx, gy, gz, cost, \
 		counter, top32, tq32, p32o, nullptr)
 /* the i-th group to walk: by descending expected cost when ordered */
 #define TDV_GROUP(i) (gorder ? (int)gorder[i] : (i))
 
-__global__ void __launch_bounds__(64) k_walk32(TDV_WALK32_ARGS)
+/* The walk is bound by instruction issue (0.9 of it at 256^3, half scalar:
+ * the record loads and the loop's branches), so the usual walks have their
+ * switches as constants (256^3 step 527 -> 481 ms, same bits) and the grid
+ * walk runs in 64 registers, eight waves per SIMD (-> 463 ms).  The split
+ * walk keeps its seven: eight cost the 100^3 box 4%. */
+template <int MODE>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8)))
+k_walk32(TDV_WALK32_ARGS)
 {
-	TDV_WALK32_CALL(TDV_GROUP((int)blockIdx.x));
+	TDV_WALK32_CALL(MODE, TDV_GROUP((int)blockIdx.x));
 }
 
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6)))
 k_walk32_w6(TDV_WALK32_ARGS)
 {
-	TDV_WALK32_CALL(TDV_GROUP((int)blockIdx.x));
+	TDV_WALK32_CALL(WALK32_ANY, TDV_GROUP((int)blockIdx.x));
 }
 
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8)))
 k_walk32_w8(TDV_WALK32_ARGS)
 {
-	TDV_WALK32_CALL(TDV_GROUP((int)blockIdx.x));
+	TDV_WALK32_CALL(WALK32_ANY, TDV_GROUP((int)blockIdx.x));
 }
 
 /* Parts per group: 1 when the active groups alone fill the chip, else
@@ -1308,8 +1340,8 @@ __global__ void __launch_bounds__(64) k_walk32_queue(const int *__restrict__ nac
 		if (item >= nitems)
 			break;
 		const int gi = item / nparts;
-		TDV_WALK32_CALL_PARTW(TDV_GROUP(gi), item - gi * nparts, nparts,
-				partial, nslot, wmask);
+		TDV_WALK32_CALL_PARTW(WALK32_ANY, TDV_GROUP(gi), item - gi * nparts,
+				nparts, partial, nslot, wmask);
 	}
 }
 
@@ -1318,7 +1350,7 @@ __global__ void __launch_bounds__(64) k_walk32_queue(const int *__restrict__ nac
  * queue.  A grid sized for the largest case serves any active count (a
  * captured graph), the workgroups past the last item leave at once; with
  * the register budgets of the plain walk. */
-#define TDV_WALK32_ITEMS_BODY                                               \
+#define TDV_WALK32_ITEMS_BODY(MODE)                                            \
 	nact = *nact_dev;                                                      \
 	const int ngroups = (nact + 63) / 64;                                  \
 	const int nparts = walk32_parts(ngroups, split);                       \
@@ -1326,15 +1358,16 @@ __global__ void __launch_bounds__(64) k_walk32_queue(const int *__restrict__ nac
 	if (item >= ngroups * nparts)                                          \
 		return;                                                            \
 	const int gi = item / nparts;                                          \
-	TDV_WALK32_CALL_PARTW(TDV_GROUP(gi), item - gi * nparts, nparts,       \
+	TDV_WALK32_CALL_PARTW(MODE, TDV_GROUP(gi), item - gi * nparts, nparts, \
 			partial, ngroups * 64, wmask)
 
+template <int MODE>
 __global__ void __launch_bounds__(64) k_walk32_items(
 		const int *__restrict__ nact_dev, int split,
 		double4 *__restrict__ partial,
 		const unsigned long long *__restrict__ wmask, TDV_WALK32_ARGS)
 {
-	TDV_WALK32_ITEMS_BODY;
+	TDV_WALK32_ITEMS_BODY(MODE);
 }
 
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6)))
@@ -1342,7 +1375,7 @@ k_walk32_items_w6(const int *__restrict__ nact_dev, int split,
 		double4 *__restrict__ partial,
 		const unsigned long long *__restrict__ wmask, TDV_WALK32_ARGS)
 {
-	TDV_WALK32_ITEMS_BODY;
+	TDV_WALK32_ITEMS_BODY(WALK32_ANY);
 }
 
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8)))
@@ -1350,7 +1383,7 @@ k_walk32_items_w8(const int *__restrict__ nact_dev, int split,
 		double4 *__restrict__ partial,
 		const unsigned long long *__restrict__ wmask, TDV_WALK32_ARGS)
 {
-	TDV_WALK32_ITEMS_BODY;
+	TDV_WALK32_ITEMS_BODY(WALK32_ANY);
 }
 
 /* The parts' sums of a split walk, in part order, to the particles (as
@@ -1654,6 +1687,8 @@ int tdv_walk32(tdv_context *c, int use_bh)
 	w.crit3 = c->par.fp32_criterion == 3;
 	w.bundle_min = c->par.fp32_bundle_min == 0 ? 4
 			: c->par.fp32_bundle_min < 0 ? 0x7FFFFFFF : c->par.fp32_bundle_min;
+	const int mode = use_bh || !w.quad ? WALK32_ANY
+			: w.periodic ? WALK32_PERIODIC : WALK32_ISOLATED;
 	const int split = c->par.fp32_split;
 	const int ngroups_h = (int)((c->nactive + 63) / 64);
 	const int nparts_h = walk32_parts(ngroups_h, split);
@@ -1698,7 +1733,10 @@ int tdv_walk32(tdv_context *c, int use_bh)
 				? std::max((n + 63) / 64, (size_t)TDV_SPLIT_ITEMS)
 				: (size_t)ngroups_h * nparts_h;
 		auto kern = c->par.fp32_waves == 6 ? k_walk32_items_w6
-				: c->par.fp32_waves == 8 ? k_walk32_items_w8 : k_walk32_items;
+				: c->par.fp32_waves == 8 ? k_walk32_items_w8
+				: mode == WALK32_PERIODIC ? k_walk32_items<WALK32_PERIODIC>
+				: mode == WALK32_ISOLATED ? k_walk32_items<WALK32_ISOLATED>
+				: k_walk32_items<WALK32_ANY>;
 		hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(64), 0,
 				c->stream, c->d_nactive, split, c->partial, c->wmask, 0,
 				c->active,
@@ -1737,7 +1775,10 @@ int tdv_walk32(tdv_context *c, int use_bh)
 	}
 	TDV_TRY(tdv_clear_counts(c));
 	auto kern = c->par.fp32_waves == 6 ? k_walk32_w6
-			: c->par.fp32_waves == 8 ? k_walk32_w8 : k_walk32;
+			: c->par.fp32_waves == 8 ? k_walk32_w8
+			: mode == WALK32_PERIODIC ? k_walk32<WALK32_PERIODIC>
+			: mode == WALK32_ISOLATED ? k_walk32<WALK32_ISOLATED>
+			: k_walk32<WALK32_ANY>;
 	hipLaunchKernelGGL(kern, dim3(tdv_blocks((size_t)c->nactive, 64)),
 			dim3(64), 0, c->stream, c->nactive, c->active, c->p32, c->last_acc,
 			c->top, reinterpret_cast<const Node32 *>(c->rec32), c->ewald16, w,

@@ -35,6 +35,33 @@ def test_queue_walk_matches_grid_walk():
     assert a.interaction_counts() == b.interaction_counts()
 
 
+@pytest.mark.parametrize("periodic,n,order,split", [
+    (True, 20, 2, 1), (True, 13, 2, 0), (True, 20, 1, 0),
+    (False, 30011, 2, 1), (False, 3, 2, 0), (False, 999, 2, 0)])
+def test_usual_walk_matches_general_walk(periodic, n, order, split):
+    """The walks with the usual switches as constants take the same terms in
+    the same order as the general kernel (fp32_waves=6): equal bit for bit."""
+    if periodic:
+        pos, _, m = ics.zeldovich_box(n, seed=7)
+    else:
+        pos, _, m = ics.hernquist_sphere(n, seed=7)
+    got = []
+    for waves in (0, 6):
+        e = Engine(periodic=periodic, softening=1 / 640. if periodic else 0.01,
+                   alpha_rel=0.01, precision="fp32", compat=False,
+                   ewald_size=0.125, ewald_accuracy=1.0, fp32_order=order,
+                   fp32_criterion=3, fp32_waves=waves, fp32_split=split)
+        e.set_particles(pos, m)
+        e.setup_domain()
+        e.domain_decomposition()
+        e.compute_acceleration(True)
+        e.compute_acceleration(False)
+        got.append((e.get("acc", "cost"), e.interaction_counts()))
+    np.testing.assert_array_equal(got[0][0]["acc"], got[1][0]["acc"])
+    np.testing.assert_array_equal(got[0][0]["cost"], got[1][0]["cost"])
+    assert got[0][1] == got[1][1]
+
+
 def test_graph_replays_match_eager_walk():
     pos, _, m = ics.zeldovich_box(32, seed=7)
     e = _engine(pos, m, 1)
