@@ -156,6 +156,33 @@ __device__ __forceinline__ double lane_f64(double v, int l)
 	return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
 }
 
+/* 1 / sqrt(x), each rounded once, as `1 / sqrt(x)` gives them, where *ok
+ * holds; elsewhere (exponents beyond 2^+-500, zero, infinity, NaN) the
+ * caller takes `1 / sqrt(x)`.  The root by Goldschmidt's iteration from the
+ * hardware's estimate with two exact residuals, as the compiler's own; its
+ * half-reciprocal h, good to 2^-45 then, also starts the division: one
+ * Newton step brings 2h within (1/2 + 2^-30) ulp of 1 / g, and a second one,
+ * its residual exact, rounds correctly (Markstein, IBM J. Res. Dev. 34,
+ * 1990) for every g but the one with all mantissa bits set, which only x
+ * just below an even power of two has: those are left to the caller too.
+ * 20 instructions instead of 29, without the scaling and fix-up steps of
+ * either operation. */
+__device__ __forceinline__ double inv_sqrt(double x, bool *ok)
+{
+	const uint32_t hi = (uint32_t)((uint64_t)__double_as_longlong(x) >> 32);
+	*ok = hi - (523u << 20) < (1000u << 20) && ((hi + 1) & 0xFFFFFu) != 0;
+	const double r = __builtin_amdgcn_rsq(x);
+	double g = x * r, h = 0.5 * r;
+	const double e = __builtin_fma(-h, g, 0.5);
+	h = __builtin_fma(h, e, h);
+	g = __builtin_fma(g, e, g);
+	g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+	g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+	double y = h + h;
+	y = __builtin_fma(__builtin_fma(-g, y, 1.0), y, y);
+	return __builtin_fma(__builtin_fma(-g, y, 1.0), y, y);
+}
+
 /* Ewald_Correction, Gravity/periodic.c:35-113 (table already / Box^2):
  * the table cell of a separation, its trilinear weights and the signs */
 struct EwaldCell {

@@ -61,7 +61,10 @@ __device__ __forceinline__ double kernel_fac(double m, double r2,
 		const double u2 = r2 / w.eps2;
 		fac *= (175 - u2 * (294 - u2 * 135)) / (16 * w.eps3);
 	} else {
-		const double r_inv = 1 / sqrt(r2);
+		bool ok;
+		double r_inv = inv_sqrt(r2, &ok);
+		if (!ok)
+			r_inv = 1 / sqrt(r2);
 		fac *= r_inv * r_inv * r_inv;
 	}
 	return fac;
@@ -143,38 +146,52 @@ __device__ __forceinline__ void team_add(Acc &a, double x, double y, double z,
 	a.cost += __popcll(hits & ((1ull << L) - 1));
 }
 
-/* P-P with U particles of a uniform range, in the reference's order.  Where
- * no pair is inside the softening length (and none is the particle itself)
- * the U roots and divisions, which are most of an interaction, are
- * independent chains. */
+/* The factors of U interactions with r2 > 0 (kernel_fac): the roots and
+ * divisions, which are most of an interaction, as independent chains */
+template <int U>
+__device__ __forceinline__ void kernel_facs(double (&fac)[U],
+		const double (&m)[U], const double (&r2)[U], const WalkParams &w)
+{
+	bool all = true;
+#pragma unroll
+	for (int u = 0; u < U; u++) {
+		bool ok;
+		const double r_inv = inv_sqrt(r2[u], &ok);
+		fac[u] = w.G * m[u];
+		fac[u] *= r_inv * r_inv * r_inv;
+		all = all && ok && !(r2[u] < w.eps2);
+	}
+	if (!all) {
+#pragma unroll
+		for (int u = 0; u < U; u++)
+			fac[u] = kernel_fac(m[u], r2[u], w);
+	}
+}
+
+/* P-P with U particles of a uniform range, in the reference's order */
 template <int U>
 __device__ __forceinline__ void pp_batch(Acc &a, const double4 (&q)[U],
 		double px, double py, double pz, const WalkParams &w)
 {
-	double dx[U], dy[U], dz[U], r2[U];
-	bool near = false;
+	double dx[U], dy[U], dz[U], r2[U], m[U], fac[U];
+	bool self = false;
 #pragma unroll
 	for (int u = 0; u < U; u++) {
 		dx[u] = wrap(q[u].x - px, w);
 		dy[u] = wrap(q[u].y - py, w);
 		dz[u] = wrap(q[u].z - pz, w);
 		r2[u] = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u];
-		near = near || !(r2[u] >= w.eps2 && r2[u] > 0);
+		m[u] = q[u].w;
+		self = self || r2[u] == 0;
 	}
-	if (near) {
+	if (self) {
 #pragma unroll
 		for (int u = 0; u < U; u++)
 			if (r2[u] != 0)
-				interact(a, q[u].w, dx[u], dy[u], dz[u], r2[u], w);
+				interact(a, m[u], dx[u], dy[u], dz[u], r2[u], w);
 		return;
 	}
-	double fac[U];
-#pragma unroll
-	for (int u = 0; u < U; u++) {
-		const double r_inv = 1 / sqrt(r2[u]);
-		fac[u] = w.G * q[u].w;
-		fac[u] *= r_inv * r_inv * r_inv;
-	}
+	kernel_facs<U>(fac, m, r2, w);
 #pragma unroll
 	for (int u = 0; u < U; u++) {
 		a.x += fac[u] * dx[u];
@@ -206,20 +223,21 @@ __device__ __forceinline__ void pp_range_on(Acc &a, const double4 *pm,
 		}
 	} else {
 		const int sub = threadIdx.x & (L - 1);
-		double4 n = pm[first + sub < last ? first + sub : last - 1];
+		double4 n = pm[min(first + sub, last - 1)];
 		for (int j = first; j < last; j += L) {
 			const double4 q = n;
-			const int kn = j + L + sub;
-			n = pm[kn < last ? kn : last - 1];
+			n = pm[min(j + L + sub, last - 1)];
 			if (!on)
 				continue;
 			const double dx = wrap(q.x - px, w), dy = wrap(q.y - py, w),
 					dz = wrap(q.z - pz, w);
 			const double r2 = dx * dx + dy * dy + dz * dz;
 			const bool hit = j + sub < last && r2 != 0;
-			const double fac = hit ? kernel_fac(q.w, r2, w) : 0.0;
-			team_add<L>(a, hit ? fac * dx : 0.0, hit ? fac * dy : 0.0,
-					hit ? fac * dz : 0.0, hit, last - j);
+			const double m[1] = { q.w }, d2[1] = { hit ? r2 : 1.0 };
+			double fac[1];
+			kernel_facs<1>(fac, m, d2, w);
+			team_add<L>(a, hit ? fac[0] * dx : 0.0, hit ? fac[0] * dy : 0.0,
+					hit ? fac[0] * dz : 0.0, hit, last - j);
 		}
 	}
 }
@@ -257,7 +275,13 @@ __device__ __forceinline__ int wave_min(int v)
  * neighbours' walks share most nodes, so the wavefront visits little more
  * than one walk's nodes, without the per-lane gathers and divergent
  * branches of independent loops. */
-template <int L>
+/* Bound by instruction latency and, in the tail, by the longest walks.  With
+ * the periodic switch a constant and the short inverse root (inv_sqrt) the
+ * Hernquist sphere of 65536 takes 2.5 ms instead of 3.0, 14000 particles 1.2
+ * instead of 1.5, the box of 64^3 126 instead of 157.  Two particles per
+ * lane and turn gained nothing (and 24 registers more), nor did loading a
+ * node's three records at once. */
+template <int L, bool PERIODIC>
 __global__ void __launch_bounds__(256) k_walk64(int nact,
 		const int *__restrict__ active, const double4 *__restrict__ pm,
 		const double *__restrict__ last_acc, TopNodes T,
@@ -268,6 +292,7 @@ __global__ void __launch_bounds__(256) k_walk64(int nact,
 		double *__restrict__ gz, double *__restrict__ cost, int npart_total,
 		unsigned *err, unsigned long long *counter)
 {
+	w.periodic = PERIODIC;               /* a constant */
 	const int gid = (int)((blockIdx.x * blockDim.x + threadIdx.x) / L);
 	const bool live = gid < nact;
 	const int ip = live ? active[gid] : 0;
@@ -406,7 +431,6 @@ __device__ __forceinline__ void ewald_pp_range_on(Acc &a, const double *tab,
 		double pz, bool on, const WalkParams &w)
 {
 	constexpr int U = 2;
-	const int sub = threadIdx.x & (L - 1);
 	if constexpr (L == 1) {
 		int j = first;
 		for (; j + U <= last; j += U) {
@@ -442,11 +466,11 @@ __device__ __forceinline__ void ewald_pp_range_on(Acc &a, const double *tab,
 				ewald_cube(a, tab, dx, dy, dz, q.w, w);
 		}
 	} else {
-		double4 n = pm[first + sub < last ? first + sub : last - 1];
+		const int sub = threadIdx.x & (L - 1);
+		double4 n = pm[min(first + sub, last - 1)];
 		for (int j = first; j < last; j += L) {
 			const double4 q = n;
-			const int kn = j + L + sub;
-			n = pm[kn < last ? kn : last - 1];
+			n = pm[min(j + L + sub, last - 1)];
 			if (!on)
 				continue;
 			const double dx = wrap(q.x - px, w), dy = wrap(q.y - py, w),
@@ -474,6 +498,7 @@ __global__ void __launch_bounds__(256) k_walk64_ewald(int nact,
 		double *__restrict__ cost, int npart_total, unsigned *err,
 		unsigned long long *counter)
 {
+	w.periodic = 1;                      /* a constant */
 	const int gid = (int)((blockIdx.x * blockDim.x + threadIdx.x) / L);
 	const bool live = gid < nact;
 	const int ip = live ? active[gid] : 0;
@@ -631,25 +656,27 @@ static WalkParams walk_params(const tdv_context *c, int use_bh)
  * wavefront to wait for); they pay with L instead of one addition per
  * component for each of the wavefront's pairs, a quarter of the Newton
  * walk's time with teams of 4 and 1.5 times it with 16, little beside the
- * Ewald walk's gathers.  Measured in ms for teams of 1, 4 and 16, the walk
- * with one lane per particle in workgroups of 256 before them in brackets:
- *   Newton, Hernquist  8192: 1.63, 1.05, 0.88 [2.26]; 14000: 2.56, 1.64,
- *     1.74 [3.52]; 65536: 4.30, 3.79, 5.23 [5.91]; 10^6: 24.4, 24.0 [30.1]
- *   Newton, periodic box 24^3: 4.36, 2.21, 2.72 [5.72]; 40^3: 18.8, 19.6,
- *     38.3 [23.8]; 64^3: 157, 221, 452 [169]
- *   Ewald, periodic box 24^3: 6.52, 3.47, 3.57 [10.4]; 40^3: 20.2, 19.4,
- *     23.3 [28.8]; 64^3: 225, 223, 230 [310]; 80^3: 87, 51 [94]
- * So the Newton walk takes teams of 4 while one lane each would be less
- * than a wavefront per SIMD (65536 particles), the Ewald walk always, both
- * teams of 16 up to 10240 particles.  A wavefront per workgroup spreads few
- * of them over more CUs; the large Newton walks keep four neighbours on one
- * CU, which share its scalar cache (64^3: 182 ms apart, 157 together). */
+ * Ewald
+ * walk's gathers.  Measured in ms for teams of 1, 4 and 16:
+ *   Newton, Hernquist  8192: 1.35, 0.88, 0.79; 14000: 1.83, 1.21, 1.48;
+ *     30000: 2.35, 1.91, 2.42; 65536: 2.48, 2.50, 3.84; 10^6: 15.2, 15.1,
+ *     26.5; periodic box 24^3: 3.79, 1.96, 2.47; 40^3: 16.7, 17.8, 32.5;
+ *     64^3: 126, 191, 393
+ *   Ewald, periodic box 20^3: 1.96, 1.89, 1.53; 24^3: 3.56, 3.41, 3.37;
+ *     40^3: 15.5, 15.6, 17; 64^3: 186, 187, 184
+ * So the Newton walk takes teams of 4 up to three quarters of a wavefront
+ * per SIMD with one lane each (49152 particles), the Ewald walk always (it
+ * needs fewer registers than one lane with two gathers: 80^3 87 and 51 ms
+ * before the inverse roots were shortened), both teams of 16 up to 10240
+ * particles.  A wavefront per workgroup spreads few of them over more CUs;
+ * the large Newton walks keep four neighbours on one CU, which share its
+ * scalar cache (64^3: 182 ms apart, 157 together, then). */
 struct Walk64Shape {
 	int team, block;
 };
 
 #define TDV_W64_TEAM16 10240
-#define TDV_W64_TEAM4 65536
+#define TDV_W64_TEAM4 49152
 #define TDV_W64_TEAM_MAX (1 << 28)       /* thread numbers within 32 bits */
 
 static Walk64Shape walk64_shape(int nact, bool ewald)
@@ -668,7 +695,11 @@ int tdv_walk64(tdv_context *c, int use_bh)
 	const WalkParams w = walk_params(c, use_bh);
 	const Walk64Shape sh = walk64_shape(c->nactive, false);
 	const int L = sh.team;
-	auto kern = L == 16 ? k_walk64<16> : L == 4 ? k_walk64<4> : k_walk64<1>;
+	auto kern = w.periodic
+			? (L == 16 ? k_walk64<16, true> : L == 4 ? k_walk64<4, true>
+				: k_walk64<1, true>)
+			: (L == 16 ? k_walk64<16, false> : L == 4 ? k_walk64<4, false>
+				: k_walk64<1, false>);
 	hipLaunchKernelGGL(kern, dim3(tdv_blocks((size_t)c->nactive * L, sh.block)),
 			dim3(sh.block), 0, c->stream, c->nactive, c->active, c->pm, c->last_acc,
 			c->top, c->node_a, c->node_b, c->node_c, w, c->acc[0], c->acc[1],

@@ -254,13 +254,23 @@ def test_lane_teams_leave_the_same_bits(periodic, ewald):
         return got["acc"][sub], got["cost"][sub], e.interaction_counts()
 
     acc, cost, _ = walk(np.arange(n, dtype=np.int32))
-    for k in (65536, 65535, 10241, 10240, 129, 1):
+    for k in (65536, 65535, 49153, 49152, 10241, 10240, 129, 1):
         sub = np.sort(np.random.Generator(np.random.Philox(k)).choice(
             n, k, replace=False)).astype(np.int32)
         a, c, counts = walk(sub)
         np.testing.assert_array_equal(a, acc[sub], err_msg=str(k))
         np.testing.assert_array_equal(c, cost[sub], err_msg=str(k))
         assert sum(counts) == int(c.sum())
+
+
+@pytest.mark.parametrize("n", [300, 20000])
+def test_walk_at_tiny_separations_matches_oracle(n):
+    """A sphere of radius ~ 2^-247: r^2 on both sides of 2^-500, where the
+    walks' inverse root changes from the short form to `1 / sqrt(r2)`."""
+    pos, _, m = ics.hernquist_sphere(n, seed=3)
+    s, e = _pipeline_pair(pos * 2.0 ** -248, m, False, None,
+                          softening=2.0 ** -256)
+    _compare(s, e)
 
 
 @pytest.mark.parametrize("n", [3, 4, 5, 257, 1025, 70001])
