@@ -15,11 +15,16 @@
 
 /* Two workgroups per CU keep the table's gathers busy, which bound a pair
  * (more of them only spread the sources' separations over more of the table:
- * 512 targets in 64^3 particles take 3.4 ms in one part each, 3.7 in four);
+ * 512 targets in 64^3 particles take 3.0 ms in one part each, 3.1 in two);
  * with fewer targets than that the sources are cut into parts of at least
  * TDV_DIRECT_MIN (16 targets 1.56 -> 0.15 ms, 100 targets 1.72 -> 0.95 ms). */
 #define TDV_DIRECT_BLOCKS 512
 #define TDV_DIRECT_MIN 2048
+/* Periodic sums from so many sources on take two at a time from the table's
+ * rows (see k_direct).  512 and 1000 targets, ms: in 24^3 particles 0.23 and
+ * 0.41 so, 0.23 and 0.39 one at a time from the components' own tables; in
+ * 32^3 0.44 and 0.84, 0.47 and 0.86; in 64^3 2.9 and 5.9, 3.4 and 6.7. */
+#define TDV_DIRECT_ROWS 32768
 
 __device__ __forceinline__ double dwrap(double d, int periodic, double box,
 		double half)
@@ -33,6 +38,13 @@ __device__ __forceinline__ double dwrap(double d, int periodic, double box,
 	return d;
 }
 
+/* Bound by the table's lines: the separations of 64 neighbouring sources lie
+ * in some hundred cells, 27 KB of the rows' lines (46 KB of the components'),
+ * each used once.  The next sources are loaded and U gathers are in flight
+ * while a pair's sum is formed: 512 targets in 64^3 particles 3.5 -> 2.9 ms
+ * (rows and U = 2; copying the cells to LDS first took 6.1, its latency bare
+ * with the few wavefronts that fit). */
+template <bool ROWS, int U>
 __global__ void __launch_bounds__(256) k_direct(int nt,
 		const int *__restrict__ idx, const double4 *__restrict__ pm, int n,
 		int periodic, double box, double G, double eps2, double eps3,
@@ -50,33 +62,48 @@ __global__ void __launch_bounds__(256) k_direct(int nt,
 	const double4 p = pm[i];
 	const double half = box / 2.0;
 	double ax = 0, ay = 0, az = 0;
-	for (int j = first + threadIdx.x; j < last; j += blockDim.x) {
-		if (j == i)
-			continue;
-		const double4 q = pm[j];
-		const double dx = dwrap(q.x - p.x, periodic, box, half);
-		const double dy = dwrap(q.y - p.y, periodic, box, half);
-		const double dz = dwrap(q.z - p.z, periodic, box, half);
-		const double r2 = dx * dx + dy * dy + dz * dz;
-		if (r2 == 0)
-			continue;
-		double fac = G * q.w;
-		if (r2 < eps2) {
-			const double u2 = r2 / eps2;
-			fac *= (175 - u2 * (294 - u2 * 135)) / (16 * eps3);
-		} else {
-			const double ri = 1 / sqrt(r2);
-			fac *= ri * ri * ri;
+	double4 next[U];
+#pragma unroll
+	for (int u = 0; u < U; u++)
+		next[u] = pm[min(first + (int)threadIdx.x + 256 * u, last - 1)];
+	for (int j = first + threadIdx.x; j < last; j += 256 * U) {
+		double dx[U], dy[U], dz[U], m[U], f[U][3];
+#pragma unroll
+		for (int u = 0; u < U; u++) {
+			dx[u] = dwrap(next[u].x - p.x, periodic, box, half);
+			dy[u] = dwrap(next[u].y - p.y, periodic, box, half);
+			dz[u] = dwrap(next[u].z - p.z, periodic, box, half);
+			m[u] = G * next[u].w;
+			next[u] = pm[min(j + 256 * (U + u), last - 1)];
+			if (periodic && ROWS)
+				ewald_corr_rows(tab, dx[u], dy[u], dz[u], b2e, f[u]);
+			else if (periodic)
+				ewald_corr(tab, dx[u], dy[u], dz[u], b2e, f[u]);
 		}
-		ax += fac * dx;
-		ay += fac * dy;
-		az += fac * dz;
-		if (periodic) {
-			double f[3];
-			ewald_corr(tab, dx, dy, dz, b2e, f);
-			ax += G * q.w * f[0];
-			ay += G * q.w * f[1];
-			az += G * q.w * f[2];
+#pragma unroll
+		for (int u = 0; u < U; u++) {
+			const double r2 = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u];
+			if (j + 256 * u >= last || j + 256 * u == i || r2 == 0)
+				continue;
+			double fac = m[u];
+			if (r2 < eps2) {
+				const double u2 = r2 / eps2;
+				fac *= (175 - u2 * (294 - u2 * 135)) / (16 * eps3);
+			} else {
+				bool ok;
+				double ri = inv_sqrt(r2, &ok);
+				if (!ok)
+					ri = 1 / sqrt(r2);
+				fac *= ri * ri * ri;
+			}
+			ax += fac * dx[u];
+			ay += fac * dy[u];
+			az += fac * dz[u];
+			if (periodic) {
+				ax += m[u] * f[u][0];
+				ay += m[u] * f[u][1];
+				az += m[u] * f[u][2];
+			}
 		}
 	}
 	red[0][threadIdx.x] = ax;
@@ -121,11 +148,14 @@ int tdv_direct_sum(tdv_context *c, int nt, const int *idx_dev, double *out_dev)
 	const int chunk = (int)((n + parts - 1) / parts);
 	parts = (n + chunk - 1) / chunk;
 	double *sums = parts > 1 ? reinterpret_cast<double *>(c->sk[0]) : out_dev;
-	hipLaunchKernelGGL(k_direct, dim3(nt, (unsigned)parts), dim3(256), 0,
+	const bool rows = c->par.periodic && n >= TDV_DIRECT_ROWS;
+	auto kern = rows ? k_direct<true, 2> : k_direct<false, 1>;
+	hipLaunchKernelGGL(kern, dim3(nt, (unsigned)parts), dim3(256), 0,
 			c->stream, nt, idx_dev, c->pm, (int)n, c->par.periodic,
 			c->par.boxsize, c->par.gravity, c->Epsilon2, c->Epsilon3,
-			c->ewald, 2 * TDV_NE / (c->par.periodic ? c->par.boxsize : 1.0),
-			chunk, sums);
+			rows ? c->ewald_rows : c->ewald,
+			2 * TDV_NE / (c->par.periodic ? c->par.boxsize : 1.0), chunk,
+			sums);
 	if (parts > 1)
 		hipLaunchKernelGGL(k_direct_parts, dim3(tdv_blocks(3 * (size_t)nt,
 				256)), dim3(256), 0, c->stream, 3 * nt, (int)parts, sums,

@@ -49,6 +49,25 @@ def test_forcetest_matches_cpu_direct_sum(periodic, table):
     assert rel_err(got, want).max() < 1e-11
 
 
+@pytest.mark.parametrize("n,nt", [(32767, 3), (32768, 3), (32769, 40),
+                                  (33281, 600), (40000, 1)])
+def test_forcetest_by_table_rows_matches_cpu(n, nt, table):
+    """Either side of the number of sources from which they are taken two at
+    a time from the table's rows, and remainders of 512."""
+    pos, _, m = ics.clustered_box(n, nhalo=16, seed=11)
+    soft = 1e-3
+    e = Engine(periodic=True, softening=soft, ewald_table=table)
+    s = oracle.Sim(pos, m, periodic=True, softening=soft, ewald_table=table,
+                   nthreads=16)
+    e.set_particles(pos, m)
+    for x in (e, s):
+        x.setup_domain()
+        x.domain_decomposition()
+    idx = np.linspace(0, n - 1, nt).astype(np.int32)
+    # same terms, different summation order
+    assert rel_err(e.forcetest(idx), s.direct_sum(idx)).max() < 1e-11
+
+
 def _fp32_error(pos, m, periodic, soft, alpha, esize, table, order=2):
     e64 = Engine(periodic=periodic, softening=soft, alpha_rel=alpha,
                  ewald_table=table if periodic else None)
