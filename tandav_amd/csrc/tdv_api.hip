@@ -431,7 +431,6 @@ void tdv_destroy(tdv_context *c)
 	dfree(c->ewald_j);
 	dfree(c->p32);
 	dfree(c->p32o);
-	dfree(c->a32);
 	dfree(c->rec32);
 	dfree(c->ctr32);
 	dfree(c->q32);

@@ -169,7 +169,7 @@ struct tdv_context {
 	int have_ewald;
 
 	/* FP32 group walk: fixed-point records */
-	int4 *p32, *a32;
+	int4 *p32;
 	int4 *rec32;                     /* 64-byte node records, 4 int4 each */
 	int4 *ctr32;                     /* node cell centres, fixed units */
 	float4 *p32o;                    /* offset from the leaf's CoM, mass' */

@@ -110,76 +110,117 @@ struct __align__(64) Node32 {
 	int4 a, b, c, q;
 };
 
-/* Every node's cell centre in fixed units, from its first particle (the
- * opening test's centre), when the records are made for a tree; a
- * substep's records keep them */
-__global__ void k_prep32_centres(size_t bound, const int *__restrict__ nn,
-		const int4 *__restrict__ nc, const double4 *__restrict__ pm,
-		double o0, double o1, double o2, double S, int bits,
-		int4 *__restrict__ ctr)
+/* One launch makes every record of a walk: workgroups of 256 nodes, then of
+ * 256 particles, then of 256 top nodes.  None needs another's (a particle
+ * takes its bundle's centre of mass from the tree).  A substep of 65,000
+ * particles: 5.7 us in three launches with gaps of 4 us between them, now
+ * 3.3 in one; a cycle of 128 substeps 38.4 -> 37.7 ms. */
+struct Prep32 {
+	size_t bound, n;                 /* nodes at most, particles */
+	unsigned nblk, pblk;             /* workgroups of nodes, of particles */
+	double o0, o1, o2, S, mscale;
+	int bits, quad, make_centres;
+	const double4 *na, *nb, *pm;
+	const int4 *nc;
+	const float4 *q32;
+	const int *leaf;
+	int4 *ctr, *t32, *p32;
+	Node32 *rec;
+	float4 *p32o;
+};
+
+__device__ __forceinline__ int4 prep_com(double x, double y, double z,
+		double m, const Prep32 &w)
 {
-	const size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (j >= bound || (long long)j >= (long long)*nn)
-		return;
-	const int4 c = nc[j];
-	if (c.w < 0) {                       /* terminator */
-		ctr[j] = make_int4(0, 0, 0, 0);
-		return;
-	}
-	const double4 q = pm[c.w];
-	const int lv = c.z & 63;
-	ctr[j] = make_int4((int)cell_centre(fixp(q.x, o0, S), lv, bits),
-			(int)cell_centre(fixp(q.y, o1, S), lv, bits),
-			(int)cell_centre(fixp(q.z, o2, S), lv, bits), 0);
+	return make_int4((int)fixp(x, w.o0, w.S), (int)fixp(y, w.o1, w.S),
+			(int)fixp(z, w.o2, w.S), __float_as_int((float)(m * w.mscale)));
 }
 
-/* the records from the tree (node_c, FP64 CoM and size) and the
- * quadrupoles; a32 keeps {CoM, m'} */
-__global__ void k_prep32_nodes(size_t bound, const int *__restrict__ nn,
-		const double4 *__restrict__ na,
-		const double4 *__restrict__ nb, const int4 *__restrict__ nc,
-		const float4 *__restrict__ q32, int quad, const int4 *__restrict__ ctr,
-		double o0, double o1, double o2, double S, double mscale,
-		int4 *__restrict__ a32, Node32 *__restrict__ rec)
+/* A node's record from the tree (node_c, FP64 CoM and size) and the
+ * quadrupoles.  Its cell centre in fixed units, from its first particle
+ * (the opening test's centre), is made with the records of a new tree; a
+ * substep's records keep it. */
+__device__ __forceinline__ void prep_node(size_t j, const Prep32 &w)
 {
-	const size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (j >= bound || (long long)j >= (long long)*nn)
-		return;
-	const double4 a = na[j], b = nb[j];
-	const int4 c = nc[j];
-	const int4 A = make_int4((int)fixp(a.x, o0, S), (int)fixp(a.y, o1, S),
-			(int)fixp(a.z, o2, S), __float_as_int((float)(a.w * mscale)));
-	a32[j] = A;
-	const float s = (float)(b.w * S);
+	const double4 a = w.na[j], b = w.nb[j];
+	const int4 c = w.nc[j];
+	int4 C = make_int4(0, 0, 0, 0);
+	if (!w.make_centres) {
+		C = w.ctr[j];
+	} else {
+		if (c.w >= 0) {                  /* not a terminator */
+			const double4 q = w.pm[c.w];
+			const int lv = c.z & 63;
+			C = make_int4(
+					(int)cell_centre(fixp(q.x, w.o0, w.S), lv, w.bits),
+					(int)cell_centre(fixp(q.y, w.o1, w.S), lv, w.bits),
+					(int)cell_centre(fixp(q.z, w.o2, w.S), lv, w.bits), 0);
+		}
+		w.ctr[j] = C;
+	}
+	const int4 A = prep_com(a.x, a.y, a.z, a.w, w);
+	const float s = (float)(b.w * w.S);
 	Node32 r;
 	r.a = A;
-	const int4 C = ctr[j];
 	r.b = make_int4(
 			__float_as_int((float)(int)((unsigned)C.x - (unsigned)A.x)),
 			__float_as_int((float)(int)((unsigned)C.y - (unsigned)A.y)),
 			__float_as_int((float)(int)((unsigned)C.z - (unsigned)A.z)),
 			__float_as_int(s));
 	float4 q0 = make_float4(0.f, 0.f, 0.f, 0.f), q1 = q0;
-	if (quad) {
-		q0 = q32[2 * j];
-		q1 = q32[2 * j + 1];
+	if (w.quad) {
+		q0 = w.q32[2 * j];
+		q1 = w.q32[2 * j + 1];
 	}
 	r.c = make_int4(c.x, c.y, __float_as_int(q0.x), __float_as_int(q0.y));
 	r.q = make_int4(__float_as_int(q0.z), __float_as_int(q0.w),
 			__float_as_int(q1.x), 0);
-	rec[j] = r;
+	w.rec[j] = r;
 }
 
-__global__ void k_prep32_top(const TopNodes T, double o0, double o1,
-		double o2, double S, double mscale, int4 *__restrict__ t32)
+/* A particle's fixed-point record (position, mass') and its offset from its
+ * bundle's centre of mass in fixed units (an exact integer difference,
+ * rounded once to FP32) with its mass', so a group taking the bundle in the
+ * CoM's frame adds one FP32 add per component.  (An offset from the bundle's
+ * cell centre, which a tree update does not move, lost an order of magnitude
+ * in accuracy on the Hernquist sphere: the centre lies farther from the
+ * particles.)  Particles of small top nodes (no leaf) are not read from the
+ * offsets. */
+__device__ __forceinline__ void prep_particle(size_t i, const Prep32 &w)
 {
-	const int t = blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= *T.ntop)
+	const double4 q = w.pm[i];
+	const int4 p = prep_com(q.x, q.y, q.z, q.w, w);
+	w.p32[i] = p;
+	const int j = w.leaf[i];
+	float4 o = make_float4(0.f, 0.f, 0.f, __int_as_float(p.w));
+	if (j >= 0) {
+		const double4 a = w.na[j];
+		const int4 c = prep_com(a.x, a.y, a.z, a.w, w);
+		o.x = (float)(int)((unsigned)p.x - (unsigned)c.x);
+		o.y = (float)(int)((unsigned)p.y - (unsigned)c.y);
+		o.z = (float)(int)((unsigned)p.z - (unsigned)c.z);
+	}
+	w.p32o[i] = o;
+}
+
+__global__ void __launch_bounds__(256) k_prep32(Prep32 w, const TopNodes T)
+{
+	if (blockIdx.x < w.nblk) {
+		const size_t j = (size_t)blockIdx.x * 256 + threadIdx.x;
+		if (j < w.bound && (long long)j < (long long)*T.nnodes)
+			prep_node(j, w);
 		return;
-	const double m = (double)T.mass[t] * mscale;
-	t32[t] = make_int4((int)fixp(T.com[3 * t], o0, S),
-			(int)fixp(T.com[3 * t + 1], o1, S), (int)fixp(T.com[3 * t + 2], o2, S),
-			__float_as_int((float)m));
+	}
+	if (blockIdx.x < w.nblk + w.pblk) {
+		const size_t i = (size_t)(blockIdx.x - w.nblk) * 256 + threadIdx.x;
+		if (i < w.n)
+			prep_particle(i, w);
+		return;
+	}
+	const int t = (int)((blockIdx.x - w.nblk - w.pblk) * 256 + threadIdx.x);
+	if (t < *T.ntop)
+		w.t32[t] = prep_com((double)T.com[3 * t], (double)T.com[3 * t + 1],
+				(double)T.com[3 * t + 2], (double)T.mass[t], w);
 }
 
 /* The walk's Ewald records, one per table node, 64 bytes: E, its first
@@ -222,37 +263,6 @@ __global__ void k_prep32_ewald_taylor(const double *__restrict__ raw,
 			pack_h2(S[2], S[3]), pack_h2(S[4], S[5]));
 	t[4 * i + 3] = make_float4(pack_h2(S[6], S[7]), pack_h2(S[8], S[9]), 0.f,
 			0.f);
-}
-
-/* Every particle's fixed-point record (position, mass') and, in one pass
- * (after the nodes' records), its offset from its bundle's centre of mass
- * in fixed units (an exact integer difference, rounded once to FP32) with
- * its mass', so a group taking the bundle in the CoM's frame adds one FP32
- * add per component.  (An offset from the bundle's cell centre, which a
- * tree update does not move, lost an order of magnitude in accuracy on the
- * Hernquist sphere: the centre lies farther from the particles.)  Particles
- * of small top nodes (no leaf) are not read from the offsets. */
-__global__ void k_prep32_particles(size_t n, const double4 *__restrict__ pm,
-		double o0, double o1, double o2, double S, double mscale,
-		const int *__restrict__ leaf, const int4 *__restrict__ a32,
-		int4 *__restrict__ p32, float4 *__restrict__ p32o)
-{
-	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	const double4 q = pm[i];
-	const int4 p = make_int4((int)fixp(q.x, o0, S), (int)fixp(q.y, o1, S),
-			(int)fixp(q.z, o2, S), __float_as_int((float)(q.w * mscale)));
-	p32[i] = p;
-	const int j = leaf[i];
-	float4 o = make_float4(0.f, 0.f, 0.f, __int_as_float(p.w));
-	if (j >= 0) {
-		const int4 c = a32[j];
-		o.x = (float)(int)((unsigned)p.x - (unsigned)c.x);
-		o.y = (float)(int)((unsigned)p.y - (unsigned)c.y);
-		o.z = (float)(int)((unsigned)p.z - (unsigned)c.z);
-	}
-	p32o[i] = o;
 }
 
 /* Quadrupoles of every node, bundle and top node, for the walk: the
@@ -1555,8 +1565,6 @@ int tdv_walk32(tdv_context *c, int use_bh)
 	}
 	if (c->n32_cap < c->node_cap) {
 		tdv_graph_drop(c);               /* the records move */
-		if (c->a32)
-			(void)hipFree(c->a32);
 		if (c->rec32)
 			(void)hipFree(c->rec32);
 		if (c->ctr32)
@@ -1567,10 +1575,9 @@ int tdv_walk32(tdv_context *c, int use_bh)
 		if (c->q_s6)
 			(void)hipFree(c->q_s6);
 		c->q_s6 = nullptr;
-		c->a32 = c->rec32 = nullptr;
+		c->rec32 = nullptr;
 		c->q32 = nullptr;
 		c->n32_cap = 0;
-		TDV_HIP(c, hipMalloc((void **)&c->a32, c->node_cap * sizeof(int4)));
 		TDV_HIP(c, hipMalloc((void **)&c->rec32,
 				c->node_cap * sizeof(Node32)));
 		TDV_HIP(c, hipMalloc((void **)&c->ctr32,
@@ -1620,23 +1627,14 @@ int tdv_walk32(tdv_context *c, int use_bh)
 			hipLaunchKernelGGL(k_moments_top, dim3((unsigned)tgrid), dim3(64), 0, c->stream, c->top, c->par.vector_size,
 					c->node_a, c->pm, c->q_s6, qscale, c->tq32);
 	}
-	if (tgrid)
-		hipLaunchKernelGGL(k_prep32_top, dim3(tdv_blocks((size_t)tgrid, 64)),
-				dim3(64), 0, c->stream, c->top, o[0], o[1], o[2], S, mscale,
-				c->top32);
-	if (bound && !c->substep_prep)
-		hipLaunchKernelGGL(k_prep32_centres, dim3(tdv_blocks(bound, 256)),
-				dim3(256), 0, c->stream, bound, c->top.nnodes, c->node_c,
-				c->pm, o[0], o[1], o[2], S, bits, c->ctr32);
-	if (bound)
-		hipLaunchKernelGGL(k_prep32_nodes, dim3(tdv_blocks(bound, 256)),
-				dim3(256), 0, c->stream, bound, c->top.nnodes, c->node_a,
-				c->node_b, c->node_c, c->q32, quad ? 1 : 0, c->ctr32, o[0],
-				o[1], o[2], S, mscale, c->a32,
-				reinterpret_cast<Node32 *>(c->rec32));
-	hipLaunchKernelGGL(k_prep32_particles, dim3(tdv_blocks(n, 256)), dim3(256),
-			0, c->stream, n, c->pm, o[0], o[1], o[2], S, mscale,
-			c->tree_parent, c->a32, c->p32, c->p32o);
+	const Prep32 prep = { bound, n, (unsigned)tdv_blocks(bound, 256),
+		(unsigned)tdv_blocks(n, 256), o[0], o[1], o[2], S, mscale, bits,
+		quad ? 1 : 0, !c->substep_prep, c->node_a, c->node_b, c->pm, c->node_c,
+		c->q32, c->tree_parent, c->ctr32, c->top32, c->p32,
+		reinterpret_cast<Node32 *>(c->rec32), c->p32o };
+	hipLaunchKernelGGL(k_prep32, dim3(prep.nblk + prep.pblk
+			+ (unsigned)tdv_blocks((size_t)tgrid, 256)), dim3(256), 0, c->stream,
+			prep, c->top);
 	if (c->par.periodic && !c->ewald16_ok) {
 		if (!c->have_ewald)
 			return tdv_fail(c, TDV_ERR_ARG, "FP32 walk without an Ewald table");
