@@ -770,8 +770,8 @@ __device__ __forceinline__ bool node_opens_ri(float m, float s, float r2,
 	const float ms2 = m * s * s;
 	const float lhs = w.crit3 ? ms2 * (s * ri) : ms2;
 	const float s6 = 0.6f * s;
-	return near | (lhs > (r2 * crit) * r2) | ((fabsf(sx) < s6)
-			& (fabsf(sy) < s6) & (fabsf(sz) < s6));
+	return near | (lhs > (r2 * crit) * r2)
+			| (fmaxf(fabsf(sx), fmaxf(fabsf(sy), fabsf(sz))) < s6);
 }
 
 /* An accepted node (r >= |eps| + s, outside the softening length): its
