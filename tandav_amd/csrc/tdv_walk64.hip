@@ -423,40 +423,17 @@ __device__ __forceinline__ void ewald_cube(Acc &a, const double *tab,
 	a.cost++;
 }
 
-/* as pp_range_on, with the Ewald correction of each pair; one lane per
- * particle takes two at a time, both gathers in flight */
+/* as pp_range_on, with the Ewald correction of each pair.  One lane per
+ * particle takes one pair at a time: with two gathers in flight it held 170
+ * registers instead of 102, two wavefronts per SIMD instead of four, and the
+ * walk of 256^3 particles took 1077 ms instead of 978. */
 template <int L>
 __device__ __forceinline__ void ewald_pp_range_on(Acc &a, const double *tab,
 		const double4 *pm, int first, int last, double px, double py,
 		double pz, bool on, const WalkParams &w)
 {
-	constexpr int U = 2;
 	if constexpr (L == 1) {
-		int j = first;
-		for (; j + U <= last; j += U) {
-			const double4 q[U] = { pm[j], pm[j + 1] };
-			if (!on)
-				continue;
-			double f[U][3];
-			bool hit[U];
-#pragma unroll
-			for (int u = 0; u < U; u++) {
-				const double dx = wrap(q[u].x - px, w),
-						dy = wrap(q[u].y - py, w), dz = wrap(q[u].z - pz, w);
-				hit[u] = dx != 0 && dy != 0 && dz != 0;
-				ewald_corr_rows(tab, dx, dy, dz, w.box2ewald, f[u]);
-			}
-#pragma unroll
-			for (int u = 0; u < U; u++) {
-				if (hit[u]) {
-					a.x += w.G * q[u].w * f[u][0];
-					a.y += w.G * q[u].w * f[u][1];
-					a.z += w.G * q[u].w * f[u][2];
-					a.cost++;
-				}
-			}
-		}
-		for (; j < last; j++) {
+		for (int j = first; j < last; j++) {
 			const double4 q = pm[j];
 			if (!on)
 				continue;
@@ -651,41 +628,61 @@ static WalkParams walk_params(const tdv_context *c, int use_bh)
 	return w;
 }
 
-/* Lanes per particle and threads per workgroup, from the active count.
- * Teams buy wavefronts and idle less in the lockstep (fewer particles per
- * wavefront to wait for); they pay with L instead of one addition per
- * component for each of the wavefront's pairs, a quarter of the Newton
- * walk's time with teams of 4 and 1.5 times it with 16, little beside the
- * Ewald
- * walk's gathers.  Measured in ms for teams of 1, 4 and 16:
- *   Newton, Hernquist  8192: 1.35, 0.88, 0.79; 14000: 1.83, 1.21, 1.48;
- *     30000: 2.35, 1.91, 2.42; 65536: 2.48, 2.50, 3.84; 10^6: 15.2, 15.1,
- *     26.5; periodic box 24^3: 3.79, 1.96, 2.47; 40^3: 16.7, 17.8, 32.5;
- *     64^3: 126, 191, 393
- *   Ewald, periodic box 20^3: 1.96, 1.89, 1.53; 24^3: 3.56, 3.41, 3.37;
- *     40^3: 15.5, 15.6, 17; 64^3: 186, 187, 184
- * So the Newton walk takes teams of 4 up to three quarters of a wavefront
- * per SIMD with one lane each (49152 particles), the Ewald walk always (it
- * needs fewer registers than one lane with two gathers: 80^3 87 and 51 ms
- * before the inverse roots were shortened), both teams of 16 up to 10240
- * particles.  A wavefront per workgroup spreads few of them over more CUs;
- * the large Newton walks keep four neighbours on one CU, which share its
- * scalar cache (64^3: 182 ms apart, 157 together, then). */
+/* Lanes per particle and threads per workgroup.  Teams buy wavefronts and
+ * idle less in the lockstep (fewer particles per wavefront to wait for);
+ * they pay with L instead of one addition per component for each of the
+ * wavefront's pairs, and with L lanes that test every node alike.
+ *
+ * Newton walk, ms for teams of 1, 4 and 16: Hernquist 8192: 1.35, 0.88,
+ * 0.79; 14000: 1.83, 1.21, 1.48; 30000: 2.35, 1.91, 2.42; 65536: 2.48, 2.50,
+ * 3.84; 10^6: 15.2, 15.1, 26.5; periodic box 24^3: 3.79, 1.96, 2.47; 40^3:
+ * 16.7, 17.8, 32.5; 64^3: 126, 191, 393.  So teams of 4 up to three quarters
+ * of a wavefront per SIMD with one lane each (49152 particles), of 16 up to
+ * 10240.  A wavefront per workgroup spreads few of them over more CUs; the
+ * large walks keep four neighbours on one CU, which share its scalar cache
+ * (64^3: 182 ms apart, 157 together, then).
+ *
+ * Ewald walk, ms for one lane, teams of 4 and of 16: box of 20^3: 4.97, 2.00,
+ * 1.65; 24^3: 8.32, 3.62, 3.69; 32^3: 21.1, 13.2, 14.7; of 10^6 uniform
+ * particles 10000: 12.1, 5.6 (one, 4).  It is bound by pairs where its walk
+ * reaches the bundles, by the node tests where the tree is deeper than that,
+ * and teams pay only for pairs.  With 98304 particles (a wavefront and a half
+ * per SIMD with one lane each) and fewer, idle SIMDs outweigh that and teams
+ * of 4 lost in no box.  With more the tree's size decides, over up to 131072
+ * nodes teams of 4 (one lane, 4): 110^3 218, 133; 128^3 (70784 nodes) 349,
+ * 248; uniform 10^6 113, 72; clustered 2^20 (98940) 20.5, 11.1, 1.3e6
+ * (129705) 13.5, 9.3; and beyond one lane: clustered 1.5e6 (152597) 5.4, 8.8,
+ * 2^23 14.6, 43.2; uniform 3e6 48, 141; 144^3 120, 170; 256^3 978, 1093.  The
+ * Barnes-Hut walk, which opens nodes of any depth, takes one lane there:
+ * 110^3 1606, 1620; clustered 2^20 558, 837, 6e6 3834, 6131; uniform 10^7
+ * 322, 1125. */
 struct Walk64Shape {
 	int team, block;
 };
 
 #define TDV_W64_TEAM16 10240
 #define TDV_W64_TEAM4 49152
+#define TDV_W64_EWALD_TEAM4 98304
+#define TDV_W64_EWALD_NODES 131072
 #define TDV_W64_TEAM_MAX (1 << 28)       /* thread numbers within 32 bits */
 
-static Walk64Shape walk64_shape(int nact, bool ewald)
+static Walk64Shape newton_shape(int nact)
 {
 	if (nact <= TDV_W64_TEAM16)
 		return { 16, 64 };
-	if (nact <= (ewald ? TDV_W64_TEAM_MAX : TDV_W64_TEAM4))
+	if (nact <= TDV_W64_TEAM4)
 		return { 4, 64 };
 	return { 1, 256 };
+}
+
+static Walk64Shape ewald_shape(int nact, size_t nnodes, int use_bh)
+{
+	if (nact <= TDV_W64_TEAM16)
+		return { 16, 64 };
+	if (nact <= TDV_W64_EWALD_TEAM4 || (!use_bh
+			&& nnodes <= TDV_W64_EWALD_NODES && nact <= TDV_W64_TEAM_MAX))
+		return { 4, 64 };
+	return { 1, 64 };
 }
 
 int tdv_walk64(tdv_context *c, int use_bh)
@@ -693,7 +690,7 @@ int tdv_walk64(tdv_context *c, int use_bh)
 	if (!c->nactive)
 		return 0;
 	const WalkParams w = walk_params(c, use_bh);
-	const Walk64Shape sh = walk64_shape(c->nactive, false);
+	const Walk64Shape sh = newton_shape(c->nactive);
 	const int L = sh.team;
 	auto kern = w.periodic
 			? (L == 16 ? k_walk64<16, true> : L == 4 ? k_walk64<4, true>
@@ -715,7 +712,7 @@ int tdv_walk64_ewald(tdv_context *c, int use_bh)
 	if (!c->have_ewald)
 		return tdv_fail(c, TDV_ERR_ARG, "periodic walk without an Ewald table");
 	const WalkParams w = walk_params(c, use_bh);
-	const Walk64Shape sh = walk64_shape(c->nactive, true);
+	const Walk64Shape sh = ewald_shape(c->nactive, c->nnodes, use_bh);
 	const int L = sh.team;
 	auto kern = L == 16 ? k_walk64_ewald<16> : L == 4 ? k_walk64_ewald<4>
 			: k_walk64_ewald<1>;

@@ -263,6 +263,42 @@ def test_lane_teams_leave_the_same_bits(periodic, ewald):
         assert sum(counts) == int(c.sum())
 
 
+@pytest.mark.parametrize("n,use_bh,nodes", [(98304 + 77, True, 0),
+                                            (1600000, False, 131072)])
+def test_ewald_walk_of_one_lane_leaves_the_teams_bits(n, use_bh, nodes, ewald):
+    """More than 98304 active particles: the Ewald walk takes one lane each
+    over a tree of more than 131072 nodes and in the Barnes-Hut walk; subsets
+    of them, in teams of 4 and 16 lanes, leave the same bits."""
+    pos, _, m = ics.clustered_box(n, nhalo=64, seed=3)
+    e = Engine(periodic=True, alpha_rel=0.02, softening=1e-3,
+               ewald_table=ewald)
+    # the relative criterion's input: the accelerations' rough size here
+    e.set_particles(pos, m, last_acc_mag=np.full(n, 5.0))
+    e.setup_domain()
+    e.domain_decomposition()
+    e.tree_build()
+    assert e.num_nodes() > nodes
+    ref = e.get("pos", "last_acc_mag")
+
+    def walk(sub):
+        e.set_active(sub)
+        e.update_particles(ref["pos"], acc=np.zeros((n, 3)),
+                           last_acc_mag=ref["last_acc_mag"])
+        e.tree_acceleration(use_bh)
+        got = e.get("acc", "cost")
+        return got["acc"][sub], got["cost"][sub], e.interaction_counts()
+
+    acc, cost, counts = walk(np.arange(n, dtype=np.int32))
+    assert sum(counts) == int(cost.sum())
+    for k in (98305, 98304, 10240, 65):
+        sub = np.sort(np.random.Generator(np.random.Philox(k)).choice(
+            n, k, replace=False)).astype(np.int32)
+        a, c, counts = walk(sub)
+        np.testing.assert_array_equal(a, acc[sub], err_msg=str(k))
+        np.testing.assert_array_equal(c, cost[sub], err_msg=str(k))
+        assert sum(counts) == int(c.sum())
+
+
 @pytest.mark.parametrize("n", [300, 20000])
 def test_walk_at_tiny_separations_matches_oracle(n):
     """A sphere of radius ~ 2^-247: r^2 on both sides of 2^-500, where the
