@@ -215,7 +215,9 @@ int tdv_capture_step(tdv_context *ctx, double kick, double drift);
  * for bit; stage time 5 holds the whole step.  TDV_ERR_TIES (more than 4096
  * equal 64-bit key prefixes: the captured sort has no fallback) and
  * TDV_ERR_RANGE (a tree larger than the captured arrays) ask for an eager
- * step instead; a graph is dropped whenever its buffers may move. */
+ * step instead; a graph is dropped whenever its buffers may move.  After a
+ * replay whose tree has far more nodes in some levels than the captured one,
+ * the step is captured again for the next. */
 int tdv_launch_step(tdv_context *ctx);
 
 /* Gravity_Forcetest (Gravity/forcetest.c:24-174): FP64 direct summation

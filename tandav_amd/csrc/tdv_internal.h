@@ -44,6 +44,8 @@
 #define TDV_LVL_FEW 512      /* levels of up to this many nodes share a
                                 launch of one workgroup */
 #define TDV_LVL_THREADS 1024
+#define TDV_LVL_GROWN 1024   /* a level of a shared launch that holds more
+                                by now has a captured step planned again */
 
 /* stage events of a context (stage_ms: keys, sort, reorder, top nodes,
  * build, walk, Ewald walk, kick/drift) */
@@ -132,6 +134,7 @@ struct tdv_context {
 	int graph_mode;                  /* capturing the whole step: fixed
 	                                    capacities, counts on the device */
 	double step_kick, step_drift;    /* the captured step's factors */
+	unsigned step_lvl[64];           /* nodes per level it was planned for */
 
 	/* sort scratch */
 	uint64_t *sk[2];

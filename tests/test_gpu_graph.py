@@ -278,6 +278,53 @@ def test_step_graph_matches_eager_steps(ng):
         graph.get("pos")
 
 
+@pytest.mark.parametrize("n,first", [(300000, "uniform"), (60000, "clustered")])
+def test_step_graph_on_a_tree_of_other_level_counts(n, first):
+    """A step captured on one box and replayed on another, and back: levels
+    that it planned as empty or narrow hold thousands of nodes and the other
+    way round.  Every replay, with the old plan and with the one made after
+    it, leaves the eager step's columns and tree bit for bit."""
+    g = np.random.Generator(np.random.Philox(9))
+    boxes = [g.uniform(0.0, 1.0, (n, 3)), ics.clustered_box(n, nhalo=64,
+                                                            seed=3)[0]]
+    if first == "clustered":
+        boxes.reverse()
+    m = np.full(n, 1.0 / n)
+    eager, graph = (_engine(boxes[0], m, 0, softening=1e-3) for _ in range(2))
+    for e in (eager, graph):
+        e.domain_decomposition()
+        e.compute_acceleration(False)
+    graph.capture_step()
+    cols = ("pos", "acc", "grav_acc", "cost", "last_acc_mag", "tree_parent",
+            "key", "id")
+
+    def counts(e):
+        t = e.tree()
+        return np.bincount(t["Bitfield"][t["Npart"] > 0] & 63, minlength=43)
+
+    planned = counts(eager)
+    for turn, box in enumerate((1, 1, 0, 1)):
+        for e in (eager, graph):
+            e.update_particles(boxes[box][e.get("id")["id"]])
+        for step in range(2):
+            eager.domain_decomposition()
+            eager.compute_acceleration(False)
+            graph.launch_step()
+            a, b = eager.get(*cols), graph.get(*cols)
+            for f in cols:
+                np.testing.assert_array_equal(a[f], b[f], err_msg="%s %d %d"
+                                              % (f, turn, step))
+            assert eager.interaction_counts() == graph.interaction_counts()
+            ta, tb = eager.tree(), graph.tree()
+            assert len(ta) == len(tb)
+            for f in ta.dtype.names:
+                np.testing.assert_array_equal(ta[f], tb[f], err_msg=f)
+        if turn == 0:
+            assert (np.abs(counts(graph) - planned) > 600).any()
+            if first == "uniform":       # narrow or empty, far over 512 now
+                assert ((planned <= 44) & (counts(graph) > 1024)).sum() == 3
+
+
 def test_substep_walk_graph():
     """tdv_capture_substep_walk: with nothing moved, its replays equal the
     eager walk bit for bit (subsets of the particles active); after the
