@@ -231,9 +231,9 @@ __host__ __device__ inline EwaldCell ewald_cell(double dx, double dy,
 	return c;
 }
 
-/* the lookup in the table's own layout, one component after the other (the
- * host's, tdv_ewald_correction_host) */
-__host__ __device__ inline void ewald_corr(const double *__restrict__ tab,
+/* the lookup in the table's own layout, one component after the other: the
+ * host's (tdv_ewald_correction_host) */
+inline void ewald_corr(const double *__restrict__ tab,
 		double dx, double dy, double dz, double box2ewald, double f[3])
 {
 	const EwaldCell c = ewald_cell(dx, dy, dz, box2ewald);

@@ -15,22 +15,14 @@
 
 /* Two workgroups per CU keep the table's gathers busy, which bound a pair
  * (more of them only spread the sources' separations over more of the table:
- * 512 targets in 64^3 particles take 3.0 ms in one part each, 3.1 in two);
+ * 512 targets in 64^3 particles took 3.0 ms in one part each, 3.1 in two);
  * with fewer targets than that the sources are cut into parts of at least
  * TDV_DIRECT_MIN (16 targets 1.56 -> 0.15 ms, 100 targets 1.72 -> 0.95 ms). */
 #define TDV_DIRECT_BLOCKS 512
 #define TDV_DIRECT_MIN 2048
-/* Periodic sums from so many sources on take two at a time from the table's
- * rows (see k_direct).  512 and 1000 targets, ms: in 24^3 particles 0.23 and
- * 0.41 so, 0.23 and 0.39 one at a time from the components' own tables; in
- * 32^3 0.44 and 0.84, 0.47 and 0.86; in 64^3 2.9 and 5.9, 3.4 and 6.7. */
-#define TDV_DIRECT_ROWS 32768
 
-__device__ __forceinline__ double dwrap(double d, int periodic, double box,
-		double half)
+__device__ __forceinline__ double dwrap(double d, double box, double half)
 {
-	if (!periodic)
-		return d;
 	if (d > half)
 		d -= box;
 	else if (d < -half)
@@ -38,19 +30,24 @@ __device__ __forceinline__ double dwrap(double d, int periodic, double box,
 	return d;
 }
 
-/* Bound by the table's lines: the separations of 64 neighbouring sources lie
- * in some hundred cells, 27 KB of the rows' lines (46 KB of the components'),
- * each used once.  The next sources are loaded and U gathers are in flight
- * while a pair's sum is formed: 512 targets in 64^3 particles 3.5 -> 2.9 ms
- * (rows and U = 2; copying the cells to LDS first took 6.1, its latency bare
- * with the few wavefronts that fit). */
-template <bool ROWS, int U>
+/* Periodic sums are bound by the table's lines: the separations of 64
+ * neighbouring sources lie in some hundred cells, 27 KB of the rows' lines,
+ * each used once (46 KB of the components' own tables: those took 0.40 ms
+ * for 512 targets in 31^3 particles, the rows 0.34).  The next two sources
+ * are loaded and both gathers are in flight while a pair's sum is formed:
+ * 512 targets in 64^3 particles 2.3 ms.  (With `periodic` an argument the
+ * compiler keeps 120 registers instead of 178 and waits for one gather
+ * before the other: 2.5.  Copying the cells to LDS first took 6.1, its
+ * latency bare with the few wavefronts that fit.)  Isolated sums are bound by
+ * the FP64 arithmetic of a pair: 600 targets in 10^6 particles 1.4 ms. */
+template <bool PERIODIC>
 __global__ void __launch_bounds__(256) k_direct(int nt,
 		const int *__restrict__ idx, const double4 *__restrict__ pm, int n,
-		int periodic, double box, double G, double eps2, double eps3,
-		const double *__restrict__ tab, double b2e, int chunk,
+		double box, double G, double eps2, double eps3,
+		const double *__restrict__ rows, double b2e, int chunk,
 		double *__restrict__ out)
 {
+	constexpr int U = PERIODIC ? 2 : 1;
 	__shared__ double red[3][256];
 	const int t = blockIdx.x;
 	if (t >= nt)
@@ -70,36 +67,44 @@ __global__ void __launch_bounds__(256) k_direct(int nt,
 		double dx[U], dy[U], dz[U], m[U], f[U][3];
 #pragma unroll
 		for (int u = 0; u < U; u++) {
-			dx[u] = dwrap(next[u].x - p.x, periodic, box, half);
-			dy[u] = dwrap(next[u].y - p.y, periodic, box, half);
-			dz[u] = dwrap(next[u].z - p.z, periodic, box, half);
+			dx[u] = next[u].x - p.x;
+			dy[u] = next[u].y - p.y;
+			dz[u] = next[u].z - p.z;
 			m[u] = G * next[u].w;
 			next[u] = pm[min(j + 256 * (U + u), last - 1)];
-			if (periodic && ROWS)
-				ewald_corr_rows(tab, dx[u], dy[u], dz[u], b2e, f[u]);
-			else if (periodic)
-				ewald_corr(tab, dx[u], dy[u], dz[u], b2e, f[u]);
+			if (PERIODIC) {
+				dx[u] = dwrap(dx[u], box, half);
+				dy[u] = dwrap(dy[u], box, half);
+				dz[u] = dwrap(dz[u], box, half);
+				ewald_corr_rows(rows, dx[u], dy[u], dz[u], b2e, f[u]);
+			}
 		}
 #pragma unroll
 		for (int u = 0; u < U; u++) {
 			const double r2 = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u];
 			if (j + 256 * u >= last || j + 256 * u == i || r2 == 0)
 				continue;
-			double fac = m[u];
-			if (r2 < eps2) {
-				const double u2 = r2 / eps2;
-				fac *= (175 - u2 * (294 - u2 * 135)) / (16 * eps3);
-			} else {
-				bool ok;
-				double ri = inv_sqrt(r2, &ok);
-				if (!ok)
-					ri = 1 / sqrt(r2);
-				fac *= ri * ri * ri;
+			bool ok;
+			const double ri = inv_sqrt(r2, &ok);
+			double g = ri * ri * ri;
+			if (!ok || r2 < eps2) {
+				/* rare; free to, the compiler evaluates both cases for
+				 * every pair (600 targets in 10^6 isolated particles 2.9
+				 * ms) */
+				asm volatile("");
+				if (r2 < eps2) {
+					const double u2 = r2 / eps2;
+					g = (175 - u2 * (294 - u2 * 135)) / (16 * eps3);
+				} else {
+					const double rs = 1 / sqrt(r2);
+					g = rs * rs * rs;
+				}
 			}
+			const double fac = m[u] * g;
 			ax += fac * dx[u];
 			ay += fac * dy[u];
 			az += fac * dz[u];
-			if (periodic) {
+			if (PERIODIC) {
 				ax += m[u] * f[u][0];
 				ay += m[u] * f[u][1];
 				az += m[u] * f[u][2];
@@ -148,12 +153,10 @@ int tdv_direct_sum(tdv_context *c, int nt, const int *idx_dev, double *out_dev)
 	const int chunk = (int)((n + parts - 1) / parts);
 	parts = (n + chunk - 1) / chunk;
 	double *sums = parts > 1 ? reinterpret_cast<double *>(c->sk[0]) : out_dev;
-	const bool rows = c->par.periodic && n >= TDV_DIRECT_ROWS;
-	auto kern = rows ? k_direct<true, 2> : k_direct<false, 1>;
+	auto kern = c->par.periodic ? k_direct<true> : k_direct<false>;
 	hipLaunchKernelGGL(kern, dim3(nt, (unsigned)parts), dim3(256), 0,
-			c->stream, nt, idx_dev, c->pm, (int)n, c->par.periodic,
-			c->par.boxsize, c->par.gravity, c->Epsilon2, c->Epsilon3,
-			rows ? c->ewald_rows : c->ewald,
+			c->stream, nt, idx_dev, c->pm, (int)n, c->par.boxsize,
+			c->par.gravity, c->Epsilon2, c->Epsilon3, c->ewald_rows,
 			2 * TDV_NE / (c->par.periodic ? c->par.boxsize : 1.0), chunk,
 			sums);
 	if (parts > 1)

@@ -304,3 +304,55 @@ def test_forcetest_in_parts_matches_whole(nt):
     many = e.forcetest(np.arange(600))
     got = e.forcetest(np.arange(nt))
     assert rel_err(got, many[:nt]).max() < 1e-11
+
+
+def _root_arguments(g):
+    """Points whose distance from the origin squared is: anything over 2^-504
+    .. 2^504; a few units from even and odd powers of two, on both sides; with
+    all upper mantissa bits set; about 2^-500 and 2^500, where the short
+    inverse root begins and ends."""
+    j = np.arange(1, 9)
+    axis, pts = np.array([1.0, 0.0, 0.0]), []
+    u = g.normal(size=(3000, 3))
+    u /= np.linalg.norm(u, axis=1)[:, None]
+    pts.append(u * (2.0 ** g.uniform(-252, 252, 3000))[:, None])
+    for k in (-250, -249, -248, -100, -7, -1, 0, 1, 2, 33, 160, 249, 250):
+        for near in (1.0, np.sqrt(2.0)):
+            for x in (near * (1 - j * 2.0 ** -53), near * (1 + j * 2.0 ** -52)):
+                pts.append(np.outer(2.0 ** k * x, axis))
+                # and t half units more
+                y = 2.0 ** k * np.sqrt(g.integers(0, 9, 8) * 2.0 ** -53)
+                pts.append(np.stack([2.0 ** k * x, y, 0 * y], 1))
+            r = near * np.sqrt(1 - g.uniform(0, 1, 40) * 2.0 ** -21)
+            pts.append(2.0 ** k * r[:, None] * u[:40])
+            pts.append(np.outer(2.0 ** k * r, axis))
+    return np.concatenate(pts)
+
+
+@pytest.mark.parametrize("softening", [2.0 ** -300, 1.0])
+def test_pair_forces_round_as_root_and_division(softening):
+    """The pairs' short inverse root, the library form outside its range and
+    the softened form, evaluated on the device: one particle of unit mass at
+    the origin, massless ones around it, bit for bit the host's correctly
+    rounded 1 / sqrt(r2) in the same products."""
+    p = _root_arguments(np.random.Generator(np.random.Philox(31)))
+    pos = np.concatenate([np.zeros((1, 3)), p])
+    m = np.zeros(len(pos))
+    m[0] = 1.0
+    e = Engine(periodic=False, softening=softening)
+    e.set_particles(pos, m)
+    e.setup_domain()
+    got = np.empty_like(pos)
+    ids = e.get("id")["id"]
+    got[ids] = e.forcetest(np.arange(len(pos)))
+    d = -p
+    r2 = d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1] + d[:, 2] * d[:, 2]
+    assert r2.min() > 0 and (r2 < 2.0 ** -500).sum() > 50
+    assert (r2 > 2.0 ** 500).sum() > 50
+    eps = -41.0 / 32.0 * softening
+    eps2, eps3 = eps * eps, eps * eps * eps
+    ri = 1 / np.sqrt(r2)
+    u2 = np.minimum(r2, eps2) / eps2
+    fac = np.where(r2 < eps2, (175 - u2 * (294 - u2 * 135)) / (16 * eps3),
+                   ri * ri * ri)
+    np.testing.assert_array_equal(got[1:], fac[:, None] * d)
