@@ -30,6 +30,7 @@
 #include <cstring>
 
 #define NOCOLLAPSE 0xFFFFFFFFu
+#define TDV_COUNT_GRID 2048
 
 /* ------------------------------------------------------------------------ */
 /* top nodes                                                                 */
@@ -225,18 +226,27 @@ __global__ void __launch_bounds__(256) k_tree_marks(size_t n,
 		atomicMin(&minpack[q], packed);
 }
 
+/* Nodes per particle and, LEVELS (the FP32 build's passes over the levels
+ * need them), per level: gathered in LDS first, then one device-wide atomic
+ * per level and workgroup on the same few words, which serialise.  So the
+ * workgroups of the LEVELS form are at most TDV_COUNT_GRID, each striding
+ * over the particles: the FP32 build of 256^3 particles 3.11 ms with a
+ * workgroup per 256 of them, 2.47 with 2048 or 4096, 2.54 with 1024, 2.88
+ * with 256; of 128^3 0.46, 0.39, 0.41 (4096), 0.38, 0.41. */
+template <bool LEVELS>
 __global__ void __launch_bounds__(256) k_tree_counts(size_t n,
 		const uint64_t *__restrict__ key, TopNodes T, int vs,
 		const uint32_t *__restrict__ minpack, uint32_t *__restrict__ cnt,
 		int *__restrict__ lohi, unsigned *__restrict__ lvl_cnt)
 {
-	/* nodes per level, gathered per block first */
 	__shared__ unsigned h[64];
-	if (threadIdx.x < 64)
-		h[threadIdx.x] = 0;
-	__syncthreads();
-	const size_t gi = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (gi < n) {
+	if (LEVELS) {
+		if (threadIdx.x < 64)
+			h[threadIdx.x] = 0;
+		__syncthreads();
+	}
+	for (size_t gi = (size_t)blockIdx.x * 256 + threadIdx.x; gi < n;
+			gi += (size_t)gridDim.x * 256) {
 		const int i = (int)gi;
 		const TopRange r = top_of(key, gi, T, vs);
 		const int lo = r.tree ? dprev_of(key, i, r.first, r.level) : TDV_NT;
@@ -251,15 +261,18 @@ __global__ void __launch_bounds__(256) k_tree_counts(size_t n,
 			const int hi = lf < ml ? lf : ml;
 			c = hi >= lo ? hi - lo + 1 : 0;
 			pack = lo | (hi << 8) | ((ml <= lf) ? (1 << 16) : 0);
-			for (int lv = lo; lv <= hi; lv++)
-				atomicAdd(&h[lv], 1u);
+			if (LEVELS)
+				for (int lv = lo; lv <= hi; lv++)
+					atomicAdd(&h[lv], 1u);
 		}
 		cnt[i] = (uint32_t)c;
 		lohi[i] = pack;
 	}
-	__syncthreads();
-	if (threadIdx.x < 64 && h[threadIdx.x])
-		atomicAdd(&lvl_cnt[threadIdx.x], h[threadIdx.x]);
+	if (LEVELS) {
+		__syncthreads();
+		if (threadIdx.x < 64 && h[threadIdx.x])
+			atomicAdd(&lvl_cnt[threadIdx.x], h[threadIdx.x]);
+	}
 }
 
 /* the node ranges of the top nodes' subtrees, one wavefront (a scan over 64
@@ -984,7 +997,11 @@ int tdv_build_tree(tdv_context *c)
 			c->stream, n, c->minpack, c->lvl);
 	hipLaunchKernelGGL(k_tree_marks, dim3(tdv_blocks(n, 256)), dim3(256), 0,
 			c->stream, n, c->key, c->top, vs, c->minpack, c->d_err);
-	hipLaunchKernelGGL(k_tree_counts, dim3(tdv_blocks(n, 256)), dim3(256), 0,
+	const bool levels = c->par.precision == TDV_WALK_FP32;
+	const unsigned cgrid = (unsigned)tdv_blocks(n, 256);
+	auto counts = levels ? k_tree_counts<true> : k_tree_counts<false>;
+	hipLaunchKernelGGL(counts, dim3(levels ? std::min(cgrid,
+			(unsigned)TDV_COUNT_GRID) : cgrid), dim3(256), 0,
 			c->stream, n, c->key, c->top, vs, c->minpack,
 			reinterpret_cast<uint32_t *>(c->cnt), c->lohi, c->lvl);
 	TDV_TRY(tdv_scan_u32(c, reinterpret_cast<uint32_t *>(c->cnt), c->off, n));

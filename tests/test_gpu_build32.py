@@ -68,3 +68,18 @@ def test_fp32_build_matches_fp64_build(case):
         np.testing.assert_array_equal(top32[f], top64[f], err_msg=f)
     _within_ulp(top32["Mass"], top64["Mass"], "top Mass")
     _within_ulp(top32["CoM"], top64["CoM"], "top CoM")
+
+
+@pytest.mark.parametrize("n", [524288, 524289, 2 * 524288 + 77])
+def test_fp32_build_counts_every_particles_nodes(n):
+    """The nodes per level are counted by 2048 workgroups of 256: with as
+    many particles, one more, and the workgroups' third turn begun.  A node
+    missing from its level's list would keep no mass."""
+    pos, _, m = ics.clustered_box(n, nhalo=16, seed=5)
+    t64, top64, _ = _built(pos, m, True, "fp64")
+    t32, top32, _ = _built(pos, m, True, "fp32")
+    assert len(t32) == len(t64)
+    np.testing.assert_array_equal(t32["Bitfield"], t64["Bitfield"])
+    _within_ulp(t32["Mass"], t64["Mass"], "Mass")
+    _within_ulp(t32["CoM"], t64["CoM"], "CoM")
+    _within_ulp(top32["Mass"], top64["Mass"], "top Mass")
