@@ -269,6 +269,9 @@ void tdv_graph_drop(tdv_context *c);
                                             part */
 #define TDV_WANT_WORDS 4                 /* a split walk's wanted-top-node
                                             mask: up to 256 top nodes */
+#define TDV_EIGHT_MIN_GROUPS 36864       /* periodic relative grid walks: eight
+                                            waves per SIMD beyond this many
+                                            groups, seven up to it */
 #define TDV_ORDER_MIN_GROUPS 2048        /* FP32 walks of this many whole
                                             groups ... */
 #define TDV_ORDER_MAX_GROUPS (1 << 20)   /* ... to this many start the

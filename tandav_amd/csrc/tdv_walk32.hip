@@ -1223,13 +1223,21 @@ __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 /* the i-th group to walk: by descending expected cost when ordered */
 #define TDV_GROUP(i) (gorder ? (int)gorder[i] : (i))
 
-/* The walk is bound by instruction issue (0.9 of it at 256^3, half scalar:
- * the record loads and the loop's branches), so the usual walks have their
- * switches as constants (256^3 step 527 -> 481 ms, same bits) and the grid
- * walk runs in 64 registers, eight waves per SIMD (-> 463 ms).  The split
- * walk keeps its seven: eight cost the 100^3 box 4%. */
-template <int MODE>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8)))
+/* The walk is bound by instruction issue (half of it scalar: the record
+ * loads and the loop's branches), so the usual walks have their switches as
+ * constants (256^3 step 527 -> 481 ms, same bits) and the grid walk runs in
+ * 64 registers, EIGHT waves per SIMD (-> 463 ms).  In a periodic relative
+ * walk of up to TDV_EIGHT_MIN_GROUPS groups, 4.5 rounds of the 8192 waves
+ * that eight per SIMD are, the last and longest groups set the end, and they
+ * run faster beside six others: seven and eight waves, ms, 112^3 57.3, 60.2;
+ * 128^3 56.7, 60.1; 136^3 (39304 groups) 67.8, 67.3; 180^3 145, 143; clustered
+ * 2^21 (32768) 6.33, 6.85, 2^22 11.2, 10.8; without quadrupoles 128^3 58.1,
+ * 63.2, 136^3 68.0, 64.7.  The other walks gain from eight at every size
+ * (Barnes-Hut, 105^3: 13.3, 12.9; isolated 1.5e6 without quadrupoles 2.53,
+ * 2.42).  The split walk keeps its seven: eight cost the 100^3 box 4%. */
+template <int MODE, bool EIGHT>
+__global__ void __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(EIGHT ? 8 : 1)))
 k_walk32(TDV_WALK32_ARGS)
 {
 	TDV_WALK32_CALL(MODE, TDV_GROUP((int)blockIdx.x));
@@ -1772,11 +1780,15 @@ int tdv_walk32(tdv_context *c, int use_bh)
 		return tdv_check(c, hipGetLastError(), "k_walk32_parts_sum");
 	}
 	TDV_TRY(tdv_clear_counts(c));
+	const bool eight = use_bh || !w.periodic
+			|| ngroups_h > TDV_EIGHT_MIN_GROUPS;
 	auto kern = c->par.fp32_waves == 6 ? k_walk32_w6
 			: c->par.fp32_waves == 8 ? k_walk32_w8
-			: mode == WALK32_PERIODIC ? k_walk32<WALK32_PERIODIC>
-			: mode == WALK32_ISOLATED ? k_walk32<WALK32_ISOLATED>
-			: k_walk32<WALK32_ANY>;
+			: mode == WALK32_ISOLATED ? k_walk32<WALK32_ISOLATED, true>
+			: mode == WALK32_PERIODIC
+			? (eight ? k_walk32<WALK32_PERIODIC, true>
+				: k_walk32<WALK32_PERIODIC, false>)
+			: eight ? k_walk32<WALK32_ANY, true> : k_walk32<WALK32_ANY, false>;
 	hipLaunchKernelGGL(kern, dim3(tdv_blocks((size_t)c->nactive, 64)),
 			dim3(64), 0, c->stream, c->nactive, c->active, c->p32, c->last_acc,
 			c->top, reinterpret_cast<const Node32 *>(c->rec32), c->ewald16, w,

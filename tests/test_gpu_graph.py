@@ -62,6 +62,32 @@ def test_usual_walk_matches_general_walk(periodic, n, order, split):
     assert got[0][1] == got[1][1]
 
 
+@pytest.mark.parametrize("extra,order", [(0, 2), (1, 2), (0, 1), (1, 1)])
+def test_walk_either_side_of_eight_waves(extra, order):
+    """As many groups as the grid walk takes at seven waves per SIMD, and one
+    more: the general kernel's bits."""
+    n = 36864 * 64 + extra
+    pos, _, m = ics.clustered_box(n, nhalo=64, seed=3)
+    e = Engine(periodic=True, softening=1e-4, alpha_rel=0.01,
+               precision="fp32", compat=False, ewald_size=0.125,
+               ewald_accuracy=1.0, fp32_order=order, fp32_criterion=3)
+    e.set_particles(pos, m)
+    e.setup_domain()
+    e.domain_decomposition()
+    e.compute_acceleration(True)
+    ref = e.get("pos", "last_acc_mag")
+    got = []
+    for waves in (0, 6):
+        e.set_fp32_options(waves=waves)
+        e.update_particles(ref["pos"], acc=np.zeros((n, 3)),
+                           last_acc_mag=ref["last_acc_mag"])
+        e.tree_acceleration(False)
+        got.append((e.get("acc", "cost"), e.interaction_counts()))
+    np.testing.assert_array_equal(got[0][0]["acc"], got[1][0]["acc"])
+    np.testing.assert_array_equal(got[0][0]["cost"], got[1][0]["cost"])
+    assert got[0][1] == got[1][1]
+
+
 def test_graph_replays_match_eager_walk():
     pos, _, m = ics.zeldovich_box(32, seed=7)
     e = _engine(pos, m, 1)
