@@ -106,3 +106,63 @@ def test_tree_kicks_of_long_runs_match_oracle(n):
             np.testing.assert_array_equal(got[f], tree[f], err_msg=f)
         for f in ("Level", "Dp", "CoM"):
             np.testing.assert_array_equal(gtop[f], top[f], err_msg=f)
+
+
+def _quotients(g, n):
+    """Runs of the kicks' addends that the sums in whole units have to stop
+    at: ties of a float and of a double sum, sums about zero whose binade
+    changes with every term, terms from 2^-1060 to 2^60 of both signs."""
+    half = g.integers(-9, 10, n) * 1.0
+    about = g.normal(0.0, 1.0, n)
+    about[1::2] = -about[::2][:n // 2] * (1 + g.integers(-3, 4, n // 2)
+                                          * 2.0 ** -52)
+    wide = g.choice([-1.0, 1.0], n) * 2.0 ** g.uniform(-60, 60, n)
+    wide[g.integers(0, n, n // 16)] = 2.0 ** -1060
+    wide[g.integers(0, n, n // 16)] = 0.0
+    ties32, ties64 = half * 2.0 ** -24, half * 2.0 ** -53
+    for t in (ties32, ties64):
+        t[0] = 1.5                       # the sums' binade is [1, 2) then
+        t[n // 2] = -1.5
+        t[n // 2 + 1] = -0.75
+    return [ties32, ties64, about, wide]
+
+
+def test_tree_kicks_at_ties_and_sign_changes_match_oracle():
+    """Nodes of 4096 and 2048 particles of mass 1 in steps of powers of two:
+    the addends are the chosen ones exactly, in the top nodes' float sums and
+    in the nodes' double sums; three kicks on top of one another."""
+    g = np.random.Generator(np.random.Philox(23))
+    pos = np.concatenate([
+        g.uniform(0.0998, 0.1012, (4096, 3)),        # one cell of level 9
+        g.uniform(0.6, 0.62, (2048, 3)),
+        g.uniform(0.0, 1.0, (300, 3)) * (0.2, 0.2, 0.2) + (0.0, 0.0, 0.78),
+        g.uniform(0.3, 0.45, (40, 3))])              # no subtree
+    n = len(pos)
+    e = Engine(periodic=True, softening=1e-4)
+    e.set_particles(pos, np.ones(n))
+    e.setup_domain()
+    e.domain_decomposition()
+    e.tree_build()
+    tree, top = e.tree(), e.top_nodes()
+    assert {4096, 2048, 40} <= set(top["Npart"].tolist())
+    assert (tree["Npart"] == 4096).sum() >= 6
+    e.make_active_list(31, time_bin=np.full(n, 9, np.int32))
+    e.set_timeline(engine.timeline(False, 0.0, 1.0))
+    dt = np.full(n, 2.0 ** 8 / 2.0 ** 31)
+    st = e.get("mass", "tree_parent", "pos")
+    for kick in range(3):
+        acc = np.empty((n, 3))
+        for t in top:
+            f, c = int(t["First_Part"]), int(t["Npart"])
+            q = _quotients(g, c)
+            for d in range(3):
+                acc[f:f + c, d] = q[(kick + d) % 4] * (2.0 ** 23 * c)
+        e.update_particles(st["pos"], acc=acc)
+        e.kick_halfstep(update_tree=True)
+        tree, top = U.kicks(tree, top, st["mass"], acc, dt,
+                            st["tree_parent"], np.arange(n, dtype=np.int32))
+        got, gtop = e.tree(), e.top_nodes()
+        for f in ("Bitfield", "Dp"):
+            np.testing.assert_array_equal(got[f], tree[f], err_msg=f)
+        for f in ("Level", "Dp"):
+            np.testing.assert_array_equal(gtop[f], top[f], err_msg=f)
