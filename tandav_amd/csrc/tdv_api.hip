@@ -276,17 +276,23 @@ static void free_top(tdv_context *c)
 	dfree(t.com);
 	dfree(t.dp);
 	dfree(t.kicked);
-	dfree(t.ntop);
-	dfree(t.nnodes);
 	c->top_cap = 0;
 }
 
+/* room for `cap` top nodes.  The node counts are allocated once and stay:
+ * every report reads them, also after this has failed; what needs the top
+ * nodes themselves is refused then. */
 static int alloc_top(tdv_context *c, int cap)
 {
-	int *ptop = c->top.ptop;        /* per particle, owned by the columns */
-	free_top(c);
-	c->top.ptop = ptop;
 	TopNodes &t = c->top;
+	c->have_top = c->have_tree = 0;
+	tdv_graph_drop(c);
+	free_top(c);
+	if (!t.ntop)
+		TDV_TRY(dalloc(c, &t.ntop, 1));
+	if (!t.nnodes)
+		TDV_TRY(dalloc(c, &t.nnodes, 1));
+	TDV_HIP(c, hipMemset(t.ntop, 0, sizeof(int)));
 	TDV_TRY(dalloc(c, &t.first, cap));
 	TDV_TRY(dalloc(c, &t.npart, cap));
 	TDV_TRY(dalloc(c, &t.level, cap));
@@ -298,9 +304,6 @@ static int alloc_top(tdv_context *c, int cap)
 	TDV_TRY(dalloc(c, &t.com, 3 * (size_t)cap));
 	TDV_TRY(dalloc(c, &t.dp, 3 * (size_t)cap));
 	TDV_TRY(dalloc(c, &t.kicked, cap));
-	TDV_TRY(dalloc(c, &t.ntop, 1));
-	TDV_TRY(dalloc(c, &t.nnodes, 1));
-	TDV_HIP(c, hipMemset(t.ntop, 0, sizeof(int)));
 	c->top_cap = cap;
 	return 0;
 }
@@ -419,6 +422,8 @@ void tdv_destroy(tdv_context *c)
 		(void)hipStreamSynchronize(c->stream);
 	free_particles(c);
 	free_top(c);
+	dfree(c->top.ntop);
+	dfree(c->top.nnodes);
 	dfree(c->node_a);
 	dfree(c->node_b);
 	dfree(c->node_c);
@@ -759,6 +764,8 @@ int tdv_domain_decomposition(tdv_context *c)
 {
 	if (!c)
 		return TDV_ERR_ARG;
+	if (c->top_cap < 64)             /* a larger table could not be had */
+		TDV_TRY(alloc_top(c, 64));
 	TDV_TRY(computational_domain(c));
 	c->have_domain_set = 1;
 	TDV_TRY(launch_sort_reorder(c, true));

@@ -87,3 +87,28 @@ def test_domain_targets_of_long_cost_sums_match_oracle(n, ntarget):
     for f in ("Key", "Level", "First_Part", "Npart"):
         np.testing.assert_array_equal(top[f], rec[f], err_msg=f)
     np.testing.assert_array_equal(tasks, -rec["Target"] - 1)
+
+
+def test_reports_after_the_top_node_table_grew():
+    """More than 64 top nodes move the table; the counts that every call's
+    report reads stay, and so does what comes after."""
+    pos, _, m = ics.clustered_box(20000, nhalo=8, seed=4)
+    e = Engine(periodic=True, softening=1e-3, alpha_rel=0.005)
+    e.set_particles(pos, m)
+    e.setup_domain()
+    e.domain_decomposition()
+    e.compute_acceleration(True)
+    few = e.top_nodes()
+    for _ in range(2):
+        e.domain_decomposition_targets(60)
+        assert len(e.top_nodes()) > 64
+        e.tree_build()
+        assert int(e.top_nodes()["Npart"].sum()) == len(m)
+        keys = np.arange(2 * 5000, dtype=np.uint64).reshape(5000, 2)[::-1]
+        np.testing.assert_array_equal(e.sort_keys(np.ascontiguousarray(keys)),
+                                      np.arange(5000)[::-1])
+        e.set_particles(pos, m)
+        e.setup_domain()
+        e.domain_decomposition()
+        e.compute_acceleration(True)
+        np.testing.assert_array_equal(e.top_nodes(), few)
