@@ -1223,9 +1223,11 @@ __device__ __forceinline__ void walk32_body(int group, int part, int nparts,
 /* the i-th group to walk: by descending expected cost when ordered */
 #define TDV_GROUP(i) (gorder ? (int)gorder[i] : (i))
 
-/* The walk is bound by instruction issue (half of it scalar: the record
- * loads and the loop's branches), so the usual walks have their switches as
- * constants (256^3 step 527 -> 481 ms, same bits) and the grid walk runs in
+/* The walk is bound by the issue of vector instructions: 3.36e11 of them in
+ * the 436 ms of a 256^3 walk are 7.7e11 a second, where a SIMD's waves reach
+ * 9.1e11 (fma) to 1.04e12 (add) on vector registers and 5.8e11 with a scalar
+ * operand.  So the usual walks have their switches as constants (256^3 step
+ * 527 -> 481 ms, same bits) and the grid walk runs in
  * 64 registers, EIGHT waves per SIMD (-> 463 ms).  In a periodic relative
  * walk of up to TDV_EIGHT_MIN_GROUPS groups, 4.5 rounds of the 8192 waves
  * that eight per SIMD are, the last and longest groups set the end, and they
