@@ -652,10 +652,13 @@ static WalkParams walk_params(const tdv_context *c, int use_bh)
  * nodes teams of 4 (one lane, 4): 110^3 218, 133; 128^3 (70784 nodes) 349,
  * 248; uniform 10^6 113, 72; clustered 2^20 (98940) 20.5, 11.1, 1.3e6
  * (129705) 13.5, 9.3; and beyond one lane: clustered 1.5e6 (152597) 5.4, 8.8,
- * 2^23 14.6, 43.2; uniform 3e6 48, 141; 144^3 120, 170; 256^3 978, 1093.  The
- * Barnes-Hut walk, which opens nodes of any depth, takes one lane there:
- * 110^3 1606, 1620; clustered 2^20 558, 837, 6e6 3834, 6131; uniform 10^7
- * 322, 1125. */
+ * 2^23 14.6, 43.2; uniform 3e6 48, 141; 144^3 120, 170; 256^3 978, 1093.
+ * (All with alpha 0.005.  0.001: clustered 2^20 30, 18; 128^3 2890, 3010.
+ * 0.02: 4.3, 5.3; 216, 123; uniform 10^6 54, 35.)  The Barnes-Hut walk and
+ * relative walks of a looser criterion, which stay above the bundles, take
+ * one lane there: Barnes-Hut, 110^3 1606, 1620; clustered 2^20 558, 837, 6e6
+ * 3834, 6131; uniform 10^7 322, 1125; alpha 0.1, clustered 2^20 1.7, 3.5,
+ * uniform 10^6 8.8, 16.8. */
 struct Walk64Shape {
 	int team, block;
 };
@@ -664,6 +667,7 @@ struct Walk64Shape {
 #define TDV_W64_TEAM4 49152
 #define TDV_W64_EWALD_TEAM4 98304
 #define TDV_W64_EWALD_NODES 131072
+#define TDV_W64_EWALD_ALPHA 0.02
 #define TDV_W64_TEAM_MAX (1 << 28)       /* thread numbers within 32 bits */
 
 static Walk64Shape newton_shape(int nact)
@@ -675,11 +679,12 @@ static Walk64Shape newton_shape(int nact)
 	return { 1, 256 };
 }
 
-static Walk64Shape ewald_shape(int nact, size_t nnodes, int use_bh)
+static Walk64Shape ewald_shape(int nact, size_t nnodes, const WalkParams &w)
 {
 	if (nact <= TDV_W64_TEAM16)
 		return { 16, 64 };
-	if (nact <= TDV_W64_EWALD_TEAM4 || (!use_bh
+	if (nact <= TDV_W64_EWALD_TEAM4 || (!w.use_bh
+			&& w.alpha_rel <= TDV_W64_EWALD_ALPHA
 			&& nnodes <= TDV_W64_EWALD_NODES && nact <= TDV_W64_TEAM_MAX))
 		return { 4, 64 };
 	return { 1, 64 };
@@ -712,7 +717,7 @@ int tdv_walk64_ewald(tdv_context *c, int use_bh)
 	if (!c->have_ewald)
 		return tdv_fail(c, TDV_ERR_ARG, "periodic walk without an Ewald table");
 	const WalkParams w = walk_params(c, use_bh);
-	const Walk64Shape sh = ewald_shape(c->nactive, c->nnodes, use_bh);
+	const Walk64Shape sh = ewald_shape(c->nactive, c->nnodes, w);
 	const int L = sh.team;
 	auto kern = L == 16 ? k_walk64_ewald<16> : L == 4 ? k_walk64_ewald<4>
 			: k_walk64_ewald<1>;
